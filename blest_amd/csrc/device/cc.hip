@@ -6,11 +6,11 @@
 // (CC/BVSSCCKernel.cuh:1269-1290) is not reproduced, labels are canonicalised to the
 // smallest ORIGINAL vertex ID of the component instead.
 //
-// algo 0 (default): hook + compress.  Every slice (row i, mask m) of rset r is the set
-//   of edges {i, 8r+b : bit b of m}; each undirected edge is hooked once (i < 8r+b).
-//   Roots are linked larger-under-smaller with a compare-and-swap, so every parent is
-//   smaller than its child and the surviving root of a component is its smallest
-//   vertex.  One pass over the slices + one compression pass, independent of diameter.
+// algo 0 (default): hook + compress, roots linked larger-under-smaller with a
+//   compare-and-swap, independent of diameter.  With the CSR resident: a seed forest, a
+//   few sampled neighbours, then only the vertices outside the largest tree.  Without it:
+//   every slice (row i, mask m) of rset r is the set of edges {i, 8r+b : bit b of m},
+//   each undirected edge hooked once (i < 8r+b).
 // algo 1: min-label propagation, the reference's iteration (frontier = rsets whose
 //   labels dropped), two stream-ordered kernels per iteration.
 #include "dgraph.hpp"
@@ -22,8 +22,8 @@ __device__ __forceinline__ uint32_t ld_parent(const uint32_t* p, uint32_t x) {
     return __hip_atomic_load(p + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Root of x with path halving.  Parents only ever decrease and always name an
-// ancestor, so concurrent halving stores keep the forest valid.
+// Root of x with path halving.  A parent always names an ancestor, so concurrent halving
+// stores keep the forest valid.
 __device__ __forceinline__ uint32_t find_root(uint32_t* p, uint32_t x) {
     uint32_t par = ld_parent(p, x);
     while (par != x) {
@@ -101,18 +101,216 @@ __global__ void __launch_bounds__(256) cc_hook_kernel(GraphView g, uint32_t* p) 
     }
 }
 
+// Parents read through the CU's own cache: an old value is an old ancestor (a parent only
+// ever moves up its own tree), and a root that looks like one but no longer is loses its
+// compare-and-swap and goes on from the value that returns.
+__device__ __forceinline__ uint32_t ld_parent_near(const uint32_t* p, uint32_t x) {
+    return __hip_atomic_load(p + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // After hooking the roots are final.  Compression must store roots only: a
 // path-halving store (an ancestor that is not the root) racing with another thread's
 // final store could overwrite it.  Every value a thread can read here (an old parent or
 // a root) is an ancestor, so the read-only walk always ends at the root.
 __global__ void cc_compress_kernel(uint32_t* p, uint32_t n) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        uint32_t x = i, par = ld_parent(p, x);
+        uint32_t x = i, par = ld_parent_near(p, x);
         while (par != x) {
             x = par;
-            par = ld_parent(p, x);
+            par = ld_parent_near(p, x);
         }
         if (x != i) __hip_atomic_store(p + i, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// ----------------------------------------------- components from the CSR (algo 0)
+// Hooking every edge of the graph costs a pass over all slices with two dependent walks
+// per edge, and on a social graph the concurrent compare-and-swaps meet at the hubs'
+// roots.  With the (symmetric) CSR resident almost no edge needs to be hooked:
+//   seed    a vertex takes its highest-degree neighbour (the first of its list) as
+//           parent when that neighbour ranks above it: (degree, smaller ID).  Ranks rise
+//           along parents, so this is a forest, made without one atomic;
+//   sample  each vertex hooks its first neighbour, then (the trees compressed) its next
+//           kCcSampled ones; after that nearly every vertex of a large component hangs
+//           under one root;
+//   giant   the most frequent root among kCcVotes sampled vertices;
+//   rest    only vertices outside that tree hook the rest of their lists (an edge that
+//           leaves the tree is in the list of its outer end too: the graph is symmetric).
+// Hooks link roots only, larger ID under smaller, so a root is hooked at most once and
+// the links between roots fall in ID: no cycle whatever the seed forest's order was.
+// Roots are no longer the smallest vertices of their components; the labels come from
+// the minimum taken over each tree at the end.
+// Bound by the launches and the dependent walks, not by memory (R-MAT 20: 8 MB of
+// offsets, probes and parents).  Measured (MI355X, whole call): R-MAT 20 natural order,
+// labels on the device, 1.5-3.9 ms with every slice hooked (by the graph's seed) ->
+// 0.142 ms; 1023-square grid in RCM order, labels to the host, 13.2 -> 0.50 ms.
+constexpr uint32_t kCcSampled = 2;
+constexpr unsigned kCcVotes = 256;
+constexpr uint32_t kCcHeavy = 64;  // longer lists are hooked by a whole wave
+constexpr int kCcBlock = 256;
+
+__device__ __forceinline__ uint32_t find_root_near(uint32_t* p, uint32_t x) {
+    uint32_t par = ld_parent_near(p, x);
+    while (par != x) {
+        const uint32_t gp = ld_parent_near(p, par);
+        if (gp == par) return par;
+        __hip_atomic_store(p + x, gp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        x = gp;
+        par = ld_parent_near(p, x);
+    }
+    return x;
+}
+
+__device__ __forceinline__ void hook_near(uint32_t* p, uint32_t a, uint32_t b) {
+    uint32_t ra = find_root_near(p, a), rb = find_root_near(p, b);
+    if (ra == rb) return;
+    for (;;) {
+        // the CU's own copy may lag behind: go on to the current roots before the swap (a
+        // swap that fails meets every other one at that root, a load does not)
+        ra = find_root(p, ra);
+        rb = find_root(p, rb);
+        if (ra == rb) return;
+        if (ra > rb) {
+            const uint32_t t = ra;
+            ra = rb;
+            rb = t;
+        }
+        uint32_t expected = rb;
+        if (__hip_atomic_compare_exchange_strong(p + rb, &expected, ra, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
+            return;
+        rb = expected;  // rb was hooked meanwhile: go on from its parent
+    }
+}
+
+// p = the seed forest, minOf = no minimum yet.
+__global__ void __launch_bounds__(kCcBlock) cc_seed_kernel(GraphView g, uint32_t* p, uint32_t* minOf) {
+    for (uint32_t v = blockIdx.x * kCcBlock + threadIdx.x; v < g.n; v += gridDim.x * kCcBlock) {
+        const uint32_t b = g.csrPtr[v], deg = g.csrPtr[v + 1] - b;
+        uint32_t par = v;
+        if (deg) {
+            const uint32_t u = g.probe ? g.probe[v] : g.csrIdx[b];
+            const uint32_t du = g.csrPtr[u + 1] - g.csrPtr[u];
+            if (du > deg || (du == deg && u < v)) par = u;
+        }
+        p[v] = par;
+        minOf[v] = 0xFFFFFFFFu;
+    }
+}
+
+// Hooks entries [first, last) of every vertex's list; trees already joined are told apart
+// by one load each (p is compressed).
+__global__ void __launch_bounds__(kCcBlock) cc_sample_hook_kernel(GraphView g, uint32_t* p, uint32_t first,
+                                                                  uint32_t last) {
+    for (uint32_t v = blockIdx.x * kCcBlock + threadIdx.x; v < g.n; v += gridDim.x * kCcBlock) {
+        const uint32_t b = g.csrPtr[v], e = g.csrPtr[v + 1];
+        for (uint32_t i = b + first; i < min(e, b + last); ++i) {
+            const uint32_t u = g.csrIdx[i];
+            if (ld_parent_near(p, u) != ld_parent_near(p, v)) hook_near(p, v, u);
+        }
+    }
+}
+
+// giant[0] = the root that most of the sampled vertices hang under (one workgroup; p is
+// compressed).  Each thread counts the votes for its own sample's root.
+__global__ void __launch_bounds__(kCcVotes) cc_giant_kernel(const uint32_t* p, uint32_t n, uint32_t* giant) {
+    __shared__ uint32_t root[kCcVotes];
+    __shared__ unsigned long long best;
+    const unsigned t = threadIdx.x;
+    const uint32_t r = p[uint64_t(t) * n / kCcVotes];
+    root[t] = r;
+    if (t == 0) best = 0;
+    __syncthreads();
+    unsigned votes = 0;
+    for (unsigned i = 0; i < kCcVotes; ++i) votes += root[i] == r;
+    atomicMax(&best, (unsigned long long)votes << 32 | r);
+    __syncthreads();
+    if (t == 0) giant[0] = uint32_t(best);
+}
+
+__global__ void __launch_bounds__(kCcBlock) cc_rest_kernel(GraphView g, uint32_t* p, const uint32_t* giant) {
+    const unsigned lane = lane_id();
+    const uint32_t big = giant[0];
+    const uint32_t n64 = (g.n + kWave - 1) / kWave * kWave;  // whole waves: the ballots below
+    for (uint32_t v = blockIdx.x * kCcBlock + threadIdx.x; v < n64; v += gridDim.x * kCcBlock) {
+        uint32_t b = 0, e = 0;
+        if (v < g.n && ld_parent_near(p, v) != big) {
+            b = g.csrPtr[v] + kCcSampled + 1;
+            e = g.csrPtr[v + 1];
+        }
+        const bool heavy = b < e && e - b > kCcHeavy;
+        if (!heavy)
+            for (uint32_t i = b; i < e; ++i) hook_near(p, v, g.csrIdx[i]);
+        for (unsigned long long h = __ballot(heavy); h; h &= h - 1) {
+            const int l = __builtin_ctzll(h);
+            const uint32_t hv = __shfl(v, l, kWave), hb = __shfl(b, l, kWave), he = __shfl(e, l, kWave);
+            for (uint32_t i = hb + lane; i < he; i += kWave) hook_near(p, hv, g.csrIdx[i]);
+        }
+    }
+}
+
+// minOf[root] = smallest original ID in the component (the giant tree's as one minimum per
+// workgroup, giantMin), and the number of roots per workgroup (their sum is the component
+// count).  A wave carries the running minimum of the root it met last in a register and
+// gives it up, one atomic, when another root takes its place or at the end; an atomic is
+// only issued when it would lower the value.  (An atomicMin per vertex serialised at the
+// giant component's address: 11.9 ms for the 1 M vertices of a 1023-square grid; one per
+// wave still 71 us there and 230 us on R-MAT 20.)
+__device__ __forceinline__ void lower_min(uint32_t* minOf, uint32_t root, uint32_t id) {
+    if (id < __hip_atomic_load(minOf + root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(minOf + root, id);
+}
+
+__global__ void __launch_bounds__(kCcBlock) cc_min_original_kernel(const uint32_t* p, const uint32_t* newToOld,
+                                                                   uint32_t* minOf, const uint32_t* giant,
+                                                                   uint32_t* giantMin, uint32_t* rootsPerBlock,
+                                                                   uint32_t n) {
+    __shared__ unsigned long long tmp64[16];
+    __shared__ uint32_t blockMin;
+    const unsigned lane = lane_id();
+    const uint32_t big = giant[0];
+    if (threadIdx.x == 0) blockMin = 0xFFFFFFFFu;
+    __syncthreads();
+    uint32_t bigMin = 0xFFFFFFFFu;
+    uint32_t held = 0xFFFFFFFFu, heldMin = 0xFFFFFFFFu, roots = 0;  // held: wave-uniform
+    const uint32_t n64 = (n + kWave - 1) / kWave * kWave;
+    for (uint32_t i = blockIdx.x * kCcBlock + threadIdx.x; i < n64; i += gridDim.x * kCcBlock) {
+        const bool ok = i < n;
+        const uint32_t r = ok ? p[i] : 0xFFFFFFFFu;
+        const uint32_t id = ok ? (newToOld ? newToOld[i] : i) : 0xFFFFFFFFu;
+        roots += r == i;
+        bool left = ok && r != big;
+        if (ok && !left) bigMin = min(bigMin, id);
+        // the root met last, then the roots of the first two lanes that differ; the rest
+        // are small components, whose lanes go alone
+        for (int round = 0; round < 3; ++round) {
+            const unsigned long long open = __ballot(left);
+            if (!open) break;
+            const uint32_t cand = round == 0 ? held : uint32_t(__shfl(r, __builtin_ctzll(open), kWave));
+            const unsigned long long same = __ballot(left && r == cand);
+            if (!same) continue;
+            if (__popcll(same) == 1 && cand != held) {  // alone: no reduction, nothing replaced
+                if (left && r == cand) lower_min(minOf, r, id);
+            } else {
+                uint32_t m = left && r == cand ? id : 0xFFFFFFFFu;
+                for (int d = kWave / 2; d > 0; d >>= 1) m = min(m, uint32_t(__shfl_xor(m, d, kWave)));
+                if (cand != held) {
+                    if (lane == 0 && held != 0xFFFFFFFFu) lower_min(minOf, held, heldMin);
+                    held = cand;
+                    heldMin = m;
+                } else {
+                    heldMin = min(heldMin, m);
+                }
+            }
+            left = left && r != cand;
+        }
+        if (left) lower_min(minOf, r, id);
+    }
+    if (lane == 0 && held != 0xFFFFFFFFu) lower_min(minOf, held, heldMin);
+    atomicMin(&blockMin, bigMin);  // LDS
+    const unsigned long long total = block_sum_u64(roots, tmp64);  // its barriers complete blockMin
+    if (threadIdx.x == 0) {
+        rootsPerBlock[blockIdx.x] = uint32_t(total);
+        giantMin[blockIdx.x] = blockMin;
     }
 }
 
@@ -120,17 +318,24 @@ __global__ void fill_u32_kernel(uint32_t* a, uint32_t v, uint32_t n) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) a[i] = v;
 }
 
-// minOrig[root] = smallest original ID in the component.
-__global__ void cc_min_original_kernel(const uint32_t* p, const uint32_t* newToOld, uint32_t* minOrig, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        atomicMin(minOrig + p[i], newToOld[i]);
-}
-
-// out[old] = minOrig[root(new(old))]
-__global__ void cc_relabel_kernel(const uint32_t* p, const uint32_t* oldToNew, const uint32_t* minOrig,
-                                  uint32_t* out, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        out[i] = minOrig[p[oldToNew[i]]];
+// out[old] = minOf[root(new(old))]; launched with the grid of cc_min_original_kernel, whose
+// workgroups left one minimum of the giant tree each.
+__global__ void __launch_bounds__(kCcBlock) cc_relabel_kernel(const uint32_t* p, const uint32_t* oldToNew,
+                                                              const uint32_t* minOf, const uint32_t* giant,
+                                                              const uint32_t* giantMin, uint32_t* out, uint32_t n) {
+    __shared__ uint32_t all;
+    const uint32_t big = giant[0];
+    if (threadIdx.x == 0) all = 0xFFFFFFFFu;
+    __syncthreads();
+    uint32_t m = 0xFFFFFFFFu;
+    for (uint32_t i = threadIdx.x; i < gridDim.x; i += kCcBlock) m = min(m, giantMin[i]);
+    atomicMin(&all, m);  // LDS
+    __syncthreads();
+    const uint32_t bigMin = all;
+    for (uint32_t i = blockIdx.x * kCcBlock + threadIdx.x; i < n; i += gridDim.x * kCcBlock) {
+        const uint32_t r = p[oldToNew ? oldToNew[i] : i];
+        out[i] = r == big ? bigMin : minOf[r];
+    }
 }
 
 // ------------------------------------------------------------ label propagation
@@ -271,20 +476,47 @@ static void cc_run(Query& q, int algo, uint32_t* hostLabels, blest_cc_stats* st)
     DeviceGraph& g = *q.g;
     if (!g.symmetric) throw Error(BLEST_ERR_UNSUPPORTED, "connected components need a symmetric graph");
     const bool labelsOnDevice = hostLabels && check_result_range(hostLabels, 4 * size_t(g.n), g.device, "labels");
+    if (algo != 0 && algo != 1) throw Error(BLEST_ERR_INVALID_ARGUMENT, "unknown CC algorithm");
+    const dim3 block(dev::kCcBlock);
+    const dim3 grid(std::min<uint32_t>(uint32_t(g.cus) * 8, (g.n + dev::kCcBlock - 1) / dev::kCcBlock));
+    // the sampled hooks meet at the trees that swallow the rest: fewer waves at once fail
+    // fewer swaps (1023-square grid 157 -> 96 us for the second entry, 8 -> 2 workgroups per CU)
+    const dim3 few(std::min<uint32_t>(grid.x, uint32_t(g.cus) * 2));
     if (!q.labels) {
         q.labels = q.alloc<uint32_t>(g.n);
         q.labelsAux = q.alloc<uint32_t>(g.n);
+        q.ccCounts = q.alloc<uint32_t>(2 * size_t(g.cus) * 8 + 1);
+        q.hostCcCounts.resize(size_t(g.cus) * 8);
     }
     GraphView gv = g.view();
-    const dim3 grid(uint32_t(g.cus) * 8), block(256);
     unsigned iterations = 1;
+    uint32_t *giantMin = q.ccCounts + size_t(g.cus) * 8, *giant = giantMin + size_t(g.cus) * 8;
+    const auto vote = [&] {
+        hipLaunchKernelGGL(dev::cc_giant_kernel, dim3(1), dim3(dev::kCcVotes), 0, q.stream, q.labels, g.n, giant);
+    };
     BLEST_HIP(hipEventRecord(q.ev0, q.stream));
-    if (algo == 0) {
-        hipLaunchKernelGGL(dev::cc_init_kernel, grid, block, 0, q.stream, q.labels, g.n);
-        hipLaunchKernelGGL(dev::cc_hook_kernel, grid, block, 0, q.stream, gv, q.labels);
+    if (algo == 0 && g.hasCsr) {
+        hipLaunchKernelGGL(dev::cc_seed_kernel, grid, block, 0, q.stream, gv, q.labels, q.labelsAux);
         hipLaunchKernelGGL(dev::cc_compress_kernel, grid, block, 0, q.stream, q.labels, g.n);
+        hipLaunchKernelGGL(dev::cc_sample_hook_kernel, grid, block, 0, q.stream, gv, q.labels, 0u, 1u);
+        hipLaunchKernelGGL(dev::cc_compress_kernel, grid, block, 0, q.stream, q.labels, g.n);
+        hipLaunchKernelGGL(dev::cc_sample_hook_kernel, few, block, 0, q.stream, gv, q.labels, 1u,
+                           dev::kCcSampled + 1u);
+        hipLaunchKernelGGL(dev::cc_compress_kernel, grid, block, 0, q.stream, q.labels, g.n);
+        vote();
+        hipLaunchKernelGGL(dev::cc_rest_kernel, grid, block, 0, q.stream, gv, q.labels, giant);
+        hipLaunchKernelGGL(dev::cc_compress_kernel, grid, block, 0, q.stream, q.labels, g.n);
+        vote();
         BLEST_HIP(hipGetLastError());
-    } else if (algo == 1) {
+    } else if (algo == 0) {
+        // no CSR resident: every slice's edges are hooked
+        hipLaunchKernelGGL(dev::cc_init_kernel, grid, block, 0, q.stream, q.labels, g.n);
+        hipLaunchKernelGGL(dev::cc_hook_kernel, dim3(uint32_t(g.cus) * 8), block, 0, q.stream, gv, q.labels);
+        hipLaunchKernelGGL(dev::cc_compress_kernel, grid, block, 0, q.stream, q.labels, g.n);
+        hipLaunchKernelGGL(dev::fill_u32_kernel, grid, block, 0, q.stream, q.labelsAux, 0xFFFFFFFFu, g.n);
+        vote();
+        BLEST_HIP(hipGetLastError());
+    } else {
         dev::LpArgs a;
         a.labels = q.labels;
         a.front0 = q.front0;
@@ -301,44 +533,34 @@ static void cc_run(Query& q, int algo, uint32_t* hostLabels, blest_cc_stats* st)
             hipLaunchKernelGGL(dev::cc_lp_expand_kernel, lg, lb, 0, q.stream, gv, a, L);
             hipLaunchKernelGGL(dev::cc_lp_update_kernel, lg, lb, 0, q.stream, gv, a, L);
         });
+        hipLaunchKernelGGL(dev::fill_u32_kernel, grid, block, 0, q.stream, q.labelsAux, 0xFFFFFFFFu, g.n);
+        vote();
         BLEST_HIP(hipGetLastError());
-    } else {
-        throw Error(BLEST_ERR_INVALID_ARGUMENT, "unknown CC algorithm");
-    }
-    BLEST_HIP(hipEventRecord(q.ev1, q.stream));
-    BLEST_HIP(hipStreamSynchronize(q.stream));
-    if (algo == 1) {
         dev::Ctrl c;
         BLEST_HIP(hipMemcpyAsync(&c, q.ctrl, sizeof(c), hipMemcpyDeviceToHost, q.stream));
-    BLEST_HIP(hipStreamSynchronize(q.stream));
+        BLEST_HIP(hipStreamSynchronize(q.stream));
         iterations = c.iterations;
     }
-    float ms = 0;
-    BLEST_HIP(hipEventElapsedTime(&ms, q.ev0, q.ev1));
-    const uint32_t* result = q.labels;
-    if (g.hasPerm) {
-        hipLaunchKernelGGL(dev::fill_u32_kernel, grid, block, 0, q.stream, q.labelsAux, 0xFFFFFFFFu, g.n);
-        hipLaunchKernelGGL(dev::cc_min_original_kernel, grid, block, 0, q.stream, q.labels, g.permNewToOld,
-                           q.labelsAux, g.n);
-        hipLaunchKernelGGL(dev::cc_relabel_kernel, grid, block, 0, q.stream, q.labels, g.permOldToNew, q.labelsAux,
-                           reinterpret_cast<uint32_t*>(q.levels), g.n);
-        BLEST_HIP(hipGetLastError());
-        result = reinterpret_cast<const uint32_t*>(q.levels);
-    }
-    // Components = vertices that are their own label, counted on the host from host
-    // memory only: when the caller's array is device memory the count reads a host copy.
-    if (hostLabels) BLEST_HIP(hipMemcpyAsync(hostLabels, result, 4 * size_t(g.n), hipMemcpyDefault, q.stream));
-    std::vector<uint32_t> tmp;
-    const uint32_t* counted = hostLabels;
-    if (!hostLabels || labelsOnDevice) {
-        tmp.resize(g.n);
-        BLEST_HIP(hipMemcpyAsync(tmp.data(), result, 4 * size_t(g.n), hipMemcpyDeviceToHost, q.stream));
-        counted = tmp.data();
-    }
+    // canonical labels, straight into the caller's array when it is device memory (host
+    // results are staged: over the parents, or in the level array when the relabelling
+    // permutes), and the component count
+    uint32_t* result = labelsOnDevice ? hostLabels : g.hasPerm ? reinterpret_cast<uint32_t*>(q.levels) : q.labels;
+    hipLaunchKernelGGL(dev::cc_min_original_kernel, grid, block, 0, q.stream, q.labels,
+                       g.hasPerm ? g.permNewToOld : nullptr, q.labelsAux, giant, giantMin, q.ccCounts, g.n);
+    if (hostLabels)
+        hipLaunchKernelGGL(dev::cc_relabel_kernel, grid, block, 0, q.stream, q.labels,
+                           g.hasPerm ? g.permOldToNew : nullptr, q.labelsAux, giant, giantMin, result, g.n);
+    BLEST_HIP(hipGetLastError());
+    BLEST_HIP(hipEventRecord(q.ev1, q.stream));
+    BLEST_HIP(hipMemcpyAsync(q.hostCcCounts.data(), q.ccCounts, 4 * size_t(grid.x), hipMemcpyDeviceToHost, q.stream));
+    if (hostLabels && !labelsOnDevice)
+        BLEST_HIP(hipMemcpyAsync(hostLabels, result, 4 * size_t(g.n), hipMemcpyDefault, q.stream));
     BLEST_HIP(hipStreamSynchronize(q.stream));
     if (st) {
+        float ms = 0;
+        BLEST_HIP(hipEventElapsedTime(&ms, q.ev0, q.ev1));
         uint32_t comps = 0;
-        for (uint32_t v = 0; v < g.n; ++v) comps += counted[v] == v;
+        for (uint32_t i = 0; i < grid.x; ++i) comps += q.hostCcCounts[i];
         st->kernel_ms = ms;
         st->no_components = comps;
         st->iterations = iterations;

@@ -136,6 +136,8 @@ struct Query {
     int32_t* levelsOut = nullptr;  // original-order copy (when the graph carries a permutation)
     uint32_t* labels = nullptr;    // CC
     uint32_t* labelsAux = nullptr;
+    uint32_t* ccCounts = nullptr;  // per workgroup: roots, the giant tree's minimum; then its root
+    std::vector<uint32_t> hostCcCounts;
     // multi-source state, allocated on first use: words per vertex x n
     uint32_t mbfsWords = 0;
     unsigned long long *mVis = nullptr, *mFront0 = nullptr, *mFront1 = nullptr, *mNext = nullptr;
