@@ -1,29 +1,26 @@
-// Many small graphs in one launch: one workgroup traverses one graph from its root,
-// with the visited / frontier / next bitmaps held in LDS (n <= 131072 per graph:
-// 3 x 16 KiB), so levels are separated by workgroup barriers only and the bottom-up
-// frontier tests never leave the CU.  Top-down streams the graph's BVSS quads
-// (slice size 8) for every rset with a frontier byte; bottom-up pulls over the CSR.
+// Many small graphs in one launch: one workgroup of 1,024 threads traverses one graph from
+// its root, with the visited / frontier / next bitmaps held in LDS (n <= 131072 per graph:
+// 3 x 16 KiB), so levels are separated by workgroup barriers only and no bitmap access
+// leaves the CU.  The graphs are symmetric, so one CSR serves both directions.
+#include <cstring>
+
 #include "dgraph.hpp"
 
 namespace blest {
 namespace dev {
 
 struct BatchGraph {
-    uint32_t n, R;
+    uint32_t n;
+    uint32_t narrow;     // 1: list entries are 16-bit (n <= 65536), 0: 32-bit
     uint64_t levelOff;   // into the concatenated level array
-    uint64_t rsetOff;    // into rsetQuad (R + 1 entries per graph, graph-relative quads)
-    uint64_t quadOff;    // into rows / masks
     uint64_t csrPtrOff;  // into csrPtr (n + 1 entries per graph, graph-relative)
-    uint64_t csrIdxOff;  // into csrIdx
+    uint64_t csrIdxOff;  // into csrIdx, in 16-bit units (even)
 };
 
 struct BatchArgs {
     const BatchGraph* graphs;
-    const uint32_t* rsetQuad;
-    const uint4* rows;
-    const uint32_t* masks;
     const uint32_t* csrPtr;
-    const uint32_t* csrIdx;
+    const uint16_t* csrIdx;
     const uint32_t* roots;
     const uint32_t* order;
     int32_t* levels;
@@ -31,25 +28,66 @@ struct BatchArgs {
     double alpha;
 };
 
-__global__ void __launch_bounds__(512) batch_bfs_kernel(BatchArgs a) {
-    extern __shared__ unsigned long long lds[];
-    __shared__ unsigned s_new;
-    __shared__ unsigned long long s_edges;
-    const uint32_t gi = a.order[blockIdx.x];
-    const BatchGraph G = a.graphs[gi];
-    const uint32_t W = (G.n + 63) / 64;
+// What bounds the kernel is not bandwidth (a graph's 2 MB of lists are read about once) but
+// the round trips of dependent loads: list bounds, list entries, one after another, in one
+// workgroup.  Hence 32 waves per CU (two graphs), and in every step as many independent
+// loads as the registers of 8 waves per SIMD hold:
+//   top-down   the frontier vertices of 64 bitmap words are dealt out to the lanes one each
+//              (a sparse frontier fills whole waves), kBatchTd list entries per step;
+//   bottom-up  a lane takes its vertex of kBatchWords words at once, kBatchBu entries of
+//              each per step; found vertices go straight into visited and next;
+//   a list still open after kBatchOwn entries is finished by its whole wave;
+//   graphs of at most 65536 vertices keep 16-bit list entries (635 -> 560 us below), and
+//   the switch to bottom-up waits until the frontier's edges are a quarter of the open
+//   ones (alpha 4): a top-down discovery is an LDS atomic, while a bottom-up sweep reads
+//   every line of the lists (alpha 15: 560 us, 8: 490, 4: 440, 2: 440).
+// Measured (MI355X), 512 Erdos-Renyi graphs, n ~ U[1024, 65536], degree 8: 2.06 ms with a
+// wave per rset (16 lanes busy at degree 8) and a lane walking one vertex's list entry by
+// entry, 0.37 ms in this form (4 words 0.40, 8 entries of 4 words spill: 0.55).
+constexpr int kBatchBlock = 1024;
+constexpr int kBatchTd = 8, kBatchWords = 3, kBatchBu = 4;
+constexpr uint32_t kBatchOwn = 32;
+
+// N list entries as one load per 16 bytes.  A CU's vector cache takes about one line per
+// clock, so entry-wise loads of 64 lists cost a line access per entry (628 us for 512 graphs
+// of 65536 vertices, 575 us with these); lists start at any entry, which unaligned vector
+// loads take, and the list array is padded by a step's length past its last entry.
+template <class Idx, int N>
+struct __attribute__((packed, aligned(sizeof(Idx)))) ListStep {
+    Idx v[N];
+};
+template <int N, class Idx>
+__device__ __forceinline__ ListStep<Idx, N> load_step(const Idx* ci, uint32_t p) {
+    return *reinterpret_cast<const ListStep<Idx, N>*>(ci + p);
+}
+
+// Position of the k-th (from 0) set bit of x; x has more than k bits.
+__device__ __forceinline__ unsigned nth_bit(unsigned long long x, unsigned k) {
+    unsigned pos = 0;
+#pragma unroll
+    for (int width = 32; width > 0; width >>= 1) {
+        const unsigned c = __popcll((x >> pos) & ((1ull << width) - 1));
+        if (k >= c) {
+            k -= c;
+            pos += width;
+        }
+    }
+    return pos;
+}
+
+// sNew / sEdges: vertices discovered by level (slot L % 3) and their degree sum.
+template <class Idx>
+__device__ __forceinline__ void batch_traverse(const BatchArgs& a, const BatchGraph& G, uint32_t src, const Idx* ci,
+                                               unsigned long long* lds, unsigned* sNew, unsigned long long* sEdges) {
+    const uint32_t n = G.n, W = (n + 63) / 64;
     unsigned long long* vis = lds;
     unsigned long long* front = lds + a.maxWords;
     unsigned long long* next = lds + 2 * a.maxWords;
-    const uint32_t* rq = a.rsetQuad + G.rsetOff;
-    const uint4* rows = a.rows + G.quadOff;
-    const uint32_t* masks = a.masks + G.quadOff;
     const uint32_t* cp = a.csrPtr + G.csrPtrOff;
-    const uint32_t* ci = a.csrIdx + G.csrIdxOff;
     int32_t* levels = a.levels + G.levelOff;
-    const unsigned lane = lane_id(), wave = threadIdx.x / kWave, nwaves = blockDim.x / kWave;
-    const uint32_t src = a.roots[gi];
-    for (uint32_t w = threadIdx.x; w < W; w += blockDim.x) {
+    const unsigned lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    constexpr unsigned nwaves = kBatchBlock / kWave;
+    for (uint32_t w = threadIdx.x; w < W; w += kBatchBlock) {
         const unsigned long long x = (w == src / 64) ? (1ull << (src & 63)) : 0ull;
         vis[w] = x;
         front[w] = x;
@@ -57,83 +95,195 @@ __global__ void __launch_bounds__(512) batch_bfs_kernel(BatchArgs a) {
     }
     if (threadIdx.x == 0) {
         levels[src] = 0;
-        s_new = 1;
-        s_edges = cp[src + 1] - cp[src];
+        sNew[0] = 1;
+        sEdges[0] = cp[src + 1] - cp[src];
+        sNew[1] = 0;
+        sEdges[1] = 0;
     }
     __syncthreads();
-    const unsigned long long m = cp[G.n];
+    const unsigned long long m = cp[n];
     unsigned long long seenEdges = 0;
-    bool bottomUp = false;
+    bool bottomUp = false, clean = true;  // clean: next is all zero
     for (unsigned L = 1;; ++L) {
-        const unsigned nf = s_new;
-        const unsigned long long mf = s_edges;
+        const unsigned nf = sNew[(L - 1) % 3];
+        const unsigned long long mf = sEdges[(L - 1) % 3];
         if (nf == 0) break;
         seenEdges += mf;
         if (!bottomUp && double(mf) * a.alpha > double(m - min(seenEdges, m))) bottomUp = true;
-        else if (bottomUp && nf * 24ull < G.n) bottomUp = false;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            s_new = 0;
-            s_edges = 0;
+        else if (bottomUp && nf * 24ull < n) bottomUp = false;
+        if (threadIdx.x == 0) {  // last read at the top of the level before, a barrier ago
+            sNew[(L + 1) % 3] = 0;
+            sEdges[(L + 1) % 3] = 0;
         }
-        if (!bottomUp) {
-            const uint8_t* fb = reinterpret_cast<const uint8_t*>(front);
-            for (uint32_t r = wave; r < G.R; r += nwaves) {
-                const uint32_t f = fb[r];
-                if (!f) continue;
-                for (uint32_t q = rq[r] + lane; q < rq[r + 1]; q += kWave) {
-                    const uint4 r4 = rows[q];
-                    const uint32_t mk = masks[q];
-                    const uint32_t rv[4] = {r4.x, r4.y, r4.z, r4.w};
-#pragma unroll
-                    for (int s = 0; s < 4; ++s)
-                        if ((mk >> (8 * s)) & f) {
-                            const uint32_t row = rv[s];
-                            if (!((vis[row >> 6] >> (row & 63)) & 1ull)) atomicOr(&next[row >> 6], 1ull << (row & 63));
-                        }
-                }
-            }
-        } else {
-            for (uint32_t v0 = wave * kWave; v0 < W * 64; v0 += nwaves * kWave) {
-                const uint32_t v = v0 + lane;
-                bool found = false;
-                if (v < G.n && !((vis[v >> 6] >> (v & 63)) & 1ull))
-                    for (uint32_t p = cp[v]; p < cp[v + 1]; ++p) {
-                        const uint32_t u = ci[p];
-                        if ((front[u >> 6] >> (u & 63)) & 1ull) {
-                            found = true;
-                            break;
-                        }
-                    }
-                const unsigned long long b = __ballot(found);
-                if (lane == 0 && b) next[v0 >> 6] = b;
-            }
-        }
-        __syncthreads();
         unsigned cnt = 0;
         unsigned long long edges = 0;
-        for (uint32_t w = threadIdx.x; w < W; w += blockDim.x) {
-            const unsigned long long nw = next[w] & ~vis[w];
-            next[w] = 0ull;
-            vis[w] |= nw;
-            front[w] = nw;
-            for (unsigned long long b = nw; b; b &= b - 1) {
-                const uint32_t v = w * 64 + __builtin_ctzll(b);
-                levels[v] = int32_t(L);
-                edges += cp[v + 1] - cp[v];
-                ++cnt;
+        if (!bottomUp) {
+            if (!clean) {
+                for (uint32_t w = threadIdx.x; w < W; w += kBatchBlock) next[w] = 0ull;
+                __syncthreads();
             }
+            const uint32_t* vis32 = reinterpret_cast<const uint32_t*>(vis);
+            uint32_t* next32 = reinterpret_cast<uint32_t*>(next);
+            auto reach = [&](uint32_t u) {
+                const uint32_t bit = 1u << (u & 31);
+                if (!(vis32[u >> 5] & bit)) atomicOr(&next32[u >> 5], bit);
+            };
+            // words wave, wave + nwaves, ...: 64 of them at a time, word i0 + lane per lane
+            for (uint32_t i0 = 0; i0 * nwaves + wave < W; i0 += kWave) {
+                const uint32_t w = (i0 + lane) * nwaves + wave;
+                const unsigned long long f = w < W ? front[w] : 0ull;
+                const unsigned c = __popcll(f);
+                const unsigned incl = wave_inclusive_scan(c), excl = incl - c;
+                const unsigned total = __shfl(incl, kWave - 1, kWave);
+                for (unsigned t0 = 0; t0 < total; t0 += kWave) {
+                    const unsigned t = t0 + lane;
+                    const unsigned owner = wave_owner(excl, min(t, total - 1));
+                    const unsigned long long of = __shfl(f, owner, kWave);
+                    const unsigned oex = __shfl(excl, owner, kWave);
+                    uint32_t p = 0, e = 0;
+                    if (t < total) {
+                        const uint32_t v = ((i0 + owner) * nwaves + wave) * 64 + nth_bit(of, t - oex);
+                        p = cp[v];
+                        e = cp[v + 1];
+                    }
+                    const uint32_t own = min(e, p + kBatchOwn);
+                    while (p < own) {
+                        const auto step = load_step<kBatchTd>(ci, p);
+#pragma unroll
+                        for (int j = 0; j < kBatchTd; ++j) reach(p + j < own ? uint32_t(step.v[j]) : src);  // src: visited
+                        p += kBatchTd;
+                    }
+                    p = own;
+                    for (unsigned long long h = __ballot(p < e); h; h &= h - 1) {
+                        const int l = __builtin_ctzll(h);
+                        const uint32_t hp = __shfl(p, l, kWave), he = __shfl(e, l, kWave);
+                        for (uint32_t q0 = hp; q0 < he; q0 += 4 * kWave) {
+                            uint32_t u[4];
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                const uint32_t q = q0 + j * kWave + lane;
+                                u[j] = q < he ? uint32_t(ci[q]) : src;
+                            }
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) reach(u[j]);
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+            // fold: lane per vertex; the spent frontier becomes the next level's empty `next`
+            for (uint32_t w0 = wave; w0 < W; w0 += nwaves * kBatchWords) {
+                unsigned long long nw[kBatchWords];
+                uint32_t lo[kBatchWords], hi[kBatchWords];
+#pragma unroll
+                for (int k = 0; k < kBatchWords; ++k) {
+                    const uint32_t w = w0 + k * nwaves, v = w * 64 + lane;
+                    nw[k] = w < W ? next[w] : 0ull;
+                    lo[k] = hi[k] = 0;
+                    if ((nw[k] >> lane) & 1ull) {
+                        lo[k] = cp[v];
+                        hi[k] = cp[v + 1];
+                        levels[v] = int32_t(L);
+                        ++cnt;
+                    }
+                    if (lane == 0 && w < W) {
+                        vis[w] |= nw[k];
+                        front[w] = 0ull;
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < kBatchWords; ++k) edges += hi[k] - lo[k];
+            }
+            clean = true;
+        } else {
+            const uint32_t* front32 = reinterpret_cast<const uint32_t*>(front);
+            for (uint32_t w0 = wave; w0 < W; w0 += nwaves * kBatchWords) {
+                uint32_t b[kBatchWords], e[kBatchWords];
+                unsigned open = 0, found = 0;  // bit k: the vertex of word k
+#pragma unroll
+                for (int k = 0; k < kBatchWords; ++k) {
+                    const uint32_t w = w0 + k * nwaves, v = w * 64 + lane;
+                    const bool o = w < W && v < n && !((vis[min(w, W - 1)] >> lane) & 1ull);
+                    b[k] = o ? cp[v] : 0u;
+                    e[k] = o ? cp[v + 1] : 0u;
+                }
+#pragma unroll
+                for (int k = 0; k < kBatchWords; ++k)
+                    if (b[k] < e[k]) open |= 1u << k;
+                for (uint32_t off = 0; off < kBatchOwn && __ballot(open != 0); off += kBatchBu) {
+                    ListStep<Idx, kBatchBu> u[kBatchWords];
+#pragma unroll
+                    for (int k = 0; k < kBatchWords; ++k)
+                        if ((open >> k) & 1u) u[k] = load_step<kBatchBu>(ci, b[k] + off);
+#pragma unroll
+                    for (int k = 0; k < kBatchWords; ++k) {
+                        if ((open >> k) & 1u) {
+                            bool hit = false;
+#pragma unroll
+                            for (int j = 0; j < kBatchBu; ++j)
+                                if (b[k] + off + j < e[k]) hit |= (front32[u[k].v[j] >> 5] >> (u[k].v[j] & 31)) & 1u;
+                            if (hit) found |= 1u << k;
+                            if (hit || b[k] + off + kBatchBu >= e[k]) open &= ~(1u << k);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < kBatchWords; ++k) {
+                    for (unsigned long long h = __ballot((open >> k) & 1u); h; h &= h - 1) {
+                        const int l = __builtin_ctzll(h);
+                        const uint32_t hp = __shfl(b[k], l, kWave) + kBatchOwn, he = __shfl(e[k], l, kWave);
+                        bool hit = false;
+                        for (uint32_t q0 = hp; q0 < he && !hit; q0 += kWave) {  // wave-uniform
+                            const uint32_t q = q0 + lane;
+                            const uint32_t u = ci[min(q, he - 1)];
+                            hit = __ballot(q < he && ((front32[u >> 5] >> (u & 31)) & 1u)) != 0ull;
+                        }
+                        if (hit && lane == unsigned(l)) found |= 1u << k;
+                    }
+                    const uint32_t w = w0 + k * nwaves;
+                    const bool f = (found >> k) & 1u;
+                    const unsigned long long fw = __ballot(f);
+                    if (f) {
+                        levels[w * 64 + lane] = int32_t(L);
+                        ++cnt;
+                        edges += e[k] - b[k];
+                    }
+                    if (lane == 0 && w < W) {
+                        next[w] = fw;
+                        if (fw) vis[w] |= fw;  // this wave's word alone
+                    }
+                }
+            }
+            clean = false;  // the spent frontier becomes `next`
         }
         cnt = wave_sum_u32(cnt);
         edges = wave_sum_u64(edges);
         if (lane == 0 && cnt) {
-            atomicAdd(&s_new, cnt);
-            atomicAdd(&s_edges, edges);
+            atomicAdd(&sNew[L % 3], cnt);
+            atomicAdd(&sEdges[L % 3], edges);
         }
         __syncthreads();
+        unsigned long long* spent = front;
+        front = next;
+        next = spent;
     }
-    for (uint32_t v = threadIdx.x; v < G.n; v += blockDim.x)
-        if (!((vis[v >> 6] >> (v & 63)) & 1ull)) levels[v] = -1;
+    for (uint32_t w = wave; w < W; w += nwaves) {
+        const uint32_t v = w * 64 + lane;
+        if (v < n && !((vis[w] >> lane) & 1ull)) levels[v] = -1;
+    }
+}
+
+__global__ void __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(8))) batch_bfs_kernel(BatchArgs a) {
+    extern __shared__ unsigned long long lds[];
+    __shared__ unsigned sNew[3];
+    __shared__ unsigned long long sEdges[3];
+    const uint32_t gi = a.order[blockIdx.x];
+    const BatchGraph G = a.graphs[gi];
+    const uint16_t* ci = a.csrIdx + G.csrIdxOff;
+    if (G.narrow)
+        batch_traverse(a, G, a.roots[gi], ci, lds, sNew, sEdges);
+    else
+        batch_traverse(a, G, a.roots[gi], reinterpret_cast<const uint32_t*>(ci), lds, sNew, sEdges);
 }
 
 }  // namespace dev
@@ -144,9 +294,9 @@ struct GraphBatch {
     uint64_t totalN = 0;
     std::vector<uint32_t> sizes;
     dev::BatchGraph* graphs = nullptr;
-    uint32_t *rsetQuad = nullptr, *masks = nullptr, *csrPtr = nullptr, *csrIdx = nullptr, *roots = nullptr;
+    uint32_t *csrPtr = nullptr, *roots = nullptr;
+    uint16_t* csrIdx = nullptr;
     uint32_t* order = nullptr;  // workgroup -> graph
-    uint4* rows = nullptr;
     int32_t* levels = nullptr;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -188,8 +338,6 @@ blest_status blest_graph_batch_create(const blest_csc* const* graphs, uint32_t c
             gb.device = device;
             BLEST_HIP(hipSetDevice(device));
             std::vector<dev::BatchGraph> info(count);
-            // Per-graph BVSS (variable layout) built in parallel, then concatenated.
-            std::vector<BVSS> parts(count);
             std::vector<int> bad(count, 0);
             for (uint32_t i = 0; i < count; ++i)
                 if (!graphs[i]) throw Error(BLEST_ERR_INVALID_ARGUMENT, "null graph in batch");
@@ -197,45 +345,38 @@ blest_status blest_graph_batch_create(const blest_csc* const* graphs, uint32_t c
                 const CSC& g = csc_of(graphs[i]);
                 if (g.n == 0 || g.n > 131072) bad[i] = 1;
                 else if (!csc_is_symmetric(g, 1)) bad[i] = 2;
-                else parts[i] = bvss_build(g, 8, 4, false, 1);
             });
             for (uint32_t i = 0; i < count; ++i) {
                 if (bad[i] == 1) throw Error(BLEST_ERR_UNSUPPORTED, "batched graphs need 1 <= n <= 131072");
                 if (bad[i] == 2) throw Error(BLEST_ERR_UNSUPPORTED, "batched graphs must be symmetric");
             }
-            uint64_t lv = 0, nr = 0, nq = 0, ncp = 0, nci = 0;
+            uint64_t lv = 0, ncp = 0, nci = 0;
             for (uint32_t i = 0; i < count; ++i) {
                 const CSC& g = csc_of(graphs[i]);
-                const BVSS& b = parts[i];
                 dev::BatchGraph& G = info[i];
                 G.n = g.n;
-                G.R = b.noRealSliceSets;
                 G.levelOff = lv;
-                G.rsetOff = nr;
-                G.quadOff = nq;
                 G.csrPtrOff = ncp;
                 G.csrIdxOff = nci;
                 lv += g.n;
-                nr += uint64_t(b.noRealSliceSets) + 1;
-                nq += b.masks.size();
                 ncp += g.colPtrs.size();
-                nci += g.rows.size();
+                G.narrow = g.n <= 65536;
+                nci += G.narrow ? (g.rows.size() + 1) / 2 * 2 : 2 * g.rows.size();
                 gb.sizes.push_back(g.n);
                 gb.maxWords = std::max(gb.maxWords, (g.n + 63) / 64);
             }
-            std::vector<uint32_t> rq(nr), masks(nq), rowWords(nq * 4), cpAll(ncp), ciAll(nci);
+            std::vector<uint32_t> cpAll(ncp);
+            std::vector<uint16_t> ciAll(nci + 2 * dev::kBatchTd);  // a step may read past the last list
             parallel_dynamic(count, hw_threads(), 16, [&](uint64_t i, unsigned) {
                 const CSC& g = csc_of(graphs[i]);
-                const BVSS& b = parts[i];
                 const dev::BatchGraph& G = info[i];
-                for (uint32_t r = 0; r <= b.noRealSliceSets; ++r)
-                    rq[G.rsetOff + r] = uint32_t(b.sliceSetPtrs[b.realPtrs[r]] / 4);
-                std::copy(b.masks.begin(), b.masks.end(), masks.begin() + G.quadOff);
-                std::copy(b.rowIds.begin(), b.rowIds.end(), rowWords.begin() + G.quadOff * 4);
                 std::copy(g.colPtrs.begin(), g.colPtrs.end(), cpAll.begin() + G.csrPtrOff);
-                std::copy(g.rows.begin(), g.rows.end(), ciAll.begin() + G.csrIdxOff);
+                uint16_t* to = ciAll.data() + G.csrIdxOff;
+                if (G.narrow)
+                    std::transform(g.rows.begin(), g.rows.end(), to, [](uint32_t r) { return uint16_t(r); });
+                else if (!g.rows.empty())
+                    std::memcpy(to, g.rows.data(), 4 * g.rows.size());
             });
-            parts.clear();
             // Workgroups start roughly in index order: largest graphs first, so the
             // small ones fill in behind them (longest-processing-time order).
             std::vector<uint32_t> order(count);
@@ -245,9 +386,6 @@ blest_status blest_graph_batch_create(const blest_csc* const* graphs, uint32_t c
             gb.count = count;
             gb.totalN = lv;
             gb.graphs = gb.upload(info);
-            gb.rsetQuad = gb.upload(rq);
-            gb.masks = gb.upload(masks);
-            gb.rows = reinterpret_cast<uint4*>(gb.upload(rowWords));
             gb.csrPtr = gb.upload(cpAll);
             gb.csrIdx = gb.upload(ciAll);
             gb.roots = gb.upload(std::vector<uint32_t>(count, 0));
@@ -272,26 +410,24 @@ blest_status blest_graph_batch_bfs(blest_graph_batch* h, const uint32_t* roots, 
         BLEST_HIP(hipSetDevice(gb.device));
         for (uint32_t i = 0; i < gb.count; ++i)
             if (roots[i] >= gb.sizes[i]) throw Error(BLEST_ERR_INVALID_ARGUMENT, "root out of range");
-        if (levels) check_result_range(levels, 4 * size_t(gb.totalN), gb.device, "levels");
+        // device results are written in place, host ones staged in gb.levels
+        const bool onDevice = levels && check_result_range(levels, 4 * size_t(gb.totalN), gb.device, "levels");
         BLEST_HIP(hipMemcpyAsync(gb.roots, roots, 4 * size_t(gb.count), hipMemcpyHostToDevice, gb.stream));
         dev::BatchArgs a;
         a.graphs = gb.graphs;
-        a.rsetQuad = gb.rsetQuad;
-        a.rows = gb.rows;
-        a.masks = gb.masks;
         a.csrPtr = gb.csrPtr;
         a.csrIdx = gb.csrIdx;
         a.roots = gb.roots;
         a.order = gb.order;
-        a.levels = gb.levels;
+        a.levels = onDevice ? levels : gb.levels;
         a.maxWords = gb.maxWords;
-        a.alpha = 15.0;
+        a.alpha = 4.0;
         const size_t lds = size_t(3) * gb.maxWords * sizeof(unsigned long long);
         BLEST_HIP(hipEventRecord(gb.ev0, gb.stream));
-        hipLaunchKernelGGL(dev::batch_bfs_kernel, dim3(gb.count), dim3(512), lds, gb.stream, a);
+        hipLaunchKernelGGL(dev::batch_bfs_kernel, dim3(gb.count), dim3(dev::kBatchBlock), lds, gb.stream, a);
         BLEST_HIP(hipGetLastError());
         BLEST_HIP(hipEventRecord(gb.ev1, gb.stream));
-        if (levels)
+        if (levels && !onDevice)
             BLEST_HIP(hipMemcpyAsync(levels, gb.levels, 4 * gb.totalN, hipMemcpyDefault, gb.stream));
         BLEST_HIP(hipStreamSynchronize(gb.stream));
         float ms = 0;
