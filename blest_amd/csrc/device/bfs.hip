@@ -898,21 +898,32 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID bfs_update
     }
 }
 
-// Unreached vertices get -1 (lane per vertex: coalesced stores).
-__global__ void __launch_bounds__(kProducerBlock) bfs_final_kernel(GraphView g, BfsArgs a) {
-    const unsigned tid = blockIdx.x * blockDim.x + threadIdx.x;
-    const unsigned wave = tid / kWave, nwaves = (gridDim.x * blockDim.x) / kWave;
+// Closes a traversal, once it is done (enqueued ahead of every poll): unreached vertices
+// get -1 (lane per vertex: coalesced stores), the caller's device array its levels in
+// original order, the host its copy of the control block.
+__global__ void __launch_bounds__(kProducerBlock) bfs_final_kernel(GraphView g, BfsArgs a, const uint32_t* oldToNew,
+                                                                   int32_t* dst, Ctrl* host) {
+    if (blockIdx.x == 0) publish_ctrl(a.ctrl, host);
+    if (!ld_relaxed(&a.ctrl->done)) return;
+    const unsigned tid = blockIdx.x * blockDim.x + threadIdx.x, nthreads = gridDim.x * blockDim.x;
+    const unsigned wave = tid / kWave, nwaves = nthreads / kWave;
     const unsigned lane = lane_id();
+    const bool same = dst && !oldToNew;
     for (uint32_t w = wave; w < g.W; w += nwaves) {
         const unsigned long long vis = a.visited[w];
         const uint32_t u = w * 64 + lane;
-        if (u < g.n && !((vis >> lane) & 1ull)) a.levels[u] = -1;
+        if (u >= g.n) continue;
+        const bool reached = (vis >> lane) & 1ull;
+        if (!reached) a.levels[u] = -1;
+        if (same) dst[u] = reached ? a.levels[u] : -1;
     }
-}
-
-__global__ void unpermute_levels_kernel(int32_t* out, const int32_t* in, const uint32_t* oldToNew, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        out[i] = in[oldToNew[i]];
+    if (dst && oldToNew)  // a level from the visited bit, not from the stores above
+        for (uint32_t i = tid; i < g.n; i += nthreads) {
+            const uint32_t u = oldToNew[i];
+            const bool reached = test_bit(a.visited, u);
+            const int32_t l = a.levels[u];
+            dst[i] = reached ? l : -1;
+        }
 }
 
 }  // namespace dev
@@ -928,7 +939,7 @@ static ExpandKernel expand_kernel_for(const DeviceGraph& g) {
     }
 }
 
-void bfs_launch(Query& q, uint32_t src, bool trace) {
+void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
     DeviceGraph& g = *q.g;
     dev::BfsArgs a;
     a.levels = q.levels;
@@ -955,7 +966,11 @@ void bfs_launch(Query& q, uint32_t src, bool trace) {
     const GraphView gv = g.view();
     const dim3 grid = level_grid(g), block(dev::kProducerBlock);
     const ExpandKernel expand = expand_kernel_for(g);
+    const uint32_t* oldToNew = g.hasPerm ? g.permOldToNew : nullptr;
     BLEST_HIP(hipEventRecord(q.ev0, q.stream));
+    const auto close = [&] {
+        hipLaunchKernelGGL(dev::bfs_final_kernel, grid, block, 0, q.stream, gv, a, oldToNew, dst, q.hostCtrl);
+    };
     hipLaunchKernelGGL(dev::bfs_init_kernel, grid, block, 0, q.stream, gv, a);
     // small levels between chunks of level kernels: from the root, and after every chunk
     const bool fused = a.fuseQuads != 0;
@@ -979,9 +994,8 @@ void bfs_launch(Query& q, uint32_t src, bool trace) {
                 hipLaunchKernelGGL(dev::bfs_update_kernel, grid, block, 0, q.stream, gv, a, L);
                 mark();
             },
-            [&] { hipLaunchKernelGGL(dev::bfs_final_kernel, grid, block, 0, q.stream, gv, a); });
+            close);
         BLEST_HIP(hipGetLastError());
-        BLEST_HIP(hipEventRecord(q.ev1, q.stream));
         q.lastSource = src;
         q.pending = true;
         return;
@@ -992,7 +1006,7 @@ void bfs_launch(Query& q, uint32_t src, bool trace) {
             hipLaunchKernelGGL(expand, grid, block, 0, q.stream, gv, a, L);
             hipLaunchKernelGGL(dev::bfs_update_kernel, grid, block, 0, q.stream, gv, a, L);
         },
-        [&] { hipLaunchKernelGGL(dev::bfs_final_kernel, grid, block, 0, q.stream, gv, a); },
+        close,
         &q.graphs[kGraphBfs],
         [&](unsigned k) {
             hipLaunchKernelGGL(expand, grid, block, 0, q.stream, gv, ar, k);
@@ -1009,18 +1023,17 @@ void bfs_launch(Query& q, uint32_t src, bool trace) {
         })
               : nullptr);
     BLEST_HIP(hipGetLastError());
-    BLEST_HIP(hipEventRecord(q.ev1, q.stream));
     q.lastSource = src;
     q.pending = true;
 }
 
+// hostLevels: a result that the closing kernel has not written (host memory, or the query's
+// own level array); with a permutation it was staged in levelsOut.
 void bfs_finish(Query& q, int32_t* hostLevels, blest_bfs_stats* st) {
     DeviceGraph& g = *q.g;
     BLEST_HIP(hipStreamSynchronize(q.stream));
     q.pending = false;
-    dev::Ctrl c;
-    BLEST_HIP(hipMemcpyAsync(&c, q.ctrl, sizeof(c), hipMemcpyDeviceToHost, q.stream));
-    BLEST_HIP(hipStreamSynchronize(q.stream));
+    const dev::Ctrl& c = *q.hostCtrl;
     // level kernels the next traversal enqueues before the fused kernel takes over: up to
     // the final run of small shrinking levels, else all this traversal used
     q.levelHint = c.tailFrom ? c.tailFrom - 1 : c.levels - c.fusedLevels;
@@ -1036,16 +1049,17 @@ void bfs_finish(Query& q, int32_t* hostLevels, blest_bfs_stats* st) {
         st->bottom_up_mask = c.buMask;
     }
     if (hostLevels) {
-        const int32_t* src = q.levels;
-        if (g.hasPerm) {
-            hipLaunchKernelGGL(dev::unpermute_levels_kernel, dim3(1024), dim3(256), 0, q.stream, q.levelsOut,
-                               q.levels, g.permOldToNew, g.n);
-            BLEST_HIP(hipGetLastError());
-            src = q.levelsOut;
-        }
-        BLEST_HIP(hipMemcpyAsync(hostLevels, src, sizeof(int32_t) * g.n, hipMemcpyDefault, q.stream));
+        BLEST_HIP(hipMemcpyAsync(hostLevels, g.hasPerm ? q.levelsOut : q.levels, sizeof(int32_t) * g.n,
+                                 hipMemcpyDefault, q.stream));
         BLEST_HIP(hipStreamSynchronize(q.stream));
     }
+}
+
+// A traversal with its result in `levels` (nullable; host or device memory).
+static void bfs_run(Query& q, uint32_t src, int32_t* levels, bool trace, blest_bfs_stats* st) {
+    int32_t* dst = direct_result(q, levels, q.g->n, "levels");
+    bfs_launch(q, map_source(*q.g, src), trace, dst ? dst : (levels && q.g->hasPerm) ? q.levelsOut : nullptr);
+    bfs_finish(q, dst ? nullptr : levels, st);
 }
 
 }  // namespace blest
@@ -1060,9 +1074,7 @@ blest_status blest_bfs(blest_query* qh, uint32_t src, int32_t* levels, blest_bfs
         Query& q = qh->q;
         std::lock_guard<std::mutex> lk(q.mu);
         BLEST_HIP(hipSetDevice(q.g->device));
-        if (levels) check_result_range(levels, sizeof(int32_t) * size_t(q.g->n), q.g->device, "levels");
-        bfs_launch(q, map_source(*q.g, src));
-        bfs_finish(q, levels, st);
+        bfs_run(q, src, levels, false, st);
     });
 }
 
@@ -1105,10 +1117,8 @@ blest_status blest_bfs_trace(blest_query* qh, uint32_t src, int32_t* levels, ble
         Query& q = qh->q;
         std::lock_guard<std::mutex> lk(q.mu);
         BLEST_HIP(hipSetDevice(q.g->device));
-        if (levels) check_result_range(levels, sizeof(int32_t) * size_t(q.g->n), q.g->device, "levels");
-        bfs_launch(q, map_source(*q.g, src), true);
         blest_bfs_stats s{};
-        bfs_finish(q, levels, &s);
+        bfs_run(q, src, levels, true, &s);
         if (st) *st = s;
         // events per level L = 1, 2, ...: before expand(L), after it, after update(L)
         const uint32_t nl = std::min<uint32_t>(s.total_levels, uint32_t(q.traceEvents.size() / 3));

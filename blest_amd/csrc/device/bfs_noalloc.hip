@@ -27,13 +27,14 @@ __device__ __align__(256) unsigned char scratch[kScratchBytes];
 constexpr int kMaxDevices = 64;
 
 // Per-device set-up: the device address of `scratch` (each GPU holds its own copy of
-// the array at its own address; the host-side name is only a stand-in) and the events
-// the level driver records.
+// the array at its own address; the host-side name is only a stand-in), the events the
+// level driver records and the pinned control block it polls (256 bytes of host memory).
 struct DeviceSlot {
     std::once_flag once;
     std::mutex mu;  // serialises calls on this device
     unsigned char* ptr = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr, evChunk = nullptr;
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    dev::Ctrl* hostCtrl = nullptr;  // pinned
     hipError_t setupErr = hipSuccess;
     std::string setupWhat;
     unsigned levelHint = 0;  // depth of the last traversal (sizes the level driver's first chunk)
@@ -61,10 +62,10 @@ DeviceSlot& slot_for(int device) {
                 return;
             }
         }
-        e = hipEventCreateWithFlags(&s.evChunk, hipEventDisableTiming);
+        e = hipHostMalloc(reinterpret_cast<void**>(&s.hostCtrl), sizeof(dev::Ctrl), hipHostMallocDefault);
         if (e != hipSuccess) {
             s.setupErr = e;
-            s.setupWhat = "hipEventCreateWithFlags";
+            s.setupWhat = "hipHostMalloc";
         }
     });
     if (s.setupErr != hipSuccess)
@@ -111,8 +112,8 @@ size_t carve_state(const DeviceGraph& g, unsigned char* base, Query& q, bool lev
 struct BorrowedQuery : Query {
     ~BorrowedQuery() {
         stream = nullptr;
-        ev0 = ev1 = evChunk = evIn = nullptr;
-        hostDone = nullptr;
+        ev0 = ev1 = evIn = nullptr;
+        hostCtrl = nullptr;
         allocations.clear();
     }
 };
@@ -120,11 +121,6 @@ struct BorrowedQuery : Query {
 __global__ void clear_ctrl_kernel(dev::Ctrl* c) {
     unsigned* w = reinterpret_cast<unsigned*>(c);
     for (unsigned i = threadIdx.x; i < sizeof(dev::Ctrl) / sizeof(unsigned); i += blockDim.x) w[i] = 0u;
-}
-
-__global__ void unpermute_kernel(int32_t* out, const int32_t* in, const uint32_t* oldToNew, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        out[i] = in[oldToNew[i]];
 }
 
 }  // namespace
@@ -163,26 +159,19 @@ blest_status blest_bfs_noalloc(const blest_device_graph* dg, uint32_t src, int32
                             std::to_string(kScratchBytes) + "-byte scratch of blest_bfs_noalloc (use blest_bfs)");
         DeviceSlot& slot = slot_for(g.device);
         std::lock_guard<std::mutex> lk(slot.mu);
-        unsigned hostDone = 0;
         q.g = &g;
         q.maxSources = 1;
         q.stream = static_cast<hipStream_t>(stream);
         q.ev0 = slot.ev0;
         q.ev1 = slot.ev1;
-        q.evChunk = slot.evChunk;
-        q.hostDone = &hostDone;
+        q.hostCtrl = slot.hostCtrl;
         q.noGraphs = true;  // instantiating a captured graph would allocate
         q.levelHint = slot.levelHint;
         carve_state(g, slot.ptr, q, g.hasPerm);
         if (!g.hasPerm) q.levels = levels;  // reordered IDs are the caller's IDs
         hipLaunchKernelGGL(clear_ctrl_kernel, dim3(1), dim3(64), 0, q.stream, q.ctrl);
         BLEST_HIP(hipGetLastError());
-        bfs_launch(q, s);
-        if (g.hasPerm) {
-            hipLaunchKernelGGL(unpermute_kernel, dim3(1024), dim3(256), 0, q.stream, levels, q.levels, g.permOldToNew,
-                               g.n);
-            BLEST_HIP(hipGetLastError());
-        }
+        bfs_launch(q, s, false, g.hasPerm ? levels : nullptr);
         bfs_finish(q, nullptr, st);
         slot.levelHint = q.levelHint;
     });

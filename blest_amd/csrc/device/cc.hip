@@ -536,10 +536,7 @@ static void cc_run(Query& q, int algo, uint32_t* hostLabels, blest_cc_stats* st)
         hipLaunchKernelGGL(dev::fill_u32_kernel, grid, block, 0, q.stream, q.labelsAux, 0xFFFFFFFFu, g.n);
         vote();
         BLEST_HIP(hipGetLastError());
-        dev::Ctrl c;
-        BLEST_HIP(hipMemcpyAsync(&c, q.ctrl, sizeof(c), hipMemcpyDeviceToHost, q.stream));
-        BLEST_HIP(hipStreamSynchronize(q.stream));
-        iterations = c.iterations;
+        iterations = q.hostCtrl->iterations;
     }
     // canonical labels, straight into the caller's array when it is device memory (host
     // results are staged: over the parents, or in the level array when the relabelling

@@ -4,6 +4,7 @@
 #include <cstring>
 
 #include "dgraph.hpp"
+#include "level_common.hpp"
 #include "segments.hpp"
 
 namespace blest {
@@ -19,10 +20,9 @@ Query::~Query() {
         if (lg.exec) (void)hipGraphExecDestroy(lg.exec);
     for (hipEvent_t e : traceEvents) (void)hipEventDestroy(e);
     for (void* p : allocations) (void)hipFree(p);
-    if (hostDone) (void)hipHostFree(hostDone);
+    if (hostCtrl) (void)hipHostFree(hostCtrl);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
-    if (evChunk) (void)hipEventDestroy(evChunk);
     if (evIn) (void)hipEventDestroy(evIn);
     if (stream) (void)hipStreamDestroy(stream);
 }
@@ -38,6 +38,9 @@ namespace dev {
 __global__ void advance_levels_kernel(Ctrl* c, unsigned count) {
     if (threadIdx.x == 0) c->levelBase += count;
 }
+
+// The closing kernel of a traversal that has none of its own.
+__global__ void publish_ctrl_kernel(const Ctrl* c, Ctrl* host) { publish_ctrl(c, host); }
 }  // namespace dev
 
 uint64_t launch_key(double alpha, double beta, int direction, uint64_t extra) {
@@ -79,14 +82,14 @@ static void capture_levels(Query& q, LevelGraph& lg, const std::function<void(un
 }
 
 static bool poll_done(Query& q, const std::function<void()>& tail) {
-    // The tail (e.g. marking unreached vertices) is idempotent and harmless before the
-    // end: enqueuing it ahead of the poll hides the host round trip when the chunk was
-    // the last one.
-    if (tail) tail();
-    BLEST_HIP(hipMemcpyAsync(q.hostDone, &q.ctrl->done, sizeof(unsigned), hipMemcpyDeviceToHost, q.stream));
-    BLEST_HIP(hipEventRecord(q.evChunk, q.stream));
-    BLEST_HIP(hipEventSynchronize(q.evChunk));
-    return *q.hostDone != 0;
+    if (tail)
+        tail();
+    else
+        hipLaunchKernelGGL(dev::publish_ctrl_kernel, dim3(1), dim3(64), 0, q.stream, q.ctrl, q.hostCtrl);
+    BLEST_HIP(hipGetLastError());
+    BLEST_HIP(hipEventRecord(q.ev1, q.stream));
+    BLEST_HIP(hipStreamSynchronize(q.stream));
+    return q.hostCtrl->done != 0;
 }
 
 // The first chunk covers the previous traversal's depth (levelHint) plus two levels.  A
@@ -154,6 +157,14 @@ bool check_result_range(const void* dst, size_t bytes, int device, const char* w
                                                     " bytes, the device allocation holds " +
                                                     std::to_string(size_t(b + extent - d)) + " from there");
     return true;
+}
+
+int32_t* direct_result(const Query& q, int32_t* dst, size_t count, const char* what) {
+    if (!dst || !check_result_range(dst, sizeof(int32_t) * count, q.g->device, what)) return nullptr;
+    // a result in the query's own level array: the traversal reads there what it writes
+    const int32_t* own = q.levels;
+    if (dst < own + size_t(q.g->n) * q.maxSources && own < dst + count) return nullptr;
+    return dst;
 }
 
 uint32_t map_source(const DeviceGraph& g, uint32_t src) {
@@ -455,9 +466,9 @@ blest_status blest_query_create(blest_device_graph* dg, uint32_t max_sources, bl
             BLEST_HIP(hipStreamCreateWithFlags(&q.stream, hipStreamNonBlocking));
             BLEST_HIP(hipEventCreate(&q.ev0));
             BLEST_HIP(hipEventCreate(&q.ev1));
-            BLEST_HIP(hipEventCreateWithFlags(&q.evChunk, hipEventDisableTiming));
             BLEST_HIP(hipEventCreateWithFlags(&q.evIn, hipEventDisableTiming));
-            BLEST_HIP(hipHostMalloc(reinterpret_cast<void**>(&q.hostDone), sizeof(unsigned), hipHostMallocDefault));
+            BLEST_HIP(hipHostMalloc(reinterpret_cast<void**>(&q.hostCtrl), sizeof(dev::Ctrl), hipHostMallocDefault));
+            std::memset(static_cast<void*>(q.hostCtrl), 0, sizeof(dev::Ctrl));
             q.ctrl = q.alloc<dev::Ctrl>(1);
             BLEST_HIP(hipMemset(q.ctrl, 0, sizeof(dev::Ctrl)));
             q.levels = q.alloc<int32_t>(size_t(g.n) * max_sources);

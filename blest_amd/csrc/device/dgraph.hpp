@@ -119,9 +119,11 @@ struct Query {
     DeviceGraph* g = nullptr;
     uint32_t maxSources = 1;
     hipStream_t stream = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr, evChunk = nullptr;
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t evIn = nullptr;     // a caller's stream position that the next launch waits for
-    unsigned* hostDone = nullptr;  // pinned: the traversal's done flag, polled per chunk
+    // pinned: a chunk's closing kernel stores the control block here, so a poll is one
+    // stream synchronisation (no copy, no second round trip for the totals)
+    dev::Ctrl* hostCtrl = nullptr;
     unsigned levelHint = 0;        // levels of the last traversal (sizes the first chunk)
     dev::Ctrl* ctrl = nullptr;
     int32_t* levels = nullptr;  // n * maxSources
@@ -175,7 +177,9 @@ struct Query {
 };
 
 // Level-loop driver: enqueues level(L) for L = 1, 2, ... in chunks and polls the
-// device's done flag after each chunk.  With lg and levelRel given (levelRel(k) launches
+// device's done flag after each chunk.  tail (nullable) enqueues the traversal's closing
+// kernel after each chunk: it stores the control block in q.hostCtrl and does its work
+// only once the traversal is done; ev1 is recorded after it.  With lg and levelRel given (levelRel(k) launches
 // level levelBase + k), deep traversals replay a captured chunk of levels instead
 // (device opts use_graphs: 0 auto, 1 always, 2 never; queries with noGraphs never).
 dim3 level_grid(const DeviceGraph& g);
@@ -203,8 +207,12 @@ inline uint32_t mbfs_history_levels(uint32_t n, uint32_t nw) {
 // Returns whether dst is device memory.
 bool check_result_range(const void* dst, size_t bytes, int device, const char* what);
 // trace (nullable): record an event after the init kernel and after every level kernel.
-void bfs_launch(Query& q, uint32_t srcReordered, bool trace = false);
+// dst (nullable): the caller's device array (original order), written by the closing kernel.
+void bfs_launch(Query& q, uint32_t srcReordered, bool trace = false, int32_t* dst = nullptr);
 void bfs_finish(Query& q, int32_t* hostLevels, blest_bfs_stats* st);
+// Where a traversal may write n x rows results directly: dst when it is device memory
+// (checked to fit) apart from the query's own level array, else null.
+int32_t* direct_result(const Query& q, int32_t* dst, size_t count, const char* what);
 
 }  // namespace blest
 

@@ -164,6 +164,14 @@ __device__ __forceinline__ void level_state_reset(Ctrl* c) {
     c->state[1] = c->state[0];
 }
 
+// The control block to its pinned host copy (one workgroup of at least 64 threads).
+__device__ __forceinline__ void publish_ctrl(const Ctrl* c, Ctrl* host) {
+    constexpr unsigned kWords = sizeof(Ctrl) / sizeof(unsigned);
+    static_assert(kWords == 64, "a word per thread of one wave");
+    if (threadIdx.x < kWords)
+        reinterpret_cast<unsigned*>(host)[threadIdx.x] = reinterpret_cast<const unsigned*>(c)[threadIdx.x];
+}
+
 // Level of a kernel: fixed at launch, or (in a replayed chunk of levels) the chunk's
 // base level held in ctrl plus the kernel's position in the chunk.
 __device__ __forceinline__ unsigned level_of(const Ctrl* c, int fromCtrl, unsigned L) {

@@ -739,12 +739,16 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID mbfs_updat
 // from five bit-planes (plane b = OR of the words of the levels with bit b set), so a
 // vertex costs its history words in and its k levels out, nothing else.  Pairs found
 // past the history were written when found; the rest are unreached (-1).  Root-major
-// rows: for each root the threads store consecutive levels.  Idempotent: enqueued ahead
-// of each completion poll, it reads only levels whose words are complete.
+// rows: for each root the threads store consecutive levels, into the query's level array
+// and, in natural order, the caller's device array (dst, nullable) at once.  Enqueued
+// ahead of each completion poll; until the traversal is done it only publishes the control
+// block.
 constexpr unsigned kFinalBlock = 256;
 
 template <int NW>
-__global__ void __launch_bounds__(kFinalBlock) mbfs_final_kernel(GraphView g, MbfsArgs a) {
+__global__ void __launch_bounds__(kFinalBlock) mbfs_final_kernel(GraphView g, MbfsArgs a, int32_t* dst, Ctrl* host) {
+    if (blockIdx.x == 0) publish_ctrl(a.ctrl, host);
+    if (!ld_relaxed(&a.ctrl->done)) return;
     const unsigned top = min(__hip_atomic_load(&a.ctrl->histTop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
                              a.histLevels);
     for (uint32_t v = blockIdx.x * kFinalBlock + threadIdx.x; v < g.n; v += gridDim.x * kFinalBlock) {
@@ -762,16 +766,19 @@ __global__ void __launch_bounds__(kFinalBlock) mbfs_final_kernel(GraphView g, Mb
             const unsigned long long vis = vis_at<NW>(a, v)[i];
             const unsigned jn = min(64u, a.k - 64u * i);
             for (unsigned j = 0; j < jn; ++j) {
-                int32_t* out = a.levels + size_t(64 * i + j) * g.n + v;
+                const size_t at = size_t(64 * i + j) * g.n + v;
                 // streaming stores: the k x n output is written once and not read here
+                int32_t l = -1;
                 if ((inHist >> j) & 1ull) {
-                    int32_t l = 0;
+                    l = 0;
 #pragma unroll
                     for (int b = 0; b < 5; ++b) l |= int32_t((plane[b] >> j) & 1ull) << b;
-                    __builtin_nontemporal_store(l, out);
-                } else if (!((vis >> j) & 1ull)) {
-                    __builtin_nontemporal_store(int32_t(-1), out);
+                } else if ((vis >> j) & 1ull) {
+                    if (dst) dst[at] = a.levels[at];  // past the history: stored when found
+                    continue;
                 }
+                __builtin_nontemporal_store(l, a.levels + at);
+                if (dst) __builtin_nontemporal_store(l, dst + at);
             }
         }
     }
@@ -866,7 +873,7 @@ static void mbfs_ensure_state(Query& q, uint32_t nw) {
 }
 
 template <int NW, int ALGO>
-static void mbfs_enqueue_levels(Query& q, const dev::MbfsArgs& a) {
+static void mbfs_enqueue_levels(Query& q, const dev::MbfsArgs& a, int32_t* dst) {
     DeviceGraph& g = *q.g;
     const GraphView gv = g.view();
     const dim3 grid = level_grid(g), block(dev::kProducerBlock), eblock(dev::mbfs_expand_block<NW>());
@@ -883,7 +890,8 @@ static void mbfs_enqueue_levels(Query& q, const dev::MbfsArgs& a) {
         },
         [&] {
             const uint32_t fb = std::min<uint32_t>((g.n + dev::kFinalBlock - 1) / dev::kFinalBlock, uint32_t(g.cus) * 8);
-            hipLaunchKernelGGL(dev::mbfs_final_kernel<NW>, dim3(fb), dim3(dev::kFinalBlock), 0, q.stream, gv, a);
+            hipLaunchKernelGGL(dev::mbfs_final_kernel<NW>, dim3(fb), dim3(dev::kFinalBlock), 0, q.stream, gv, a, dst,
+                               q.hostCtrl);
         },
         &q.graphs[NW == 1 ? kGraphMbfs1 : kGraphMbfs2],
         [&](unsigned k) {
@@ -904,7 +912,8 @@ static void mbfs_run(Query& q, const uint32_t* srcs, uint32_t k, int32_t* hostLe
     if (algo != 0 && algo != 1) throw Error(BLEST_ERR_INVALID_ARGUMENT, "algo must be 0 (bit-parallel) or 1 (i8 MFMA)");
     const uint32_t nw = (k > 64 || (o && o->batch > 64)) ? 2 : 1;
     // result destinations are checked before anything runs
-    if (hostLevels) check_result_range(hostLevels, sizeof(int32_t) * size_t(g.n) * k, g.device, "levels");
+    int32_t* const direct = direct_result(q, hostLevels, size_t(g.n) * k, "levels");
+    int32_t* const dst = g.hasPerm ? nullptr : direct;  // written by the closing kernel
     if (rows)
         for (uint32_t j = 0; j < k; ++j) {
             if (!rows[j]) throw Error(BLEST_ERR_INVALID_ARGUMENT, "null result row");
@@ -947,17 +956,13 @@ static void mbfs_run(Query& q, const uint32_t* srcs, uint32_t k, int32_t* hostLe
     a.levelFromCtrl = 0;
     BLEST_HIP(hipEventRecord(q.ev0, q.stream));
     if (nw == 1) {
-        if (algo == 1) mbfs_enqueue_levels<1, 1>(q, a);
-        else mbfs_enqueue_levels<1, 0>(q, a);
+        if (algo == 1) mbfs_enqueue_levels<1, 1>(q, a, dst);
+        else mbfs_enqueue_levels<1, 0>(q, a, dst);
     } else {
-        if (algo == 1) mbfs_enqueue_levels<2, 1>(q, a);
-        else mbfs_enqueue_levels<2, 0>(q, a);
+        if (algo == 1) mbfs_enqueue_levels<2, 1>(q, a, dst);
+        else mbfs_enqueue_levels<2, 0>(q, a, dst);
     }
-    BLEST_HIP(hipEventRecord(q.ev1, q.stream));
-    BLEST_HIP(hipStreamSynchronize(q.stream));
-    dev::Ctrl c;
-    BLEST_HIP(hipMemcpyAsync(&c, q.ctrl, sizeof(c), hipMemcpyDeviceToHost, q.stream));
-    BLEST_HIP(hipStreamSynchronize(q.stream));
+    const dev::Ctrl& c = *q.hostCtrl;  // as of the last poll
     q.levelHint = c.levels;
     float ms = 0;
     BLEST_HIP(hipEventElapsedTime(&ms, q.ev0, q.ev1));
@@ -988,21 +993,21 @@ static void mbfs_run(Query& q, const uint32_t* srcs, uint32_t k, int32_t* hostLe
             perRoot[j].edges_traversed_component = rs[j].degreeSum / 2;
         }
     }
-    if (hostLevels || rows) {
+    if ((hostLevels && !dst) || rows) {
         const int32_t* src = q.levels;
         if (g.hasPerm) {
+            int32_t* out = direct ? direct : q.levelsOut;
             hipLaunchKernelGGL(dev::unpermute_rows_kernel, dim3(256, std::min<uint32_t>(k, 65535)), dim3(256), 0,
-                               q.stream, q.levelsOut, q.levels, g.permOldToNew, g.n, k);
+                               q.stream, out, q.levels, g.permOldToNew, g.n, k);
             BLEST_HIP(hipGetLastError());
-            src = q.levelsOut;
+            src = out;
         }
-        if (hostLevels)
+        if (hostLevels && !direct)
             BLEST_HIP(hipMemcpyAsync(hostLevels, src, sizeof(int32_t) * size_t(g.n) * k, hipMemcpyDefault,
                                      q.stream));
-        else
-            for (uint32_t j = 0; j < k; ++j)
-                BLEST_HIP(hipMemcpyAsync(rows[j], src + size_t(g.n) * j, sizeof(int32_t) * size_t(g.n),
-                                         hipMemcpyDefault, q.stream));
+        for (uint32_t j = 0; rows && j < k; ++j)
+            BLEST_HIP(hipMemcpyAsync(rows[j], src + size_t(g.n) * j, sizeof(int32_t) * size_t(g.n),
+                                     hipMemcpyDefault, q.stream));
         BLEST_HIP(hipStreamSynchronize(q.stream));
     }
 }
