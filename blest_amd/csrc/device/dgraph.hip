@@ -6,6 +6,7 @@
 #include "dgraph.hpp"
 #include "level_common.hpp"
 #include "segments.hpp"
+#include "small_traverse.hpp"
 
 namespace blest {
 
@@ -331,7 +332,7 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                     BLEST_HIP(hipMemcpy(g.csrPtr, csr->colPtrs.data(), 4 * (size_t(c.n) + 1), hipMemcpyHostToDevice));
                     const std::vector<uint32_t>& cp = csr->colPtrs;
                     const std::vector<uint32_t>& ci = csr->rows;
-                    g.csrIdx = g.alloc<uint32_t>(csr->nnz());
+                    g.csrIdx = g.alloc<uint32_t>(csr->nnz() + dev::kBatchTd);  // small_traverse reads whole steps
                     if (opts.bu_probe >= 0) {
                         // Each vertex's in-neighbours by degree, highest first (ties by ID):
                         // high-degree vertices are reached first, so a bottom-up scan meets a
