@@ -63,26 +63,41 @@ __device__ __forceinline__ uint32_t stream_load_u32(const uint32_t* p, uint32_t 
 // ------------------------------------------------------------------ wave helpers
 __device__ __forceinline__ unsigned lane_id() { return __lane_id(); }
 
-__device__ __forceinline__ unsigned wave_inclusive_scan(unsigned x) {
-    const unsigned l = lane_id();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        unsigned y = __shfl_up(x, d, kWave);
-        if (l >= unsigned(d)) x += y;
-    }
+// Scans and sums through the VALU's own lane paths (DPP: shifts within a row of 16, then
+// the last lane of a row to the next one and of the first half to the second), one move
+// and one add a step and no LDS: a shuffle is an LDS instruction with an address and a
+// wait, and a level kernel's preamble alone did 36 of them.  Every lane must be active.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned dpp_or_zero(unsigned x) {
+    return unsigned(__builtin_amdgcn_update_dpp(0, int(x), CTRL, ROWS, 0xf, false));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_or_zero(unsigned long long x) {
+    const unsigned lo = dpp_or_zero<CTRL, ROWS>(unsigned(x)), hi = dpp_or_zero<CTRL, ROWS>(unsigned(x >> 32));
+    return (unsigned long long)hi << 32 | lo;
+}
+
+template <class T>
+__device__ __forceinline__ T wave_inclusive_scan(T x) {
+    x += dpp_or_zero<0x111, 0xf>(x);  // row_shr 1, 2, 4, 8
+    x += dpp_or_zero<0x112, 0xf>(x);
+    x += dpp_or_zero<0x114, 0xf>(x);
+    x += dpp_or_zero<0x118, 0xf>(x);
+    x += dpp_or_zero<0x142, 0xa>(x);  // row_bcast 15: rows 1 and 3
+    x += dpp_or_zero<0x143, 0xc>(x);  // row_bcast 31: rows 2 and 3
     return x;
 }
 
+__device__ __forceinline__ unsigned read_lane(unsigned x, unsigned lane) {
+    return unsigned(__builtin_amdgcn_readlane(int(x), int(lane)));
+}
+__device__ __forceinline__ unsigned long long read_lane(unsigned long long x, unsigned lane) {
+    return (unsigned long long)read_lane(unsigned(x >> 32), lane) << 32 | read_lane(unsigned(x), lane);
+}
+
+__device__ __forceinline__ unsigned wave_sum_u32(unsigned x) { return read_lane(wave_inclusive_scan(x), kWave - 1); }
 __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long x) {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) x += __shfl_xor(x, d, kWave);
-    return x;
-}
-
-__device__ __forceinline__ unsigned wave_sum_u32(unsigned x) {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) x += __shfl_xor(x, d, kWave);
-    return x;
+    return read_lane(wave_inclusive_scan(x), kWave - 1);
 }
 
 // Largest lane j whose value excl[j] <= t, given excl ascending over lanes with

@@ -72,31 +72,23 @@ __device__ __forceinline__ bool level_begin(Ctrl* c, const SegCounters& sc, uint
     // levels enqueued past the end of the traversal stop here, before any reduction
     if (__syncthreads_or(doneIn != 0)) return false;
     // the two sums and the two scans share one exchange through LDS (one barrier, not
-    // eight): each wave posts its totals, every thread then adds up the waves before it
+    // eight): each wave posts its totals, every wave then adds up the waves before it
     {
-        const unsigned lane = lane_id(), wave = t / kWave, nw = nb / kWave;
+        const unsigned lane = lane_id(), wave = t / kWave;
         const unsigned long long wnf = wave_sum_u64(nf), wmf = wave_sum_u64(mf);
         const unsigned incl = wave_inclusive_scan(mine), cincl = wave_inclusive_scan(cmine);
         if (lane == kWave - 1) {
             s_tmp32[wave] = incl;
             s_ctmp32[wave] = cincl;
-        }
-        if (lane == 0) {
             s_tmp[wave] = wnf;
             s_etmp[wave] = wmf;
         }
         __syncthreads();
-        nf = mf = 0;
-        unsigned before = 0, cbefore = 0, tot = 0, ctot = 0;
-        for (unsigned i = 0; i < nw; ++i) {
-            nf += s_tmp[i];
-            mf += s_etmp[i];
-            const unsigned x = s_tmp32[i], y = s_ctmp32[i];
-            before += i < wave ? x : 0u;
-            cbefore += i < wave ? y : 0u;
-            tot += x;
-            ctot += y;
-        }
+        unsigned long long unused;
+        nf = wave_totals(s_tmp, unused);
+        mf = wave_totals(s_etmp, unused);
+        unsigned before = 0, cbefore = 0;
+        const unsigned tot = wave_totals(s_tmp32, before), ctot = wave_totals(s_ctmp32, cbefore);
         if (pre) {
             *total = tot;
             const unsigned ex = before + incl - mine;

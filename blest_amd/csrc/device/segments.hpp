@@ -54,21 +54,31 @@ __host__ __device__ __forceinline__ uint32_t rset_chunks(uint32_t cnt) {
     return cnt > kChunkVsets ? (cnt + kChunkVsets - 1) / kChunkVsets : 0u;
 }
 
+// The totals that the block's waves (at most 16) left in tmp: their sum over the waves
+// before this one in `before`, over all in the result.  A lane takes one wave's total and a
+// row scan adds them up: one LDS read a lane instead of one per wave and lane.
+template <class T>
+__device__ __forceinline__ T wave_totals(const T* tmp, T& before) {
+    const unsigned nw = blockDim.x / kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const T mine = lane_id() < nw ? tmp[lane_id()] : T(0);
+    T incl = mine;
+    incl += dpp_or_zero<0x111, 0xf>(incl);
+    incl += dpp_or_zero<0x112, 0xf>(incl);
+    incl += dpp_or_zero<0x114, 0xf>(incl);
+    incl += dpp_or_zero<0x118, 0xf>(incl);
+    before = read_lane(T(incl - mine), wave);
+    return read_lane(incl, 15);
+}
+
 // Exclusive scan over the block (blockDim.x <= 1024, multiple of 64); returns the
 // thread's exclusive prefix and the block total.  `tmp` holds >= 16 entries.
 __device__ __forceinline__ unsigned block_exclusive_scan(unsigned x, unsigned* tmp, unsigned& total) {
-    const unsigned lane = lane_id(), wave = threadIdx.x / kWave, nw = blockDim.x / kWave;
     const unsigned incl = wave_inclusive_scan(x);
     __syncthreads();
-    if (lane == kWave - 1) tmp[wave] = incl;
+    if (lane_id() == kWave - 1) tmp[threadIdx.x / kWave] = incl;
     __syncthreads();
-    unsigned before = 0, all = 0;
-    for (unsigned i = 0; i < nw; ++i) {
-        const unsigned t = tmp[i];
-        before += (i < wave) ? t : 0u;
-        all += t;
-    }
-    total = all;
+    unsigned before;
+    total = wave_totals(tmp, before);
     return before + incl - x;
 }
 
@@ -76,37 +86,28 @@ __device__ __forceinline__ unsigned block_exclusive_scan(unsigned x, unsigned* t
 // scan): returns x's exclusive prefix, y's in ey, and the totals.  `tmp` holds >= 32.
 __device__ __forceinline__ unsigned block_exclusive_scan2(unsigned x, unsigned y, unsigned* tmp, unsigned& total,
                                                           unsigned& ey, unsigned& ytotal) {
-    const unsigned lane = lane_id(), wave = threadIdx.x / kWave, nw = blockDim.x / kWave;
+    const unsigned wave = threadIdx.x / kWave;
     const unsigned ix = wave_inclusive_scan(x), iy = wave_inclusive_scan(y);
     __syncthreads();
-    if (lane == kWave - 1) {
+    if (lane_id() == kWave - 1) {
         tmp[wave] = ix;
         tmp[16 + wave] = iy;
     }
     __syncthreads();
-    unsigned bx = 0, by = 0, ax = 0, ay = 0;
-    for (unsigned i = 0; i < nw; ++i) {
-        const unsigned tx = tmp[i], ty = tmp[16 + i];
-        bx += (i < wave) ? tx : 0u;
-        by += (i < wave) ? ty : 0u;
-        ax += tx;
-        ay += ty;
-    }
-    total = ax;
-    ytotal = ay;
+    unsigned bx, by;
+    total = wave_totals(tmp, bx);
+    ytotal = wave_totals(tmp + 16, by);
     ey = by + iy - y;
     return bx + ix - x;
 }
 
 __device__ __forceinline__ unsigned long long block_sum_u64(unsigned long long x, unsigned long long* tmp) {
-    const unsigned lane = lane_id(), wave = threadIdx.x / kWave, nw = blockDim.x / kWave;
     x = wave_sum_u64(x);
     __syncthreads();
-    if (lane == 0) tmp[wave] = x;
+    if (lane_id() == 0) tmp[threadIdx.x / kWave] = x;
     __syncthreads();
-    unsigned long long s = 0;
-    for (unsigned i = 0; i < nw; ++i) s += tmp[i];
-    return s;
+    unsigned long long before;
+    return wave_totals(tmp, before);
 }
 
 // Loads a [segs] count row into LDS as an inclusive prefix (pre[i] = sum of counts
