@@ -291,6 +291,7 @@ __global__ void __launch_bounds__(kFusedBlock) bfs_fused_kernel(GraphView g, Bfs
     dp.beta = a.beta;
     dp.totalEdges = g.nnz;
     dp.totalItems = double(g.n);
+    dp.weighEdges = true;
     bool bottomUp = false;
     unsigned total = 0, ctotal = 0, Le = 0;
     LevelState cur, in;  // state of the level about to be expanded, and of the one before
@@ -491,6 +492,7 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID bfs_expand
     dp.beta = a.beta;
     dp.totalEdges = g.nnz;
     dp.totalItems = double(g.n);
+    dp.weighEdges = true;
     Ctrl* c = a.ctrl;
     const uint32_t segs = a.sv.segs;
     bool bottomUp = false;
@@ -774,9 +776,13 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID bfs_update
     unsigned long long* nb64 = reinterpret_cast<unsigned long long*>(a.nextB);
     const unsigned long long firstNB = nb64[size_t(w1) * 8 + b], firstFout = fout[w1];
     // a bottom-up level's discovery counts are complete (its expand kernel wrote them)
-    unsigned long long nfPart = 0;
+    unsigned long long nfPart = 0, mfPart = 0;
+    const unsigned long long cumEdges = c->state[L & 1].cumEdges;
     if (dir != 0)
-        for (uint32_t s = t; s < segs; s += nb) nfPart += a.sc.news[size_t(sOut) * segs + s];
+        for (uint32_t s = t; s < segs; s += nb) {
+            nfPart += a.sc.news[size_t(sOut) * segs + s];
+            mfPart += a.sc.edges[size_t(sOut) * segs + s];
+        }
     if (done) return;
     const bool bottomUp = dir != 0;
     const unsigned Le = L + shift;  // the level's distance
@@ -787,9 +793,10 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID bfs_update
         // The lists serve a top-down next level only.  Its direction is level_begin's rule
         // on the same inputs (this level's state and discovery count): when it stays
         // bottom-up, or nothing was discovered, no list is written.
-        const unsigned long long nf = block_sum_u64(nfPart, tmp64);
+        const unsigned long long nf = block_sum_u64(nfPart, tmp64), mf = block_sum_u64(mfPart, tmp64);
+        const double mu = double(g.nnz - min(cumEdges + mf, (unsigned long long)g.nnz));
         const bool nextBottomUp = (a.direction == 0 && canBU)
-                                      ? !(double(nf) * a.beta < double(g.n) && nf < prevNf)
+                                      ? !back_to_top_down(nf, mf, mu, prevNf, a.beta, double(g.n), true)
                                       : (a.direction == 2 && canBU);
         if (nf == 0 || nextBottomUp) {
             if (t == 0) {

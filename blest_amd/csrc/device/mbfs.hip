@@ -418,6 +418,7 @@ mbfs_expand_kernel(GraphView g, MbfsArgs a, unsigned Lk) {
     dp.beta = a.beta;
     dp.totalEdges = (unsigned long long)a.k * g.nnz;
     dp.totalItems = double(g.n) * a.k;
+    dp.weighEdges = false;
     bool bottomUp = false;
     unsigned total = 0;  // list entries of the level (top-down)
     if (!level_begin(c, a.sc, segs, L, dp, bottomUp, pre, &total)) return;
