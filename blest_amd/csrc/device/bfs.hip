@@ -1024,9 +1024,9 @@ void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
         return;
     }
     const auto close = [&] {
-        hipLaunchKernelGGL(dev::bfs_final_kernel, grid, block, 0, q.stream, gv, a, oldToNew, dst, q.hostCtrl);
+        hipLaunchKernelGGL(dev::bfs_final_kernel, wide_grid(g), block, 0, q.stream, gv, a, oldToNew, dst, q.hostCtrl);
     };
-    hipLaunchKernelGGL(dev::bfs_init_kernel, grid, block, 0, q.stream, gv, a);
+    hipLaunchKernelGGL(dev::bfs_init_kernel, wide_grid(g), block, 0, q.stream, gv, a);
     // small levels between chunks of level kernels: from the root, and after every chunk
     const bool fused = a.fuseQuads != 0;
     if (fused) hipLaunchKernelGGL(dev::bfs_fused_kernel, dim3(1), dim3(dev::kFusedBlock), 0, q.stream, gv, a, 1u, 1);

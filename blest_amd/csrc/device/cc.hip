@@ -525,9 +525,9 @@ static void cc_run(Query& q, int algo, uint32_t* hostLabels, blest_cc_stats* st)
         a.list0 = q.list0;
         a.list1 = q.list1;
         a.ctrl = q.ctrl;
-        a.sv = g.seg_view();
+        a.sv = g.wide_view();
         a.sc = q.seg_counters();
-        const dim3 lg = level_grid(g), lb(dev::kProducerBlock);
+        const dim3 lg = wide_grid(g), lb(dev::kProducerBlock);
         hipLaunchKernelGGL(dev::cc_lp_init_kernel, lg, lb, 0, q.stream, gv, a);
         run_levels(q, [&](unsigned L) {
             hipLaunchKernelGGL(dev::cc_lp_expand_kernel, lg, lb, 0, q.stream, gv, a, L);

@@ -29,8 +29,11 @@ Query::~Query() {
 }
 
 dim3 level_grid(const DeviceGraph& g) { return dim3(g.segs); }
+dim3 wide_grid(const DeviceGraph& g) { return dim3(g.wideSegs); }
 
 dev::SegView DeviceGraph::seg_view() const { return dev::SegView{segs, wps, segBase, chunkBase}; }
+
+dev::SegView DeviceGraph::wide_view() const { return dev::SegView{wideSegs, wideWps, wideBase, nullptr}; }
 
 dev::SegCounters Query::seg_counters() const { return dev::SegCounters{segCount, segNew, segEdges, segChunks}; }
 
@@ -242,19 +245,34 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
             g.W = (b.n + 63) / 64;
             g.S = b.noSlices;
             if (b.noSlices / 4 > 0xFFFFFFFFull) throw Error(BLEST_ERR_UNSUPPORTED, "more than 2^32 slice quads");
-            // Segments: one producer workgroup per contiguous run of bitmap words.
-            g.segs = std::min<uint32_t>(std::min<uint32_t>(uint32_t(g.cus) * g.blocksPerCu, dev::kMaxSegs), g.W);
-            g.wps = (g.W + g.segs - 1) / g.segs;
-            g.segs = (g.W + g.wps - 1) / g.wps;
+            // Segments: one producer workgroup per contiguous run of bitmap words, at most
+            // blocks_per_cu per CU.  Every workgroup of a level kernel first reads every
+            // segment's counters, and its instructions are most of a small level's time, so
+            // a bottom-up-capable graph gets segments of kSegmentWords (a full group for
+            // each wave) as long as every CU has one.  Mean expansion and update at 4 and
+            // 1 workgroups per CU: R-MAT 16 14.3 + 5.7 and 9.2 + 3.6 us, R-MAT 18 14.9 + 6.2
+            // and 10.0 + 4.5; past the limit it turns (2047-square grid 18.3 + 7.9 and
+            // 23.1 + 10.6, R-MAT 22 19.6 + 7.2 and 23.8 + 8.3).
+            constexpr uint32_t kSegmentWords = 64;
+            const auto cut = [&](uint32_t want, uint32_t& segs, uint32_t& wps) {
+                segs = std::min(want, g.W);
+                wps = (g.W + segs - 1) / segs;
+                segs = (g.W + wps - 1) / wps;
+            };
+            const auto list_base = [&](uint32_t segs, uint32_t wps) {
+                std::vector<uint32_t> sb(size_t(segs) + 1);
+                for (uint32_t s = 0; s <= segs; ++s) sb[s] = b.realPtrs[std::min<uint64_t>(uint64_t(s) * wps * 8, g.R)];
+                uint32_t* d = g.alloc<uint32_t>(sb.size());
+                BLEST_HIP(hipMemcpy(d, sb.data(), 4 * sb.size(), hipMemcpyHostToDevice));
+                return d;
+            };
+            const uint32_t most = std::min<uint32_t>(uint32_t(g.cus) * g.blocksPerCu, dev::kMaxSegs);
+            cut(most, g.wideSegs, g.wideWps);
+            g.wideBase = list_base(g.wideSegs, g.wideWps);
+            cut(opts.keep_csr ? std::min(most, std::max(uint32_t(g.cus), g.W / kSegmentWords)) : most, g.segs, g.wps);
             g.gridBlocks = g.segs;
             {
-                std::vector<uint32_t> sb(size_t(g.segs) + 1);
-                for (uint32_t s = 0; s <= g.segs; ++s) {
-                    const uint64_t r = std::min<uint64_t>(uint64_t(s) * g.wps * 8, g.R);
-                    sb[s] = b.realPtrs[r];
-                }
-                g.segBase = g.alloc<uint32_t>(sb.size());
-                BLEST_HIP(hipMemcpy(g.segBase, sb.data(), 4 * sb.size(), hipMemcpyHostToDevice));
+                g.segBase = g.segs == g.wideSegs ? g.wideBase : list_base(g.segs, g.wps);
                 // chunk slots: segment s may emit the chunks of its own rsets only
                 std::vector<uint32_t> cb(size_t(g.segs) + 1, 0);
                 uint64_t total = 0;
@@ -482,10 +500,10 @@ blest_status blest_query_create(blest_device_graph* dg, uint32_t max_sources, bl
             q.list1 = q.alloc<uint32_t>(g.V);
             q.chunk0 = q.alloc<uint2>(g.chunks);
             q.chunk1 = q.alloc<uint2>(g.chunks);
-            q.segChunks = q.alloc<uint32_t>(3 * size_t(g.segs));
-            q.segCount = q.alloc<uint32_t>(3 * size_t(g.segs));
-            q.segNew = q.alloc<uint32_t>(3 * size_t(g.segs));
-            q.segEdges = q.alloc<unsigned long long>(3 * size_t(g.segs));
+            q.segChunks = q.alloc<uint32_t>(3 * size_t(g.wideSegs));
+            q.segCount = q.alloc<uint32_t>(3 * size_t(g.wideSegs));
+            q.segNew = q.alloc<uint32_t>(3 * size_t(g.wideSegs));
+            q.segEdges = q.alloc<unsigned long long>(3 * size_t(g.wideSegs));
             if (g.hasPerm) q.levelsOut = q.alloc<int32_t>(size_t(g.n) * max_sources);
         } catch (...) {
             delete h;
@@ -532,7 +550,7 @@ blest_status blest_query_footprint(const blest_device_graph* dg, uint32_t max_so
         uint64_t b = sizeof(dev::Ctrl);
         const uint64_t levels = 4ull * g.n * max_sources;
         b += levels * (g.hasPerm ? 2 : 1);
-        b += 4ull * 8ull * g.W + 64ull * g.W + 2ull * 4ull * g.V + 2ull * 8ull * g.chunks + 3ull * 20ull * g.segs;
+        b += 4ull * 8ull * g.W + 64ull * g.W + 2ull * 4ull * g.V + 2ull * 8ull * g.chunks + 3ull * 20ull * g.wideSegs;
         if (max_sources > 1) {
             const uint32_t nw = max_sources > 64 ? 2 : 1;
             b += (4ull + mbfs_history_levels(g.n, nw) + 1) * 8ull * g.n * nw + 4ull * 128 + 16ull * 128;

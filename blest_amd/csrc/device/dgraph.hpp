@@ -53,11 +53,17 @@ struct DeviceGraph {
     int device = 0;
     int cus = 0;
     uint32_t blockSize = 256, blocksPerCu = 4, gridBlocks = 0;
-    uint32_t segs = 1, wps = 1;    // producer segments and bitmap words per segment
+    // Producer segments of the single-source level kernels (one workgroup each), and the
+    // wider set of the multi-source and label-propagation kernels, whose levels stream
+    // records for long enough to want every workgroup slot.
+    uint32_t segs = 1, wps = 1;    // segments and bitmap words per segment
     uint32_t* segBase = nullptr;   // segs + 1 first list slots
     uint32_t* chunkBase = nullptr; // segs + 1 first chunk slots (rsets of > kChunkVsets vsets)
     uint64_t chunks = 0;           // chunk slots in all
+    uint32_t wideSegs = 1, wideWps = 1;
+    uint32_t* wideBase = nullptr;  // wideSegs + 1 first list slots (no chunk lists)
     dev::SegView seg_view() const;
+    dev::SegView wide_view() const;
     blest_device_opts opts{};
     uint32_t n = 0, R = 0, V = 0, W = 0;
     uint64_t S = 0, Q = 0, nnz = 0;
@@ -131,9 +137,9 @@ struct Query {
     uint8_t* nextB = nullptr;  // single-source top-down discoveries, a byte per vertex (W * 64)
     uint32_t *list0 = nullptr, *list1 = nullptr;
     uint2 *chunk0 = nullptr, *chunk1 = nullptr;        // chunk lists (single-source BFS)
-    uint32_t *segCount = nullptr, *segNew = nullptr;  // [3][segs]
-    uint32_t* segChunks = nullptr;                     // [3][segs]
-    unsigned long long* segEdges = nullptr;            // [3][segs]
+    uint32_t *segCount = nullptr, *segNew = nullptr;  // [3][segments]
+    uint32_t* segChunks = nullptr;                     // [3][segments]
+    unsigned long long* segEdges = nullptr;            // [3][segments]
     dev::SegCounters seg_counters() const;
     int32_t* levelsOut = nullptr;  // original-order copy (when the graph carries a permutation)
     uint32_t* labels = nullptr;    // CC
@@ -183,6 +189,7 @@ struct Query {
 // level levelBase + k), deep traversals replay a captured chunk of levels instead
 // (device opts use_graphs: 0 auto, 1 always, 2 never; queries with noGraphs never).
 dim3 level_grid(const DeviceGraph& g);
+dim3 wide_grid(const DeviceGraph& g);
 // after / afterRel (nullable): a kernel enqueued after each chunk of levels, given the
 // next level (absolute / relative to the replayed chunk); with it the first chunk is the
 // previous traversal's levelHint levels instead of levelHint + 2.

@@ -877,7 +877,7 @@ template <int NW, int ALGO>
 static void mbfs_enqueue_levels(Query& q, const dev::MbfsArgs& a, int32_t* dst) {
     DeviceGraph& g = *q.g;
     const GraphView gv = g.view();
-    const dim3 grid = level_grid(g), block(dev::kProducerBlock), eblock(dev::mbfs_expand_block<NW>());
+    const dim3 grid = wide_grid(g), block(dev::kProducerBlock), eblock(dev::mbfs_expand_block<NW>());
     hipLaunchKernelGGL(dev::mbfs_init_kernel<NW>, grid, block, 0, q.stream, gv, a);
     hipLaunchKernelGGL(dev::mbfs_seed_kernel<NW>, dim3(2), dim3(64), 0, q.stream, gv, a);
     hipLaunchKernelGGL(dev::mbfs_first_list_kernel<NW>, grid, block, 0, q.stream, gv, a);
@@ -940,7 +940,7 @@ static void mbfs_run(Query& q, const uint32_t* srcs, uint32_t k, int32_t* hostLe
     a.srcs = q.srcs;
     a.k = k;
     a.ctrl = q.ctrl;
-    a.sv = g.seg_view();
+    a.sv = g.wide_view();
     a.sc = q.seg_counters();
     // Direction.  A symmetric graph pulls over the BVSS slices on bottom-up levels
     // (mbfs_pull), and switches by the graph's thresholds (direction 0) unless one

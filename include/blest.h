@@ -194,7 +194,9 @@ typedef struct blest_query blest_query;
 typedef struct blest_device_opts {
     int device;              /* HIP device ordinal */
     uint32_t block_size;     /* informational: the level kernels run 512-thread workgroups */
-    uint32_t blocks_per_cu;  /* 1..8: frontier segments (= workgroups per level kernel) per CU */
+    uint32_t blocks_per_cu;  /* 1..8: frontier segments (= workgroups per level kernel) per CU, at most:
+                                graphs with a resident CSR get segments of 4096 vertices down to one
+                                a CU for the single-source level kernels */
     double alpha;            /* top-down -> bottom-up when frontier edges > unexplored edges / alpha */
     double beta;             /* bottom-up -> top-down when frontier vertices < n / beta */
     int direction;           /* 0 = optimizing, 1 = top-down only, 2 = bottom-up after level 1 */
