@@ -191,6 +191,18 @@ BVSS bvss_build(const CSC& g, uint32_t sliceSize, uint32_t noMasks, bool fullPad
 }
 
 void bvss_compute_stats(BVSS& b) {
+    const uint32_t conceal = b.sliceSize == 32 ? 0xFFFFFFFFu : ((1u << b.sliceSize) - 1);
+    uint64_t real = 0, edges = 0;
+    for (uint64_t w = 0; w < b.masks.size(); ++w)
+        for (uint32_t p = 0; p < b.noMasks; ++p) {
+            uint32_t pat = (b.masks[w] >> (p * b.sliceSize)) & conceal;
+            real += pat != 0;
+            edges += uint32_t(std::popcount(pat));
+        }
+    bvss_compute_stats(b, real, edges);
+}
+
+void bvss_compute_stats(BVSS& b, uint64_t realSlices, uint64_t edges) {
     const uint32_t V = b.noVirtualSliceSets;
     double avg = 0;
     uint32_t mn = kNoVertex, mx = 0;
@@ -210,17 +222,8 @@ void bvss_compute_stats(BVSS& b) {
     b.stdSlices = V ? std::sqrt(var / V) : 0;
     b.minSlices = V ? mn : 0;
     b.maxSlices = mx;
-    const uint32_t conceal = b.sliceSize == 32 ? 0xFFFFFFFFu : ((1u << b.sliceSize) - 1);
-    uint64_t padded = 0, edges = 0;
-    for (uint64_t w = 0; w < b.masks.size(); ++w)
-        for (uint32_t p = 0; p < b.noMasks; ++p) {
-            uint32_t pat = (b.masks[w] >> (p * b.sliceSize)) & conceal;
-            uint32_t e = uint32_t(std::popcount(pat));
-            padded += e == 0;
-            edges += e;
-        }
-    b.noPaddedSlices = padded;
-    b.noUnpaddedSlices = b.noSlices - padded;
+    b.noPaddedSlices = b.noSlices - realSlices;
+    b.noUnpaddedSlices = realSlices;
     b.edgesCheck = edges;
     b.compressionRatio = b.noUnpaddedSlices ? (double(edges) / double(b.noUnpaddedSlices)) / b.sliceSize : 0;
 }

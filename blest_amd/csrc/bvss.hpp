@@ -38,6 +38,8 @@ void bvss_check_shape(uint32_t sliceSize, uint32_t noMasks);
 BVSS bvss_build(const CSC& g, uint32_t sliceSize, uint32_t noMasks, bool fullPadding,
                 unsigned threads = 0);
 void bvss_compute_stats(BVSS& b);
+// The same with the slices and edges already counted.
+void bvss_compute_stats(BVSS& b, uint64_t realSlices, uint64_t edges);
 // Checks that b's arrays form a BVSS of the reference layout that the device can run:
 // prefix-summed sliceSetPtrs / realPtrs, virtualToReal consistent with realPtrs,
 // R = ceil(n / sliceSize), vsets of whole mask words, row IDs below n (or the pad row

@@ -25,6 +25,7 @@
 
 #include "../bvss.hpp"
 #include "dgraph.hpp"
+#include "scratch.hpp"
 
 namespace blest {
 namespace dev {
@@ -82,6 +83,16 @@ __global__ void bb_slices_kernel(const uint32_t* keys, const uint32_t* flag, con
         sRows[sbase + pos[e]] = keys[e] >> 3;
         sMasks[sbase + pos[e]] = uint8_t(m);
     }
+}
+
+// Column bits of a workgroup's share of the slice masks (the edges the bit matrix holds).
+__global__ void __launch_bounds__(256) bb_edges_kernel(const uint8_t* sMasks, unsigned long long sreal,
+                                                       unsigned long long* perBlock) {
+    __shared__ unsigned long long tmp[16];
+    unsigned long long bits = 0;
+    for (uint64_t s = blockIdx.x * 256ull + threadIdx.x; s < sreal; s += gridDim.x * 256ull) bits += __popc(sMasks[s]);
+    bits = block_sum_u64(bits, tmp);
+    if (threadIdx.x == 0) perBlock[blockIdx.x] = bits;
 }
 
 // slices of rset r0 + i: slice number of its first entry to that of the next rset's
@@ -192,44 +203,7 @@ __global__ void bb_divergence_kernel(const unsigned long long* sliceSetPtrs, con
 
 namespace {
 
-// Device buffers of one construction, freed together.
-struct Scratch {
-    std::vector<void*> ptrs;
-    template <class T>
-    T* alloc(size_t count) {
-        void* p = nullptr;
-        BLEST_HIP(hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)));
-        ptrs.push_back(p);
-        return static_cast<T*>(p);
-    }
-    ~Scratch() {
-        for (void* p : ptrs) (void)hipFree(p);
-    }
-};
-
-struct StreamGuard {
-    hipStream_t s = nullptr;
-    ~StreamGuard() {
-        if (s) {
-            (void)hipStreamSynchronize(s);
-            (void)hipStreamDestroy(s);
-        }
-    }
-};
-
 constexpr uint64_t kBatchItems = uint64_t(1) << 28;
-
-dim3 grid_for(uint64_t items, unsigned block = 256) {
-    return dim3(unsigned(std::max<uint64_t>(1, std::min<uint64_t>((items + block - 1) / block, 65536))));
-}
-
-template <class T>
-T read_one(const T* d, hipStream_t s) {
-    T v{};
-    BLEST_HIP(hipMemcpyAsync(&v, d, sizeof(T), hipMemcpyDeviceToHost, s));
-    BLEST_HIP(hipStreamSynchronize(s));
-    return v;
-}
 
 BVSS bvss_build_on_device(const CSC& g, bool fullPadding, int device) {
     BLEST_HIP(hipSetDevice(device));
@@ -349,6 +323,9 @@ BVSS bvss_build_on_device(const CSC& g, bool fullPadding, int device) {
     hipLaunchKernelGGL(dev::bb_scatter_kernel, grid_for(sreal), dim3(256), 0, st, sRows, sMasks,
                        (unsigned long long)sreal, sliceStart, rsetSlot, R, int(fullPadding), dRowIds,
                        reinterpret_cast<uint8_t*>(dMasks));
+    constexpr uint32_t kCountBlocks = 1024;
+    unsigned long long* dBits = sc.alloc<unsigned long long>(kCountBlocks);
+    hipLaunchKernelGGL(dev::bb_edges_kernel, dim3(kCountBlocks), dim3(256), 0, st, sMasks, (unsigned long long)sreal, dBits);
     hipLaunchKernelGGL(dev::bb_divergence_kernel, grid_for(V), dim3(256), 0, st, dSsp, dRowIds, V, dTerm);
     BLEST_HIP(hipGetLastError());
 
@@ -366,6 +343,8 @@ BVSS bvss_build_on_device(const CSC& g, bool fullPadding, int device) {
     b.rowIds.resize(S);
     b.masks.resize(S / 4);
     std::vector<double> term(V);
+    std::vector<unsigned long long> bits(kCountBlocks);
+    BLEST_HIP(hipMemcpyAsync(bits.data(), dBits, 8 * bits.size(), hipMemcpyDeviceToHost, st));
     BLEST_HIP(hipMemcpyAsync(b.sliceSetPtrs.data(), dSsp, 8 * (size_t(V) + 1), hipMemcpyDeviceToHost, st));
     if (V) BLEST_HIP(hipMemcpyAsync(b.virtualToReal.data(), dV2r, 4 * size_t(V), hipMemcpyDeviceToHost, st));
     BLEST_HIP(hipMemcpyAsync(b.realPtrs.data(), realPtrs, 4 * (size_t(R) + 1), hipMemcpyDeviceToHost, st));
@@ -378,7 +357,9 @@ BVSS bvss_build_on_device(const CSC& g, bool fullPadding, int device) {
     double div = 0;
     for (uint32_t v = 0; v < V; ++v) div += term[v];  // the host construction's summation order
     b.updateDivergence = V ? div / V : 0.0;
-    bvss_compute_stats(b);
+    uint64_t edges = 0;
+    for (unsigned long long x : bits) edges += x;
+    bvss_compute_stats(b, sreal, edges);
     return b;
 }
 
