@@ -1,0 +1,19 @@
+// Preparation of the resident CSR on the GPU (current device; every call is complete on
+// return).  ptr: n + 1 ascending list offsets, idx: the entries.
+#pragma once
+
+#include "../csc.hpp"
+
+namespace blest {
+
+// Whether every stored edge has its reverse (columns sorted); throws
+// BLEST_ERR_INVALID_ARGUMENT for an entry that is not below n.
+bool csr_symmetric_on_device(const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t nnz);
+// Orders every list by degree, highest first, ties by ID; csr: the same lists on the host.
+void csr_sort_by_degree(const CSC& csr, const uint32_t* ptr, uint32_t* idx);
+// probe (nullable): each list's first entry, 0 for an empty one; noIn: bit v of the words
+// set where list v is empty.
+void csr_marks(const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t words, uint32_t* probe,
+               unsigned long long* noIn);
+
+}  // namespace blest

@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "csr_build.hpp"
 #include "dgraph.hpp"
 #include "level_common.hpp"
 #include "segments.hpp"
@@ -201,6 +202,28 @@ void blest_device_opts_default(blest_device_opts* o) {
 
 }  // extern "C"
 
+// On the device; on the host where the sort's scratch (about 2 GiB at most, 16 bytes a
+// vertex) does not fit beside the graph or a list is longer than a device sort takes.
+static void sort_lists_by_degree(const CSC& csr, const uint32_t* ptr, uint32_t* idx) {
+    try {
+        csr_sort_by_degree(csr, ptr, idx);
+        return;
+    } catch (const Error& e) {
+        if (e.code != BLEST_ERR_OUT_OF_DEVICE_MEMORY && e.code != BLEST_ERR_UNSUPPORTED) throw;
+        (void)hipGetLastError();
+    }
+    const std::vector<uint32_t>& cp = csr.colPtrs;
+    std::vector<uint32_t> sorted(csr.rows);
+    parallel_blocks(csr.n, hw_threads(), [&](uint64_t v0, uint64_t v1, unsigned) {
+        for (uint64_t v = v0; v < v1; ++v)
+            std::sort(sorted.data() + cp[v], sorted.data() + cp[v + 1], [&](uint32_t x, uint32_t y) {
+                const uint32_t dx = cp[x + 1] - cp[x], dy = cp[y + 1] - cp[y];
+                return dx != dy ? dx > dy : x < y;
+            });
+    });
+    BLEST_HIP(hipMemcpy(idx, sorted.data(), 4 * sorted.size(), hipMemcpyHostToDevice));
+}
+
 // gh: the CSC the BVSS was built from (ghIsCsr = false; its transpose is the bottom-up
 // CSR unless the graph is symmetric), or that transpose itself (ghIsCsr = true, as the
 // reference's BVSS keeps it, BVSS::getCSR()).
@@ -336,21 +359,32 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                     throw Error(BLEST_ERR_INVALID_ARGUMENT, ghIsCsr ? "CSR and BVSS disagree on n"
                                                                     : "CSC and BVSS disagree on n");
                 g.nnz = c.nnz();
-                g.symmetric = csc_is_symmetric(c);  // a graph is symmetric iff its transpose is
-                if (opts.keep_csr) {
+                // a graph is symmetric iff its transpose is
+                if (!opts.keep_csr) {
+                    g.symmetric = csc_is_symmetric(c);
+                } else {
+                    for (uint32_t v = 0; v < c.n; ++v)
+                        if (c.colPtrs[v + 1] < c.colPtrs[v])
+                            throw Error(BLEST_ERR_INVALID_ARGUMENT, "col_ptrs not monotone");
+                    if (c.colPtrs[0] != 0 || c.colPtrs[c.n] != c.nnz())
+                        throw Error(BLEST_ERR_INVALID_ARGUMENT, "col_ptrs and rows disagree");
                     // Bottom-up reads in-neighbours: the CSR of the edges j -> i, i.e. the
                     // transpose of the CSC (equal to it for a symmetric graph).
                     CSC tr;
                     const CSC* csr = &c;
+                    g.csrPtr = g.alloc<uint32_t>(size_t(c.n) + 1);
+                    g.csrIdx = g.alloc<uint32_t>(c.nnz() + dev::kBatchTd);  // small_traverse reads whole steps
+                    const auto upload = [&] {
+                        BLEST_HIP(hipMemcpy(g.csrPtr, csr->colPtrs.data(), 4 * (size_t(c.n) + 1), hipMemcpyHostToDevice));
+                        if (c.nnz()) BLEST_HIP(hipMemcpy(g.csrIdx, csr->rows.data(), 4 * c.nnz(), hipMemcpyHostToDevice));
+                    };
+                    upload();
+                    g.symmetric = csr_symmetric_on_device(g.csrPtr, g.csrIdx, c.n, uint32_t(c.nnz()));
                     if (!ghIsCsr && !g.symmetric) {
                         tr = csc_transpose(c);
                         csr = &tr;
+                        upload();
                     }
-                    g.csrPtr = g.alloc<uint32_t>(size_t(c.n) + 1);
-                    BLEST_HIP(hipMemcpy(g.csrPtr, csr->colPtrs.data(), 4 * (size_t(c.n) + 1), hipMemcpyHostToDevice));
-                    const std::vector<uint32_t>& cp = csr->colPtrs;
-                    const std::vector<uint32_t>& ci = csr->rows;
-                    g.csrIdx = g.alloc<uint32_t>(csr->nnz() + dev::kBatchTd);  // small_traverse reads whole steps
                     if (opts.bu_probe >= 0) {
                         // Each vertex's in-neighbours by degree, highest first (ties by ID):
                         // high-degree vertices are reached first, so a bottom-up scan meets a
@@ -358,32 +392,13 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                         // coalesced by a sweep's first probe instead of one random index line
                         // per vertex.  Levels do not depend on the scan order, and the
                         // multi-source sweeps read whole lists.
-                        std::vector<uint32_t> sorted(ci.begin(), ci.end()), probe(c.n, 0u);
-                        parallel_blocks(c.n, hw_threads(), [&](uint64_t v0, uint64_t v1, unsigned) {
-                            for (uint64_t v = v0; v < v1; ++v) {
-                                uint32_t* b0 = sorted.data() + cp[v];
-                                uint32_t* b1 = sorted.data() + cp[v + 1];
-                                std::sort(b0, b1, [&](uint32_t x, uint32_t y) {
-                                    const uint32_t dx = cp[x + 1] - cp[x], dy = cp[y + 1] - cp[y];
-                                    return dx != dy ? dx > dy : x < y;
-                                });
-                                probe[v] = b1 > b0 ? *b0 : 0u;
-                            }
-                        });
-                        if (csr->nnz())
-                            BLEST_HIP(hipMemcpy(g.csrIdx, sorted.data(), 4 * csr->nnz(), hipMemcpyHostToDevice));
+                        sort_lists_by_degree(*csr, g.csrPtr, g.csrIdx);
                         g.probe = g.alloc<uint32_t>(c.n);
-                        BLEST_HIP(hipMemcpy(g.probe, probe.data(), 4 * size_t(c.n), hipMemcpyHostToDevice));
-                    } else if (csr->nnz()) {
-                        BLEST_HIP(hipMemcpy(g.csrIdx, ci.data(), 4 * csr->nnz(), hipMemcpyHostToDevice));
                     }
                     g.hasCsr = true;
                     // vertices without in-neighbours: a bottom-up sweep skips them
-                    std::vector<unsigned long long> noIn(g.W, 0ull);
-                    for (uint32_t v = 0; v < c.n; ++v)
-                        if (cp[v + 1] == cp[v]) noIn[v >> 6] |= 1ull << (v & 63);
                     g.noIn = g.alloc<unsigned long long>(g.W);
-                    BLEST_HIP(hipMemcpy(g.noIn, noIn.data(), 8 * size_t(g.W), hipMemcpyHostToDevice));
+                    csr_marks(g.csrPtr, g.csrIdx, c.n, g.W, g.probe, g.noIn);
                 }
             }
             if (inv_perm) {
