@@ -2,6 +2,10 @@
 // return).  ptr: n + 1 ascending list offsets, idx: the entries.
 #pragma once
 
+#include <hip/hip_runtime.h>
+
+#include <functional>
+
 #include "../csc.hpp"
 
 namespace blest {
@@ -15,5 +19,10 @@ void csr_sort_by_degree(const CSC& csr, const uint32_t* ptr, uint32_t* idx);
 // set where list v is empty.
 void csr_marks(const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t words, uint32_t* probe,
                unsigned long long* noIn);
+
+// Units of the lists longer than `own` entries: how many, and (vertex, first entry) of each
+// unit of `unit` entries into units(count), which allocates.
+void csr_list_units(const uint32_t* ptr, uint32_t n, uint32_t own, uint32_t unit,
+                    const std::function<uint2*(uint32_t)>& units);
 
 }  // namespace blest

@@ -60,6 +60,8 @@ __device__ __forceinline__ uint32_t stream_load_u32(const uint32_t* p, uint32_t 
     return __builtin_nontemporal_load(p + i);
 }
 
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
 // ------------------------------------------------------------------ wave helpers
 __device__ __forceinline__ unsigned lane_id() { return __lane_id(); }
 
@@ -98,6 +100,15 @@ __device__ __forceinline__ unsigned long long read_lane(unsigned long long x, un
 __device__ __forceinline__ unsigned wave_sum_u32(unsigned x) { return read_lane(wave_inclusive_scan(x), kWave - 1); }
 __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long x) {
     return read_lane(wave_inclusive_scan(x), kWave - 1);
+}
+
+// OR over the 16 lanes of a row, to all of them (row rotations).
+__device__ __forceinline__ unsigned long long row_or(unsigned long long x) {
+    x |= dpp_or_zero<0x128, 0xf>(x);  // row_ror 8, 4, 2, 1
+    x |= dpp_or_zero<0x124, 0xf>(x);
+    x |= dpp_or_zero<0x122, 0xf>(x);
+    x |= dpp_or_zero<0x121, 0xf>(x);
+    return x;
 }
 
 // Largest lane j whose value excl[j] <= t, given excl ascending over lanes with

@@ -399,6 +399,10 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                     // vertices without in-neighbours: a bottom-up sweep skips them
                     g.noIn = g.alloc<unsigned long long>(g.W);
                     csr_marks(g.csrPtr, g.csrIdx, c.n, g.W, g.probe, g.noIn);
+                    csr_list_units(g.csrPtr, c.n, kPullOwn, kPullUnit, [&](uint32_t count) {
+                        g.pullCount = count;
+                        return g.pullUnits = g.alloc<uint2>(count);
+                    });
                 }
             }
             if (inv_perm) {

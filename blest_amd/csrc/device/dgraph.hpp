@@ -47,7 +47,13 @@ struct GraphView {
     const uint32_t* probe;        // n: each vertex's first in-neighbour (its highest-degree one:
                                   // the lists are sorted by degree); nullable
     unsigned long long nnz;       // directed edges
+    const uint2* pullUnits;       // (vertex, first entry) of the list parts past kPullOwn entries
+    uint32_t pullCount;
 };
+
+// Multi-source pull levels: a vertex's first kPullOwn list entries are scanned by the wave
+// that owns its bitmap word, the rest in units of kPullUnit entries (pullUnits).
+constexpr uint32_t kPullOwn = 64, kPullUnit = 256;
 
 struct DeviceGraph {
     int device = 0;
@@ -73,6 +79,8 @@ struct DeviceGraph {
     uint32_t *csrPtr = nullptr, *csrIdx = nullptr;
     unsigned long long* noIn = nullptr;  // bit v: v has no in-neighbour (never found bottom-up)
     uint32_t* probe = nullptr;           // first bottom-up probe per vertex
+    uint2* pullUnits = nullptr;
+    uint32_t pullCount = 0;
     uint32_t *permNewToOld = nullptr, *permOldToNew = nullptr;  // device copies
     std::vector<uint32_t> hostOldToNew, hostNewToOld;
     std::vector<uint32_t> hostDegree;  // per (reordered) vertex, for GTEPS accounting
@@ -95,6 +103,8 @@ struct DeviceGraph {
         g.noIn = noIn;
         g.probe = probe;
         g.nnz = nnz;
+        g.pullUnits = pullUnits;
+        g.pullCount = pullCount;
         return g;
     }
     template <class T>

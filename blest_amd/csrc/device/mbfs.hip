@@ -9,10 +9,10 @@
 //   expand  top-down: a slice (row i, mask m) of rset r contributes OR_{b in m} F[8r+b]
 //             to row i: the boolean product of the slice with the 8 x 64*NW frontier
 //             block of its rset.  Roots not yet at i are OR-ed into next[i].
-//           bottom-up: workgroup per segment, lane per vertex: the roots that have not
-//             reached v pull the OR of their in-neighbours' frontier words, stopping
-//             once all are found.
-//   update  top-down: lane per vertex: new = next[v]; visited |= new; levels of the new
+//           bottom-up: the roots that have not reached v pull the OR of their
+//             in-neighbours' frontier words, stopping once all are found (over the CSR,
+//             or over the slices of a symmetric graph without one).
+//   update  lane per vertex: new = next[v]; visited |= new; levels of the new
 //             (root, vertex) pairs; both directions list the vsets of rsets holding a
 //             frontier vertex of any root.
 // Levels are written root-major: levels[j * n + v].
@@ -31,7 +31,7 @@ struct MbfsArgs {
     uint32_t histLevels;
     unsigned long long* full;    // bit v: every root has reached v (top-down skips its record)
     unsigned long long* any;     // 2 x W: bit v of half L & 1: v is in the frontier of level L for some root
-    int pull;                    // symmetric graph: bottom-up levels pull over the BVSS slices
+    int slicePull;               // symmetric graph without a CSR: bottom-up levels pull over the BVSS slices
     uint8_t* dirty;              // W bytes: word w holds a vertex whose `next` word was set this level
     uint32_t* list0;
     uint32_t* list1;
@@ -212,7 +212,158 @@ constexpr unsigned mbfs_expand_block() {
     return NW == 1 ? kProducerBlock : kProducerBlock / 2;
 }
 
-// Bottom-up level of a symmetric graph as a pull over the same BVSS slices.  For a
+// Bottom-up level over the CSR: a vertex that some root has not reached pulls the OR of its
+// in-neighbours' frontier words, highest degree first, and stops once every missing root
+// has come: hubs hold most roots early, so a long list seldom has to be read to its end,
+// and the vertices every root has reached (most of the edges, after a level or two) are
+// not looked at.  A wave takes a bitmap word:
+//   lists of at most kPullLane entries: a lane each, 4 entries per step;
+//   longer ones: a row of 16 lanes each, 16 entries per step, the row's OR by rotations,
+//     up to kPullOwn entries;
+//   the rest of the lists past kPullOwn: units of kPullUnit entries dealt out to all waves
+//     after the words, skipped when the vertex has what it needs by then.
+// A neighbour's words are loaded whether it is in the frontier or not: testing its
+// frontier-any bit first cost more than it saved (1.87, 0.52 and 0.21 ms on levels 3-5).
+// The update kernel folds `next` exactly as after a push level.
+// Bound by the random 16-byte frontier loads, a line from the Infinity Cache each (level 3:
+// about 1.2 of 1.7 ms in the units past kPullOwn).  The pull over the BVSS (below), which
+// reads every slice of an rset with one open column and ORs it into 8 accumulators, took
+// 1.83, 1.75 and 0.81 ms on levels 3-5 of 128 roots on R-MAT 22 (natural order), this one
+// 1.68, 0.43 and 0.18 ms.
+constexpr uint32_t kPullLane = 8;
+
+template <int NW>
+__device__ __forceinline__ void mbfs_pull_csr(const GraphView& g, const MbfsArgs& a, const unsigned long long* fin) {
+    const unsigned lane = lane_id(), sub = lane & 15u, row = lane >> 4;
+    const unsigned wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
+    const unsigned nwaves = (gridDim.x * blockDim.x) / kWave;
+    const Bits<NW> rootMask = root_mask<NW>(a.k);
+    for (uint32_t w = wave; w < g.W; w += nwaves) {
+        const unsigned long long open = ~a.full[w];  // the slots past n are full
+        if (!open) continue;
+        const uint32_t v = w * 64 + lane;
+        const bool mine = (open >> lane) & 1ull;
+        const uint32_t p0 = mine ? g.csrPtr[v] : 0u, p1 = mine ? g.csrPtr[v + 1] : 0u, deg = p1 - p0;
+        Bits<NW> need, got;  // roots missing at v; roots that arrive
+        need.zero();
+        got.zero();
+        if (mine) need.loadp(vis_at<NW>(a, v));
+#pragma unroll
+        for (int i = 0; i < NW; ++i) need.w[i] = mine ? ~need.w[i] & rootMask.w[i] : 0ull;
+        const bool own = mine && deg <= kPullLane;
+#pragma unroll
+        for (uint32_t s = 0; s < kPullLane; s += 4) {
+            const bool act = own && s < deg;
+            if (!__ballot(act)) break;
+            if (act) {
+                const u32x4_a4 u = *reinterpret_cast<const u32x4_a4*>(g.csrIdx + p0 + s);  // padded past the end
+                Bits<NW> F[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    F[j].zero();
+                    if (s + j < deg) F[j].load(fin, u[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int i = 0; i < NW; ++i) got.w[i] |= F[j].w[i];
+            }
+        }
+        unsigned long long longer = __ballot(mine && deg > kPullLane);
+        while (longer) {
+            int l[4];  // the lanes whose vertices the four rows take
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                l[r] = longer ? __builtin_ctzll(longer) : -1;
+                longer &= longer - 1;  // 0 stays 0
+            }
+            const int from = row == 0 ? l[0] : row == 1 ? l[1] : row == 2 ? l[2] : l[3];
+            const int at = max(from, 0);
+            const uint32_t q0 = __shfl(p0, at, kWave), end = __shfl(p1, at, kWave);  // every lane shuffles
+            const uint32_t q1 = from < 0 ? q0 : min(end, q0 + kPullOwn);
+            Bits<NW> miss, acc;
+            acc.zero();
+#pragma unroll
+            for (int i = 0; i < NW; ++i) miss.w[i] = __shfl(need.w[i], at, kWave);
+            bool done = false;
+            for (uint32_t s = 0; s < kPullOwn; s += 16) {
+                const bool act = !done && q0 + s < q1;
+                if (!__ballot(act)) break;
+                const uint32_t q = q0 + s + sub;
+                Bits<NW> F;
+                F.zero();
+                if (act && q < q1) F.load(fin, g.csrIdx[q]);
+                done = true;
+#pragma unroll
+                for (int i = 0; i < NW; ++i) {
+                    acc.w[i] |= row_or(F.w[i]);
+                    done &= (acc.w[i] & miss.w[i]) == miss.w[i];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < NW; ++i) {
+                    const unsigned long long x = read_lane(acc.w[i], 16 * r);
+                    if (int(lane) == l[r]) got.w[i] = x;
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < NW; ++i) got.w[i] &= need.w[i];
+        const bool any = got.any();
+        if (any) {
+            unsigned long long* nr = next_at<NW>(a, v);
+#pragma unroll
+            for (int i = 0; i < NW; ++i) {
+                if (deg <= kPullOwn) nr[i] = got.w[i];  // this lane alone writes the record
+                else if (got.w[i]) atomicOr(nr + i, got.w[i]);
+            }
+        }
+        if (__ballot(any) && lane == 0) a.dirty[w] = 1;
+    }
+    for (uint32_t h = wave; h < g.pullCount; h += nwaves) {
+        const uint2 hu = g.pullUnits[h];
+        const uint32_t v = __builtin_amdgcn_readfirstlane(hu.x), p0 = __builtin_amdgcn_readfirstlane(hu.y);
+        if (test_bit(a.full, v)) continue;
+        const uint32_t p1 = min(g.csrPtr[v + 1], p0 + kPullUnit);
+        const unsigned long long* rec = vis_at<NW>(a, v);
+        Bits<NW> need, got;
+        got.zero();
+        bool open = false;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            need.w[i] = rootMask.w[i] & ~(rec[i] | rec[NW + i]);
+            open |= need.w[i] != 0;
+        }
+        if (!__ballot(open)) continue;
+        const uint32_t p = p0 + lane * 4;
+        if (p < p1) {
+            const u32x4_a4 u = *reinterpret_cast<const u32x4_a4*>(g.csrIdx + p);
+            Bits<NW> F[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                F[j].zero();
+                if (p + j < p1) F[j].load(fin, u[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < NW; ++i) got.w[i] |= F[j].w[i];
+        }
+        bool any = false;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            unsigned long long x = row_or(got.w[i]);
+            x = read_lane(x, 0) | read_lane(x, 16) | read_lane(x, 32) | read_lane(x, 48);
+            x &= need.w[i];
+            if (x && lane == 0) atomicOr(next_at<NW>(a, v) + i, x);
+            any |= x != 0;
+        }
+        if (any && lane == 0) a.dirty[v >> 6] = 1;
+    }
+}
+
+// Bottom-up level of a symmetric graph without a resident CSR: a pull over the BVSS slices.  For a
 // symmetric graph a slice (row i, mask m) of rset r is also the set of edges
 // i -> 8r + b (b in m), so vertex 8r + b gains OR_{slices with bit b} F[i], F = the
 // previous level's frontier words.  A vset is taken by 16 lanes (two quads each per
@@ -408,227 +559,111 @@ __global__ void __launch_bounds__(kProducerBlock) __attribute__((amdgpu_waves_pe
 mbfs_expand_kernel(GraphView g, MbfsArgs a, unsigned Lk) {
     const unsigned L = level_of(a.ctrl, a.levelFromCtrl, Lk);
     __shared__ unsigned pre[kMaxSegs];
-    __shared__ unsigned long long tmp64[16];
     Ctrl* c = a.ctrl;
     const uint32_t segs = a.sv.segs;
     DirectionParams dp;
     dp.direction = a.direction;
-    dp.canBottomUp = g.csrPtr != nullptr || a.pull;
+    dp.canBottomUp = g.csrPtr != nullptr || a.slicePull;
     dp.alpha = a.alpha;
     dp.beta = a.beta;
     dp.totalEdges = (unsigned long long)a.k * g.nnz;
     dp.totalItems = double(g.n) * a.k;
-    dp.weighEdges = false;
+    dp.weighEdges = true;
     bool bottomUp = false;
     unsigned total = 0;  // list entries of the level (top-down)
     if (!level_begin(c, a.sc, segs, L, dp, bottomUp, pre, &total)) return;
     const unsigned lane = lane_id();
     const unsigned long long* fin = mfront<NW>(a, g.n, L - 1);
-    unsigned long long* fout = mfront<NW>(a, g.n, L);
-    const bool writeLevels = L > a.histLevels;
-    const unsigned sOut = (L + 1) % 3;
     if (!bottomUp && ALGO == 1) {
         mbfs_td_mfma<NW>(g, a, (L & 1) ? a.list1 : a.list0, pre, total, fin);
         return;
     }
-    if (bottomUp && a.pull) {
-        mbfs_pull<NW>(g, a, fin, a.any + size_t((L - 1) & 1) * g.W);
+    if (bottomUp) {
+        if (a.slicePull)
+            mbfs_pull<NW>(g, a, fin, a.any + size_t((L - 1) & 1) * g.W);
+        else
+            mbfs_pull_csr<NW>(g, a, fin);
         return;
     }
-    if (!bottomUp) {
-        const uint32_t* lin = (L & 1) ? a.list1 : a.list0;
+    const uint32_t* lin = (L & 1) ? a.list1 : a.list0;
 
-        const unsigned wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-        const unsigned nwaves = (gridDim.x * blockDim.x) / kWave;
-        // m list entries per wave step (a short list is spread over as many waves)
-        const unsigned m = min(unsigned(kWave), max(1u, (total + nwaves - 1) / nwaves));
-        for (unsigned base = wave * m; base < total; base += nwaves * m) {
-            const unsigned e = base + lane;
-            uint32_t q0 = 0, qc = 0, r = 0;
-            if (lane < m && e < total) {
-                const uint32_t vs = list_entry(lin, a.sv, pre, e);
-                q0 = g.unitQuad[vs];
-                qc = g.unitQuad[vs + 1] - q0;
-                r = g.unitRset[vs];
-            }
-            const unsigned incl = wave_inclusive_scan(qc);
-            const unsigned excl = incl - qc;
-            const unsigned tq = __shfl(incl, kWave - 1, kWave);
-            for (unsigned t0 = 0; t0 < tq; t0 += kWave) {
-                const unsigned t = t0 + lane;
-                const unsigned owner = wave_owner(excl, min(t, tq - 1));
-                const uint32_t oq0 = __shfl(q0, owner, kWave);
-                const unsigned oex = __shfl(excl, owner, kWave);
-                const uint32_t orr = __shfl(r, owner, kWave);
-                if (t < tq) {
-                    const uint32_t q = oq0 + (t - oex);
-                    const uint4 r4 = stream_load_quad(g.rows, q);
-                    const uint32_t m = stream_load_u32(g.masks, q);
-                    const uint32_t um = (m | (m >> 8) | (m >> 16) | (m >> 24)) & 0xFF;
-                    Bits<NW> F[8];
+    const unsigned wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+    const unsigned nwaves = (gridDim.x * blockDim.x) / kWave;
+    // m list entries per wave step (a short list is spread over as many waves)
+    const unsigned m = min(unsigned(kWave), max(1u, (total + nwaves - 1) / nwaves));
+    for (unsigned base = wave * m; base < total; base += nwaves * m) {
+        const unsigned e = base + lane;
+        uint32_t q0 = 0, qc = 0, r = 0;
+        if (lane < m && e < total) {
+            const uint32_t vs = list_entry(lin, a.sv, pre, e);
+            q0 = g.unitQuad[vs];
+            qc = g.unitQuad[vs + 1] - q0;
+            r = g.unitRset[vs];
+        }
+        const unsigned incl = wave_inclusive_scan(qc);
+        const unsigned excl = incl - qc;
+        const unsigned tq = __shfl(incl, kWave - 1, kWave);
+        for (unsigned t0 = 0; t0 < tq; t0 += kWave) {
+            const unsigned t = t0 + lane;
+            const unsigned owner = wave_owner(excl, min(t, tq - 1));
+            const uint32_t oq0 = __shfl(q0, owner, kWave);
+            const unsigned oex = __shfl(excl, owner, kWave);
+            const uint32_t orr = __shfl(r, owner, kWave);
+            if (t < tq) {
+                const uint32_t q = oq0 + (t - oex);
+                const uint4 r4 = stream_load_quad(g.rows, q);
+                const uint32_t m = stream_load_u32(g.masks, q);
+                const uint32_t um = (m | (m >> 8) | (m >> 16) | (m >> 24)) & 0xFF;
+                Bits<NW> F[8];
 #pragma unroll
-                    for (int b = 0; b < 8; ++b) {
-                        F[b].zero();
-                        if ((um >> b) & 1) F[b].load(fin, orr * 8 + b);
+                for (int b = 0; b < 8; ++b) {
+                    F[b].zero();
+                    if ((um >> b) & 1) F[b].load(fin, orr * 8 + b);
+                }
+                const uint32_t rowv[4] = {r4.x, r4.y, r4.z, r4.w};
+                // Phased so that the four slices' loads overlap: the roots arriving
+                // per slice (registers), then the saturated-row bits (L2), then the
+                // row records, and only then the atomics (an atomic on a record may
+                // alias a later slice's load, so mixing them serialises the slices).
+                Bits<NW> acc[4];
+                bool act[4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const uint32_t ms = (m >> (8 * s)) & 0xFF;
+                    acc[s].zero();
+#pragma unroll
+                    for (int b = 0; b < 8; ++b)
+                        if ((ms >> b) & 1)
+#pragma unroll
+                            for (int i = 0; i < NW; ++i) acc[s].w[i] |= F[b].w[i];
+                    act[s] = acc[s].any();
+                }
+                unsigned long long fullw[4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) fullw[s] = act[s] ? a.full[(act[s] ? rowv[s] : 0u) >> 6] : 0ull;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) act[s] = act[s] && !((fullw[s] >> (rowv[s] & 63)) & 1ull);
+                unsigned long long seen[4][NW];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const unsigned long long* rec = vis_at<NW>(a, act[s] ? rowv[s] : 0u);
+#pragma unroll
+                    for (int i = 0; i < NW; ++i) seen[s][i] = act[s] ? (rec[i] | rec[NW + i]) : ~0ull;
+                }
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    unsigned long long* nr = next_at<NW>(a, act[s] ? rowv[s] : 0u);
+                    bool any = false;
+#pragma unroll
+                    for (int i = 0; i < NW; ++i) {
+                        const unsigned long long nv = acc[s].w[i] & ~seen[s][i];
+                        if (act[s] && nv) atomicOr(nr + i, nv);
+                        any |= act[s] && nv != 0;
                     }
-                    const uint32_t rowv[4] = {r4.x, r4.y, r4.z, r4.w};
-                    // Phased so that the four slices' loads overlap: the roots arriving
-                    // per slice (registers), then the saturated-row bits (L2), then the
-                    // row records, and only then the atomics (an atomic on a record may
-                    // alias a later slice's load, so mixing them serialises the slices).
-                    Bits<NW> acc[4];
-                    bool act[4];
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const uint32_t ms = (m >> (8 * s)) & 0xFF;
-                        acc[s].zero();
-#pragma unroll
-                        for (int b = 0; b < 8; ++b)
-                            if ((ms >> b) & 1)
-#pragma unroll
-                                for (int i = 0; i < NW; ++i) acc[s].w[i] |= F[b].w[i];
-                        act[s] = acc[s].any();
-                    }
-                    unsigned long long fullw[4];
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) fullw[s] = act[s] ? a.full[(act[s] ? rowv[s] : 0u) >> 6] : 0ull;
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) act[s] = act[s] && !((fullw[s] >> (rowv[s] & 63)) & 1ull);
-                    unsigned long long seen[4][NW];
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const unsigned long long* rec = vis_at<NW>(a, act[s] ? rowv[s] : 0u);
-#pragma unroll
-                        for (int i = 0; i < NW; ++i) seen[s][i] = act[s] ? (rec[i] | rec[NW + i]) : ~0ull;
-                    }
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        unsigned long long* nr = next_at<NW>(a, act[s] ? rowv[s] : 0u);
-                        bool any = false;
-#pragma unroll
-                        for (int i = 0; i < NW; ++i) {
-                            const unsigned long long nv = acc[s].w[i] & ~seen[s][i];
-                            if (act[s] && nv) atomicOr(nr + i, nv);
-                            any |= act[s] && nv != 0;
-                        }
-                        if (any) a.dirty[rowv[s] >> 6] = 1;  // a byte store: idempotent
-                    }
+                    if (any) a.dirty[rowv[s] >> 6] = 1;  // a byte store: idempotent
                 }
             }
         }
-        return;
-    }
-    // bottom-up over this workgroup's segment: wave per word, lane per vertex.  A vertex
-    // of degree > kHeavyDeg is deferred to a second pass in which a whole wave scans its
-    // neighbours 64 at a time: with many roots a scan rarely stops early, and one lane
-    // walking a hub's list would hold its wave (and the level) for the whole list.
-    constexpr uint32_t kHeavyDeg = 64;
-    constexpr unsigned kHeavyCap = 2048;
-    __shared__ uint32_t heavyQ[kHeavyCap];
-    __shared__ unsigned heavyN;
-    if (threadIdx.x == 0) heavyN = 0;
-    __syncthreads();
-    const Bits<NW> rootMask = root_mask<NW>(a.k);
-    const uint32_t ws = blockIdx.x * a.sv.wps, we = min(g.W, ws + a.sv.wps);
-    const unsigned wib = threadIdx.x / kWave, wpb = blockDim.x / kWave;
-    unsigned long long news = 0, edges = 0;
-    for (uint32_t w = ws + wib; w < we; w += wpb) {
-        const uint32_t v = w * 64 + lane;
-        if (v >= g.n) continue;
-        Bits<NW> vis, U, nw;
-        vis.loadp(vis_at<NW>(a, v));
-        nw.zero();
-        bool need = false;
-#pragma unroll
-        for (int i = 0; i < NW; ++i) {
-            U.w[i] = ~vis.w[i] & rootMask.w[i];
-            need |= U.w[i] != 0;
-        }
-        const uint32_t p0 = need ? g.csrPtr[v] : 0u, p1 = need ? g.csrPtr[v + 1] : 0u;
-        if (need && p1 - p0 > kHeavyDeg) {
-            const unsigned slot = atomicAdd(&heavyN, 1u);
-            if (slot < kHeavyCap) {
-                heavyQ[slot] = v;
-                need = false;  // its frontier word is written by the heavy pass
-            }
-        }
-        if (need) {
-            Bits<NW> acc;
-            acc.zero();
-            for (uint32_t p = p0; p < p1; ++p) {
-                const uint32_t u = g.csrIdx[p];
-                bool all = true;
-#pragma unroll
-                for (int i = 0; i < NW; ++i) {
-                    acc.w[i] |= fin[size_t(u) * NW + i];
-                    all &= (acc.w[i] & U.w[i]) == U.w[i];
-                }
-                if (all) break;
-            }
-#pragma unroll
-            for (int i = 0; i < NW; ++i) nw.w[i] = acc.w[i] & U.w[i];
-            if (nw.any()) {
-#pragma unroll
-                for (int i = 0; i < NW; ++i) vis.w[i] |= nw.w[i];
-                vis.storep(vis_at<NW>(a, v));
-                if (writeLevels)
-                    for (int i = 0; i < NW; ++i)
-                        for (unsigned long long b = nw.w[i]; b; b &= b - 1)
-                            a.levels[size_t(64 * i + __builtin_ctzll(b)) * g.n + v] = int32_t(L);
-                news += nw.popc();
-                edges += (unsigned long long)(p1 - p0) * nw.popc();
-            }
-        }
-        nw.store(fout, v);
-    }
-    __syncthreads();
-    const unsigned nh = min(heavyN, kHeavyCap);
-    for (unsigned h = wib; h < nh; h += wpb) {
-        const uint32_t v = heavyQ[h];
-        Bits<NW> vis, U, acc;
-        vis.loadp(vis_at<NW>(a, v));
-#pragma unroll
-        for (int i = 0; i < NW; ++i) U.w[i] = ~vis.w[i] & rootMask.w[i];
-        acc.zero();
-        const uint32_t p0 = g.csrPtr[v], p1 = g.csrPtr[v + 1];
-        for (uint32_t pb = p0; pb < p1; pb += kWave) {
-            const uint32_t p = pb + lane;
-            if (p < p1) {
-                const uint32_t u = g.csrIdx[p];
-#pragma unroll
-                for (int i = 0; i < NW; ++i) acc.w[i] |= fin[size_t(u) * NW + i];
-            }
-            bool all = true;
-#pragma unroll
-            for (int i = 0; i < NW; ++i) {
-                for (int d = kWave / 2; d > 0; d >>= 1) acc.w[i] |= __shfl_xor(acc.w[i], d, kWave);
-                all &= (acc.w[i] & U.w[i]) == U.w[i];
-            }
-            if (all) break;  // acc is the same on every lane: uniform exit
-        }
-        if (lane == 0) {
-            Bits<NW> nw;
-#pragma unroll
-            for (int i = 0; i < NW; ++i) nw.w[i] = acc.w[i] & U.w[i];
-            if (nw.any()) {
-#pragma unroll
-                for (int i = 0; i < NW; ++i) vis.w[i] |= nw.w[i];
-                vis.storep(vis_at<NW>(a, v));
-                if (writeLevels)
-                    for (int i = 0; i < NW; ++i)
-                        for (unsigned long long b = nw.w[i]; b; b &= b - 1)
-                            a.levels[size_t(64 * i + __builtin_ctzll(b)) * g.n + v] = int32_t(L);
-                news += nw.popc();
-                edges += (unsigned long long)(p1 - p0) * nw.popc();
-            }
-            nw.store(fout, v);
-        }
-    }
-    news = block_sum_u64(news, tmp64);
-    edges = block_sum_u64(edges, tmp64);
-    if (threadIdx.x == 0) {
-        a.sc.news[size_t(sOut) * segs + blockIdx.x] = unsigned(min(news, 0xFFFFFFFFull));
-        a.sc.edges[size_t(sOut) * segs + blockIdx.x] = edges;
     }
 }
 
@@ -646,11 +681,6 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID mbfs_updat
     const uint32_t segs = a.sv.segs;
     const unsigned sOut = (L + 1) % 3;
     if (blockIdx.x == 0 && threadIdx.x == 0) c->histTop = L;  // read only after this kernel
-    if (bottomUp && !a.pull) {
-        const unsigned cnt = segment_list<NW>(g, a.sv, fout, lout, l);
-        if (threadIdx.x == 0) a.sc.count[size_t(sOut) * segs + blockIdx.x] = cnt;
-        return;
-    }
     const uint32_t ws = blockIdx.x * a.sv.wps, we = min(g.W, ws + a.sv.wps);
     uint32_t first, last;
     wave_words(ws, we, threadIdx.x / kWave, blockDim.x / kWave, first, last);
@@ -934,7 +964,7 @@ static void mbfs_run(Query& q, const uint32_t* srcs, uint32_t k, int32_t* hostLe
     a.full = q.mFull;
     a.any = q.mAny;
     a.dirty = q.mDirty;
-    a.pull = g.symmetric ? 1 : 0;
+    a.slicePull = (g.symmetric && !g.hasCsr) ? 1 : 0;
     a.list0 = q.list0;
     a.list1 = q.list1;
     a.srcs = q.srcs;
@@ -942,12 +972,9 @@ static void mbfs_run(Query& q, const uint32_t* srcs, uint32_t k, int32_t* hostLe
     a.ctrl = q.ctrl;
     a.sv = g.wide_view();
     a.sc = q.seg_counters();
-    // Direction.  A symmetric graph pulls over the BVSS slices on bottom-up levels
-    // (mbfs_pull), and switches by the graph's thresholds (direction 0) unless one
-    // direction is asked for.  Otherwise top-down unless bottom-up (the CSR scan) is
-    // asked for explicitly (direction 2): with 64-128 roots a per-vertex scan must find
-    // every root still missing at a vertex, so it seldom stops early; on R-MAT scale 22
-    // (128 roots) that switching schedule took 21 ms per batch and top-down only 9.6 ms.
+    // Direction.  A symmetric graph switches by the graph's thresholds (direction 0) unless
+    // one direction is asked for; another one stays top-down unless bottom-up is asked for
+    // explicitly (direction 2).
     if (g.symmetric)
         a.direction = g.opts.direction;
     else
