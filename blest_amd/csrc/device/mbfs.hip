@@ -765,53 +765,102 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID mbfs_updat
     if (threadIdx.x == 0) a.sc.count[size_t(sOut) * segs + blockIdx.x] = running;
 }
 
-// Every (root, vertex) level at once, thread per vertex.  The level of root j is the
-// history level L whose frontier word holds bit j; with L <= 16 its five bits are read
-// from five bit-planes (plane b = OR of the words of the levels with bit b set), so a
-// vertex costs its history words in and its k levels out, nothing else.  Pairs found
-// past the history were written when found; the rest are unreached (-1).  Root-major
-// rows: for each root the threads store consecutive levels, into the query's level array
+// Every (root, vertex) level at once.  The level of root j is the history level L whose
+// frontier word holds bit j; with L <= 16 its five bits are read from five bit-planes
+// (plane b = OR of the words of the levels with bit b set), so a vertex costs its history
+// words in and its k levels out, nothing else.  Pairs found past the history were written
+// when found; the rest are unreached (-1).  Root-major rows, into the query's level array
 // and, in natural order, the caller's device array (dst, nullable) at once.  Enqueued
 // ahead of each completion poll; until the traversal is done it only publishes the control
 // block.
-constexpr unsigned kFinalBlock = 256;
+// Bound by the stores.  A workgroup turns the history of 512 vertices into planes in LDS
+// (thread per vertex, each history word read once), then a thread takes four consecutive
+// vertices and a run of roots, so that a wave stores 1 KiB of a row at a time: 2 x 2.1 GB
+// for 128 roots on R-MAT 22 in 1.02 ms, the rate of a large copy.  With 4-byte stores
+// of one vertex a thread 1.31 ms; with four vertices a thread and the history read by the
+// 32 roots, four times in all, 1.55; non-temporal stores 1.15.
+constexpr unsigned kFinalBlock = 512;  // threads, and vertices of a tile
+typedef int32_t i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // rows start at any multiple of 4 bytes
 
 template <int NW>
 __global__ void __launch_bounds__(kFinalBlock) mbfs_final_kernel(GraphView g, MbfsArgs a, int32_t* dst, Ctrl* host) {
     if (blockIdx.x == 0) publish_ctrl(a.ctrl, host);
     if (!ld_relaxed(&a.ctrl->done)) return;
+    __shared__ __align__(16) uint32_t sPlane[6][2 * NW][kFinalBlock];  // five level bits, then "in the history"
     const unsigned top = min(__hip_atomic_load(&a.ctrl->histTop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
                              a.histLevels);
-    for (uint32_t v = blockIdx.x * kFinalBlock + threadIdx.x; v < g.n; v += gridDim.x * kFinalBlock) {
+    constexpr unsigned kRows = 16 * NW;  // roots of a thread: runs of 4 vertices x 4 runs of roots
+    const unsigned t = threadIdx.x, quad = t % (kFinalBlock / 4), r0 = t / (kFinalBlock / 4) * kRows;
+    const unsigned r1 = min(r0 + kRows, a.k), grp = r0 / 32;
+    for (size_t v0 = size_t(blockIdx.x) * kFinalBlock; v0 < g.n; v0 += size_t(gridDim.x) * kFinalBlock) {
+        const size_t v = v0 + t;
+        const bool ok = v < g.n;
+        Bits<NW> plane[5], in, late;
+        in.zero();
+        late.zero();
 #pragma unroll
-        for (int i = 0; i < NW; ++i) {
-            if (64 * i >= int(a.k)) break;
-            unsigned long long plane[5] = {0, 0, 0, 0, 0}, inHist = 0;
+        for (int b = 0; b < 5; ++b) plane[b].zero();
+        if (ok) {
+            late.loadp(vis_at<NW>(a, uint32_t(v)));
             for (unsigned L = 0; L <= top; ++L) {
-                const unsigned long long x = a.hist[(size_t(L) * g.n + v) * NW + i];
-                inHist |= x;
+                Bits<NW> x;
+                x.load(a.hist + size_t(L) * g.n * NW, uint32_t(v));
 #pragma unroll
-                for (int b = 0; b < 5; ++b)
-                    if ((L >> b) & 1u) plane[b] |= x;
-            }
-            const unsigned long long vis = vis_at<NW>(a, v)[i];
-            const unsigned jn = min(64u, a.k - 64u * i);
-            for (unsigned j = 0; j < jn; ++j) {
-                const size_t at = size_t(64 * i + j) * g.n + v;
-                // streaming stores: the k x n output is written once and not read here
-                int32_t l = -1;
-                if ((inHist >> j) & 1ull) {
-                    l = 0;
+                for (int i = 0; i < NW; ++i) {
+                    in.w[i] |= x.w[i];
 #pragma unroll
-                    for (int b = 0; b < 5; ++b) l |= int32_t((plane[b] >> j) & 1ull) << b;
-                } else if ((vis >> j) & 1ull) {
-                    if (dst) dst[at] = a.levels[at];  // past the history: stored when found
-                    continue;
+                    for (int b = 0; b < 5; ++b) plane[b].w[i] |= ((L >> b) & 1u) ? x.w[i] : 0ull;
                 }
-                __builtin_nontemporal_store(l, a.levels + at);
-                if (dst) __builtin_nontemporal_store(l, dst + at);
             }
         }
+        bool deep = false;  // a pair found past the history, stored when found
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            deep |= (late.w[i] & ~in.w[i]) != 0;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int b = 0; b < 5; ++b) sPlane[b][2 * i + h][t] = uint32_t(plane[b].w[i] >> (32 * h));
+                sPlane[5][2 * i + h][t] = uint32_t(in.w[i] >> (32 * h));
+            }
+        }
+        const bool careful = __syncthreads_or(deep) || v0 + kFinalBlock > g.n;
+        uint32_t p[6][4];
+#pragma unroll
+        for (int b = 0; b < 6; ++b) {
+            const uint4 x = *reinterpret_cast<const uint4*>(&sPlane[b][grp][4 * quad]);
+            p[b][0] = x.x;
+            p[b][1] = x.y;
+            p[b][2] = x.z;
+            p[b][3] = x.w;
+        }
+        for (unsigned r = r0; r < r1; ++r) {
+            const unsigned j = r & 31u;
+            const size_t at = size_t(r) * g.n + v0 + 4 * quad;
+            i32x4_a4 l;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                uint32_t x = 0;
+#pragma unroll
+                for (int b = 0; b < 5; ++b) x |= ((p[b][q] >> j) & 1u) << b;
+                l[q] = int32_t(x) | (int32_t((p[5][q] >> j) & 1u) - 1);  // -1 where no history level has it
+            }
+            if (!careful) {
+                *reinterpret_cast<i32x4_a4*>(a.levels + at) = l;
+                if (dst) *reinterpret_cast<i32x4_a4*>(dst + at) = l;
+                continue;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const size_t u = v0 + 4 * quad + q;
+                if (u >= g.n) continue;
+                int32_t x = l[q];
+                if (x < 0 && ((vis_at<NW>(a, uint32_t(u))[r / 64] >> (r & 63u)) & 1ull)) x = a.levels[at + q];
+                else a.levels[at + q] = x;
+                if (dst) dst[at + q] = x;
+            }
+        }
+        __syncthreads();  // the next tile reuses the planes
     }
 }
 
@@ -920,7 +969,7 @@ static void mbfs_enqueue_levels(Query& q, const dev::MbfsArgs& a, int32_t* dst) 
             hipLaunchKernelGGL(dev::mbfs_update_kernel<NW>, grid, block, 0, q.stream, gv, a, L);
         },
         [&] {
-            const uint32_t fb = std::min<uint32_t>((g.n + dev::kFinalBlock - 1) / dev::kFinalBlock, uint32_t(g.cus) * 8);
+            const uint32_t fb = std::min<uint32_t>((g.n - 1) / dev::kFinalBlock + 1, uint32_t(g.cus) * 64);
             hipLaunchKernelGGL(dev::mbfs_final_kernel<NW>, dim3(fb), dim3(dev::kFinalBlock), 0, q.stream, gv, a, dst,
                                q.hostCtrl);
         },
