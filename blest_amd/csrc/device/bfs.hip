@@ -33,6 +33,7 @@
 #include "dgraph.hpp"
 #include "level_common.hpp"
 #include "small_traverse.hpp"
+#include "thin_levels.hpp"
 
 namespace blest {
 namespace dev {
@@ -159,7 +160,6 @@ constexpr int kFuseQpl = 4;                      // quads per thread per pass
 // so levels of up to kFuseShrinkScale x fuseQuads quads still run here.
 constexpr unsigned kFuseShrinkScale = 4;
 constexpr uint32_t kNoRset = 0xFFFFFFFFu;
-typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
 
 // A queue of rsets: entries below kFuseTile in LDS (the level prefix arrays, free once the
 // first level's lists are read), later ones in global memory at the same index (the
@@ -936,7 +936,6 @@ __global__ void __launch_bounds__(kProducerBlock) bfs_final_kernel(GraphView g, 
 
 // The whole traversal of a small symmetric graph in one workgroup (small_traverse.hpp):
 // no level kernel, no poll per chunk of levels.
-constexpr uint32_t kSmallVertices = 131072;    // three bitmaps of 16 KiB in LDS
 constexpr uint64_t kSmallEdges = 1u << 18;     // see small_graph()
 
 __global__ void __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(4)))
@@ -975,13 +974,56 @@ static ExpandKernel expand_kernel_for(const DeviceGraph& g) {
     }
 }
 
-// Graphs that one workgroup traverses faster than level kernels do: its time grows with
-// the edges (about 28 us at 16 K, 117 us at 264 K directed edges), a level pair costs 20 us
-// and more whatever it holds.  Only the default schedule: a fixed direction, levels never
-// fused and always-replayed chunks keep their level kernels.
+// Graphs that one workgroup traverses faster than level kernels do.  Its time grows with
+// the words of the bitmap, which every level passes over, and with the edges; a level pair
+// costs 15 us and more whatever it holds (us per call, one workgroup and level kernels:
+// Erdos-Renyi of mean degree 4, 2 K vertices 44 and 139, 8 K 78 and 142, 20 K 149 and 177;
+// mean degree 3, 50 K 397 and 224; R-MAT 13 of edge factor 16 52 and 104).  Only the
+// default schedule: a fixed direction, levels never fused and always-replayed chunks keep
+// their level kernels.
 static bool small_graph(const DeviceGraph& g) {
     return g.symmetric && g.hasCsr && g.n <= dev::kSmallVertices && g.nnz <= dev::kSmallEdges &&
            g.opts.direction == 0 && g.opts.fuse_quads > 0 && g.opts.use_graphs != 1;
+}
+
+// The traversal over vertex queues (thin_levels.hpp); ev0 is recorded.
+static void thin_launch(Query& q, const dev::BfsArgs& b, const uint32_t* oldToNew, int32_t* dst) {
+    DeviceGraph& g = *q.g;
+    const GraphView gv = g.view();
+    dev::ThinArgs a;
+    a.levels = q.levels;
+    a.visited = reinterpret_cast<uint32_t*>(q.visited);
+    a.queue0 = q.thinQueue0;
+    a.queue1 = q.thinQueue1;
+    a.count = q.thinCount;
+    a.edges = q.thinEdges;
+    a.ctrl = q.ctrl;
+    a.segs = g.thinSegs;
+    a.shift = g.thinShift;
+    a.src = b.src;
+    a.levelFromCtrl = 0;
+    dev::ThinArgs ar = a;
+    ar.levelFromCtrl = 1;
+    const dim3 grid(std::min(uint32_t(g.cus) * 2, dev::kThinMaxSegs)), block(dev::kThinBlock);
+    const auto level = [&](const dev::ThinArgs& x, unsigned L) {
+        hipLaunchKernelGGL(dev::thin_level_kernel, grid, block, 0, q.stream, gv, x, L);
+    };
+    const auto fused = [&](const dev::ThinArgs& x, unsigned L) {
+        hipLaunchKernelGGL(dev::thin_fused_kernel, dim3(1), dim3(dev::kThinFusedBlock), 0, q.stream, gv, x, L);
+    };
+    hipLaunchKernelGGL(dev::thin_init_kernel, wide_grid(g), dim3(dev::kProducerBlock), 0, q.stream, gv, a);
+    fused(a, 1);
+    run_levels(
+        q, [&](unsigned L) { level(a, L); },
+        [&] {
+            hipLaunchKernelGGL(dev::bfs_final_kernel, wide_grid(g), dim3(dev::kProducerBlock), 0, q.stream, gv, b,
+                               oldToNew, dst, q.hostCtrl);
+        },
+        &q.graphs[kGraphThin], [&](unsigned k) { level(ar, k); }, 1, [&](unsigned L) { fused(a, L); },
+        [&](unsigned k) { fused(ar, k); });
+    BLEST_HIP(hipGetLastError());
+    q.lastSource = b.src;
+    q.pending = true;
 }
 
 void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
@@ -1013,7 +1055,7 @@ void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
     const ExpandKernel expand = expand_kernel_for(g);
     const uint32_t* oldToNew = g.hasPerm ? g.permOldToNew : nullptr;
     BLEST_HIP(hipEventRecord(q.ev0, q.stream));
-    if (!trace && small_graph(g)) {
+    if (!trace && !q.thinQueue0 && small_graph(g)) {
         hipLaunchKernelGGL(dev::bfs_small_kernel, dim3(1), dim3(dev::kBatchBlock), 3 * sizeof(unsigned long long) * g.W,
                            q.stream, gv, a, oldToNew, dst, q.hostCtrl);
         BLEST_HIP(hipGetLastError());
@@ -1021,6 +1063,10 @@ void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
         BLEST_HIP(hipStreamSynchronize(q.stream));
         q.lastSource = src;
         q.pending = true;
+        return;
+    }
+    if (!trace && q.thinQueue0 && !q.thinWide && g.opts.direction == 0 && g.opts.fuse_quads > 0) {
+        thin_launch(q, a, oldToNew, dst);
         return;
     }
     const auto close = [&] {
@@ -1092,6 +1138,11 @@ void bfs_finish(Query& q, int32_t* hostLevels, blest_bfs_stats* st) {
     // level kernels the next traversal enqueues before the fused kernel takes over: up to
     // the final run of small shrinking levels, else all this traversal used
     q.levelHint = c.tailFrom ? c.tailFrom - 1 : c.levels - c.fusedLevels;
+    // (kept once seen: the bit-matrix levels that follow say the same of the graph)
+    if (q.thinQueue0 && c.levels < dev::kThinFewLevels && c.visited / std::max(c.levels, 1u) > dev::kThinWideLevel) {
+        q.levelHint = q.thinWide ? q.levelHint : 0;  // the hint counted queue levels
+        q.thinWide = true;
+    }
     float ms = 0;
     BLEST_HIP(hipEventElapsedTime(&ms, q.ev0, q.ev1));
     if (st) {

@@ -88,7 +88,7 @@ struct Carver {
 // Lays the query state of blest_query_create (single source, without the multi-source
 // and CC parts) over `base`; returns the bytes it needs.  With base == nullptr it only
 // measures.
-size_t carve_state(const DeviceGraph& g, unsigned char* base, Query& q, bool levelsInScratch) {
+size_t carve_state(const DeviceGraph& g, unsigned char* base, Query& q, bool levelsInScratch, bool thin) {
     Carver c{base};
     q.ctrl = c.take<dev::Ctrl>(1);
     if (levelsInScratch) q.levels = c.take<int32_t>(g.n);
@@ -104,6 +104,12 @@ size_t carve_state(const DeviceGraph& g, unsigned char* base, Query& q, bool lev
     q.segCount = c.take<uint32_t>(3 * size_t(g.segs));
     q.segNew = c.take<uint32_t>(3 * size_t(g.segs));
     q.segEdges = c.take<unsigned long long>(3 * size_t(g.segs));
+    if (thin) {
+        q.thinQueue0 = c.take<uint32_t>(g.thin_queue_entries());
+        q.thinQueue1 = c.take<uint32_t>(g.thin_queue_entries());
+        q.thinCount = c.take<uint32_t>(3 * size_t(dev::kThinMaxSegs));
+        q.thinEdges = c.take<unsigned long long>(dev::kThinMaxSegs);
+    }
     return c.used;
 }
 
@@ -152,7 +158,9 @@ blest_status blest_bfs_noalloc(const blest_device_graph* dg, uint32_t src, int32
             throw Error(BLEST_ERR_INVALID_ARGUMENT, "levels must hold n int32 entries");
         }
         BorrowedQuery q;
-        const size_t need = carve_state(g, nullptr, q, g.hasPerm);
+        // vertex queues where they fit as well (blest_bfs's path), else the bit-matrix levels
+        const bool thin = g.thin && carve_state(g, nullptr, q, g.hasPerm, true) <= kScratchBytes;
+        const size_t need = carve_state(g, nullptr, q, g.hasPerm, thin);
         if (need > kScratchBytes)
             throw Error(BLEST_ERR_INVALID_ARGUMENT,
                         "graph needs " + std::to_string(need) + " bytes of traversal state, above the " +
@@ -167,7 +175,7 @@ blest_status blest_bfs_noalloc(const blest_device_graph* dg, uint32_t src, int32
         q.hostCtrl = slot.hostCtrl;
         q.noGraphs = true;  // instantiating a captured graph would allocate
         q.levelHint = slot.levelHint;
-        carve_state(g, slot.ptr, q, g.hasPerm);
+        carve_state(g, slot.ptr, q, g.hasPerm, thin);
         if (!g.hasPerm) q.levels = levels;  // reordered IDs are the caller's IDs
         hipLaunchKernelGGL(clear_ctrl_kernel, dim3(1), dim3(64), 0, q.stream, q.ctrl);
         BLEST_HIP(hipGetLastError());

@@ -60,6 +60,7 @@ __device__ __forceinline__ uint32_t stream_load_u32(const uint32_t* p, uint32_t 
     return __builtin_nontemporal_load(p + i);
 }
 
+typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 // ------------------------------------------------------------------ wave helpers

@@ -363,9 +363,12 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                 if (!opts.keep_csr) {
                     g.symmetric = csc_is_symmetric(c);
                 } else {
-                    for (uint32_t v = 0; v < c.n; ++v)
+                    uint32_t maxDegree = 0;
+                    for (uint32_t v = 0; v < c.n; ++v) {
                         if (c.colPtrs[v + 1] < c.colPtrs[v])
                             throw Error(BLEST_ERR_INVALID_ARGUMENT, "col_ptrs not monotone");
+                        maxDegree = std::max(maxDegree, c.colPtrs[v + 1] - c.colPtrs[v]);
+                    }
                     if (c.colPtrs[0] != 0 || c.colPtrs[c.n] != c.nnz())
                         throw Error(BLEST_ERR_INVALID_ARGUMENT, "col_ptrs and rows disagree");
                     // Bottom-up reads in-neighbours: the CSR of the edges j -> i, i.e. the
@@ -396,6 +399,13 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                         g.probe = g.alloc<uint32_t>(c.n);
                     }
                     g.hasCsr = true;
+                    g.thin = g.symmetric && c.nnz() <= uint64_t(dev::kThinMeanDegree) * c.n &&
+                             (maxDegree <= dev::kThinMaxDegree
+                                  ? c.n <= dev::kThinMaxVertices
+                                  : maxDegree <= dev::kThinMidDegree && c.n > dev::kThinMidFrom &&
+                                        c.nnz() <= dev::kThinMidEdges);
+                    while ((g.W - 1) >> g.thinShift >= dev::kThinMaxSegs) ++g.thinShift;
+                    g.thinSegs = ((g.W - 1) >> g.thinShift) + 1;
                     // vertices without in-neighbours: a bottom-up sweep skips them
                     g.noIn = g.alloc<unsigned long long>(g.W);
                     csr_marks(g.csrPtr, g.csrIdx, c.n, g.W, g.probe, g.noIn);
@@ -523,6 +533,12 @@ blest_status blest_query_create(blest_device_graph* dg, uint32_t max_sources, bl
             q.segCount = q.alloc<uint32_t>(3 * size_t(g.wideSegs));
             q.segNew = q.alloc<uint32_t>(3 * size_t(g.wideSegs));
             q.segEdges = q.alloc<unsigned long long>(3 * size_t(g.wideSegs));
+            if (g.thin) {
+                q.thinQueue0 = q.alloc<uint32_t>(g.thin_queue_entries());
+                q.thinQueue1 = q.alloc<uint32_t>(g.thin_queue_entries());
+                q.thinCount = q.alloc<uint32_t>(3 * size_t(dev::kThinMaxSegs));
+                q.thinEdges = q.alloc<unsigned long long>(dev::kThinMaxSegs);
+            }
             if (g.hasPerm) q.levelsOut = q.alloc<int32_t>(size_t(g.n) * max_sources);
         } catch (...) {
             delete h;
@@ -570,6 +586,7 @@ blest_status blest_query_footprint(const blest_device_graph* dg, uint32_t max_so
         const uint64_t levels = 4ull * g.n * max_sources;
         b += levels * (g.hasPerm ? 2 : 1);
         b += 4ull * 8ull * g.W + 64ull * g.W + 2ull * 4ull * g.V + 2ull * 8ull * g.chunks + 3ull * 20ull * g.wideSegs;
+        if (g.thin) b += 8ull * g.thin_queue_entries() + 20ull * dev::kThinMaxSegs;
         if (max_sources > 1) {
             const uint32_t nw = max_sources > 64 ? 2 : 1;
             b += (4ull + mbfs_history_levels(g.n, nw) + 1) * 8ull * g.n * nw + 4ull * 128 + 16ull * 128;

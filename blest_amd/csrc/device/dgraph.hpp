@@ -81,6 +81,9 @@ struct DeviceGraph {
     uint32_t* probe = nullptr;           // first bottom-up probe per vertex
     uint2* pullUnits = nullptr;
     uint32_t pullCount = 0;
+    bool thin = false;                   // every list short: single-source levels over vertex queues
+    uint32_t thinSegs = 1, thinShift = 0;
+    size_t thin_queue_entries() const { return size_t(thinSegs) << (6 + thinShift); }
     uint32_t *permNewToOld = nullptr, *permOldToNew = nullptr;  // device copies
     std::vector<uint32_t> hostOldToNew, hostNewToOld;
     std::vector<uint32_t> hostDegree;  // per (reordered) vertex, for GTEPS accounting
@@ -126,7 +129,7 @@ struct LevelGraph {
     unsigned chunk = 0;
     uint64_t key = 0;
 };
-enum LevelGraphKind { kGraphBfs = 0, kGraphMbfs1 = 1, kGraphMbfs2 = 2, kGraphCount = 3 };
+enum LevelGraphKind { kGraphBfs = 0, kGraphMbfs1 = 1, kGraphMbfs2 = 2, kGraphThin = 3, kGraphCount = 4 };
 constexpr unsigned kGraphChunkLevels = 16;  // levels per replayed graph
 constexpr unsigned kGraphMinLevels = 64;    // auto mode: replay once a traversal was this deep
 
@@ -151,6 +154,10 @@ struct Query {
     uint32_t* segChunks = nullptr;                     // [3][segments]
     unsigned long long* segEdges = nullptr;            // [3][segments]
     dev::SegCounters seg_counters() const;
+    // vertex queues of a thin graph's levels (thin_levels.hpp); null otherwise
+    uint32_t *thinQueue0 = nullptr, *thinQueue1 = nullptr, *thinCount = nullptr;
+    unsigned long long* thinEdges = nullptr;
+    bool thinWide = false;  // the last such traversal had few, wide levels: the bit-matrix levels are faster
     int32_t* levelsOut = nullptr;  // original-order copy (when the graph carries a permutation)
     uint32_t* labels = nullptr;    // CC
     uint32_t* labelsAux = nullptr;
