@@ -73,46 +73,6 @@ DeviceSlot& slot_for(int device) {
     return s;
 }
 
-// Carve the traversal state out of the scratch array (256-byte aligned pieces).
-struct Carver {
-    unsigned char* base;
-    size_t used = 0;
-    template <class T>
-    T* take(size_t count) {
-        T* p = reinterpret_cast<T*>(base ? base + used : nullptr);
-        used += (std::max<size_t>(count, 1) * sizeof(T) + 255) & ~size_t(255);
-        return p;
-    }
-};
-
-// Lays the query state of blest_query_create (single source, without the multi-source
-// and CC parts) over `base`; returns the bytes it needs.  With base == nullptr it only
-// measures.
-size_t carve_state(const DeviceGraph& g, unsigned char* base, Query& q, bool levelsInScratch, bool thin) {
-    Carver c{base};
-    q.ctrl = c.take<dev::Ctrl>(1);
-    if (levelsInScratch) q.levels = c.take<int32_t>(g.n);
-    q.visited = c.take<unsigned long long>(g.W);
-    q.front0 = c.take<unsigned long long>(g.W);
-    q.front1 = c.take<unsigned long long>(g.W);
-    q.nextB = c.take<uint8_t>(size_t(g.W) * 64);
-    q.list0 = c.take<uint32_t>(g.V);
-    q.list1 = c.take<uint32_t>(g.V);
-    q.chunk0 = c.take<uint2>(g.chunks);
-    q.chunk1 = c.take<uint2>(g.chunks);
-    q.segChunks = c.take<uint32_t>(3 * size_t(g.segs));
-    q.segCount = c.take<uint32_t>(3 * size_t(g.segs));
-    q.segNew = c.take<uint32_t>(3 * size_t(g.segs));
-    q.segEdges = c.take<unsigned long long>(3 * size_t(g.segs));
-    if (thin) {
-        q.thinQueue0 = c.take<uint32_t>(g.thin_queue_entries());
-        q.thinQueue1 = c.take<uint32_t>(g.thin_queue_entries());
-        q.thinCount = c.take<uint32_t>(3 * size_t(dev::kThinMaxSegs));
-        q.thinEdges = c.take<unsigned long long>(dev::kThinMaxSegs);
-    }
-    return c.used;
-}
-
 // A Query whose buffers, stream and events are borrowed: its destructor must release
 // none of them.
 struct BorrowedQuery : Query {
@@ -159,8 +119,8 @@ blest_status blest_bfs_noalloc(const blest_device_graph* dg, uint32_t src, int32
         }
         BorrowedQuery q;
         // vertex queues where they fit as well (blest_bfs's path), else the bit-matrix levels
-        const bool thin = g.thin && carve_state(g, nullptr, q, g.hasPerm, true) <= kScratchBytes;
-        const size_t need = carve_state(g, nullptr, q, g.hasPerm, thin);
+        const bool thin = g.thin && carve_state(g, nullptr, q, g.hasPerm, true, false) <= kScratchBytes;
+        const size_t need = carve_state(g, nullptr, q, g.hasPerm, thin, false);
         if (need > kScratchBytes)
             throw Error(BLEST_ERR_INVALID_ARGUMENT,
                         "graph needs " + std::to_string(need) + " bytes of traversal state, above the " +
@@ -175,7 +135,7 @@ blest_status blest_bfs_noalloc(const blest_device_graph* dg, uint32_t src, int32
         q.hostCtrl = slot.hostCtrl;
         q.noGraphs = true;  // instantiating a captured graph would allocate
         q.levelHint = slot.levelHint;
-        carve_state(g, slot.ptr, q, g.hasPerm, thin);
+        carve_state(g, slot.ptr, q, g.hasPerm, thin, false);
         if (!g.hasPerm) q.levels = levels;  // reordered IDs are the caller's IDs
         hipLaunchKernelGGL(clear_ctrl_kernel, dim3(1), dim3(64), 0, q.stream, q.ctrl);
         BLEST_HIP(hipGetLastError());

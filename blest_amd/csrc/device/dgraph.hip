@@ -164,6 +164,36 @@ bool check_result_range(const void* dst, size_t bytes, int device, const char* w
     return true;
 }
 
+size_t carve_state(const DeviceGraph& g, unsigned char* base, Query& q, bool withLevels, bool thin, bool withNext) {
+    size_t used = 0;
+    const auto take = [&]<class T>(T*& p, size_t count) {
+        p = base ? reinterpret_cast<T*>(base + used) : nullptr;
+        used += (std::max<size_t>(count, 1) * sizeof(T) + 255) & ~size_t(255);
+    };
+    take(q.ctrl, 1);
+    if (withLevels) take(q.levels, g.n);
+    take(q.visited, g.W);
+    take(q.front0, g.W);
+    take(q.front1, g.W);
+    take(q.nextB, size_t(g.W) * 64);
+    take(q.list0, g.V);
+    take(q.list1, g.V);
+    take(q.chunk0, g.chunks);
+    take(q.chunk1, g.chunks);
+    take(q.segChunks, 3 * size_t(g.wideSegs));
+    take(q.segCount, 3 * size_t(g.wideSegs));
+    take(q.segNew, 3 * size_t(g.wideSegs));
+    take(q.segEdges, 3 * size_t(g.wideSegs));
+    if (withNext) take(q.next, g.W);
+    if (thin) {
+        take(q.thinQueue0, g.thin_queue_entries());
+        take(q.thinQueue1, g.thin_queue_entries());
+        take(q.thinCount, 3 * size_t(dev::kThinMaxSegs));
+        take(q.thinEdges, dev::kThinMaxSegs);
+    }
+    return used;
+}
+
 int32_t* direct_result(const Query& q, int32_t* dst, size_t count, const char* what) {
     if (!dst || !check_result_range(dst, sizeof(int32_t) * count, q.g->device, what)) return nullptr;
     // a result in the query's own level array: the traversal reads there what it writes
@@ -517,28 +547,13 @@ blest_status blest_query_create(blest_device_graph* dg, uint32_t max_sources, bl
             BLEST_HIP(hipEventCreateWithFlags(&q.evIn, hipEventDisableTiming));
             BLEST_HIP(hipHostMalloc(reinterpret_cast<void**>(&q.hostCtrl), sizeof(dev::Ctrl), hipHostMallocDefault));
             std::memset(static_cast<void*>(q.hostCtrl), 0, sizeof(dev::Ctrl));
-            q.ctrl = q.alloc<dev::Ctrl>(1);
+            // One allocation for the state that stays inside the library (17 took longer than
+            // the rest of the call); the level arrays are their own, so that a result range
+            // that overruns them is told apart from one that fits.
+            const size_t bytes = carve_state(g, nullptr, q, false, g.thin, true);
+            carve_state(g, q.alloc<unsigned char>(bytes), q, false, g.thin, true);
             BLEST_HIP(hipMemset(q.ctrl, 0, sizeof(dev::Ctrl)));
             q.levels = q.alloc<int32_t>(size_t(g.n) * max_sources);
-            q.visited = q.alloc<unsigned long long>(g.W);
-            q.front0 = q.alloc<unsigned long long>(g.W);
-            q.front1 = q.alloc<unsigned long long>(g.W);
-            q.next = q.alloc<unsigned long long>(g.W);
-            q.nextB = q.alloc<uint8_t>(size_t(g.W) * 64);
-            q.list0 = q.alloc<uint32_t>(g.V);
-            q.list1 = q.alloc<uint32_t>(g.V);
-            q.chunk0 = q.alloc<uint2>(g.chunks);
-            q.chunk1 = q.alloc<uint2>(g.chunks);
-            q.segChunks = q.alloc<uint32_t>(3 * size_t(g.wideSegs));
-            q.segCount = q.alloc<uint32_t>(3 * size_t(g.wideSegs));
-            q.segNew = q.alloc<uint32_t>(3 * size_t(g.wideSegs));
-            q.segEdges = q.alloc<unsigned long long>(3 * size_t(g.wideSegs));
-            if (g.thin) {
-                q.thinQueue0 = q.alloc<uint32_t>(g.thin_queue_entries());
-                q.thinQueue1 = q.alloc<uint32_t>(g.thin_queue_entries());
-                q.thinCount = q.alloc<uint32_t>(3 * size_t(dev::kThinMaxSegs));
-                q.thinEdges = q.alloc<unsigned long long>(dev::kThinMaxSegs);
-            }
             if (g.hasPerm) q.levelsOut = q.alloc<int32_t>(size_t(g.n) * max_sources);
         } catch (...) {
             delete h;
@@ -582,11 +597,9 @@ blest_status blest_query_footprint(const blest_device_graph* dg, uint32_t max_so
         if (!dg || !bytes) throw Error(BLEST_ERR_INVALID_ARGUMENT, "null argument");
         const DeviceGraph& g = dg->g;
         if (max_sources == 0) max_sources = 1;
-        uint64_t b = sizeof(dev::Ctrl);
-        const uint64_t levels = 4ull * g.n * max_sources;
-        b += levels * (g.hasPerm ? 2 : 1);
-        b += 4ull * 8ull * g.W + 64ull * g.W + 2ull * 4ull * g.V + 2ull * 8ull * g.chunks + 3ull * 20ull * g.wideSegs;
-        if (g.thin) b += 8ull * g.thin_queue_entries() + 20ull * dev::kThinMaxSegs;
+        Query q;  // measured only
+        uint64_t b = carve_state(g, nullptr, q, false, g.thin, true);
+        b += 4ull * g.n * max_sources * (g.hasPerm ? 2 : 1);
         if (max_sources > 1) {
             const uint32_t nw = max_sources > 64 ? 2 : 1;
             b += (4ull + mbfs_history_levels(g.n, nw) + 1) * 8ull * g.n * nw + 4ull * 128 + 16ull * 128;

@@ -199,6 +199,12 @@ struct Query {
     ~Query();
 };
 
+// Lays a single-source traversal's state over `base` (256-byte aligned pieces; the level
+// array too when asked for, the vertex queues of a thin graph, the bitmap of the
+// label-propagation components) and returns the bytes it takes.  With base == nullptr it
+// only measures.
+size_t carve_state(const DeviceGraph& g, unsigned char* base, Query& q, bool withLevels, bool thin, bool withNext);
+
 // Level-loop driver: enqueues level(L) for L = 1, 2, ... in chunks and polls the
 // device's done flag after each chunk.  tail (nullable) enqueues the traversal's closing
 // kernel after each chunk: it stores the control block in q.hostCtrl and does its work
