@@ -83,44 +83,112 @@ __device__ __forceinline__ void expand_slice(uint32_t row, uint32_t hit, const u
     nextB[row] = 1;
 }
 
+// Resets the traversal state and, where it is small, runs level 1 on the way: one workgroup
+// per segment, each reading the root's slices (at most kFirstQuads quads: every workgroup
+// reads them all) and keeping the rows of its own words in LDS.  What it leaves are the
+// inputs of enqueued level 1: the root's (distance 1 to come), or level 1's discoveries
+// with a shift of one level in the state.  (Level 1 in the one-workgroup fused kernel took
+// 18-20 us on R-MAT 16 and 22 after an init kernel of 3 us: its chain of round trips
+// starts with the queue's, and only one CU works on it; here 5-9 us in all.)
+constexpr uint32_t kFirstQuads = 2 * kProducerBlock;
+constexpr uint32_t kFirstWords = 1024;  // bitmap words of a segment held in LDS
+
 __global__ void __launch_bounds__(kProducerBlock) bfs_init_kernel(GraphView g, BfsArgs a) {
-    const unsigned tid = blockIdx.x * blockDim.x + threadIdx.x, nthreads = gridDim.x * blockDim.x;
-    const uint32_t sw = a.src >> 6;
+    __shared__ unsigned long long sWord[kFirstWords], tmp64[16];
+    __shared__ unsigned tmp[32];
+    const unsigned t = threadIdx.x, nb = blockDim.x, b = t & 7;
+    const uint32_t ws = blockIdx.x * a.sv.wps, we = min(g.W, ws + a.sv.wps);
+    const uint32_t sw = a.src >> 6, r0 = a.src >> 3;
     const unsigned long long sb = 1ull << (a.src & 63);
-    for (uint32_t w = tid; w < g.W; w += nthreads) {
-        const unsigned long long x = (w == sw) ? sb : 0ull;
-        a.visited[w] = x;
-        a.front1[w] = x;
+    const uint32_t u0 = g.rsetUnit[r0], u1 = g.rsetUnit[r0 + 1];
+    const unsigned long long deg = g.csrPtr ? g.csrPtr[a.src + 1] - g.csrPtr[a.src] : 0ull;
+    const uint32_t q0 = u1 > u0 ? g.unitQuad[u0] : 0u, q1 = u1 > u0 ? g.unitQuad[u1] : 0u;
+    // the same on every workgroup; the direction rule is level_begin's
+    const bool first = a.fuseQuads && a.sv.wps <= kFirstWords && q1 - q0 <= kFirstQuads &&
+                       !(a.direction == 0 && g.csrPtr && double(deg) * a.alpha > double(g.nnz - min(deg, g.nnz)));
+    if (first) {
+        for (uint32_t w = ws + t; w < we; w += nb) sWord[w - ws] = 0ull;
+        __syncthreads();
+        uint4 r4[2];
+        uint32_t m[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t q = q0 + h * nb + t;
+            r4[h] = make_uint4(0, 0, 0, 0);
+            m[h] = 0;
+            if (q < q1) {
+                r4[h] = g.rows[q];
+                m[h] = g.masks[q] & ((1u << (a.src & 7)) * 0x01010101u);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t row[4] = {r4[h].x, r4[h].y, r4[h].z, r4[h].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t w = row[j] >> 6;
+                if (((m[h] >> (8 * j)) & 0xFFu) && w >= ws && w < we && row[j] != a.src)
+                    atomicOr(&sWord[w - ws], 1ull << (row[j] & 63));
+            }
+        }
     }
     unsigned long long* nb64 = reinterpret_cast<unsigned long long*>(a.nextB);
-    for (size_t i = tid; i < size_t(g.W) * 8; i += nthreads) nb64[i] = 0ull;
-    const uint32_t srcSeg = sw / a.sv.wps;
-    for (uint32_t s = tid; s < a.sv.segs; s += nthreads) {
-        uint32_t cnt = 0, news = 0, chunks = 0;
-        unsigned long long edges = 0;
-        if (s == srcSeg) {
-            const uint32_t r = a.src >> 3;
-            const uint32_t u0 = g.rsetUnit[r], u1 = g.rsetUnit[r + 1];
-            chunks = rset_chunks(u1 - u0);
-            if (chunks) {
-                for (uint32_t j = 0; j < chunks; ++j)
-                    a.chunk1[a.sv.chunkBase[s] + j] =
-                        make_uint2(u0 + j * kChunkVsets, min(kChunkVsets, u1 - u0 - j * kChunkVsets));
-            } else {
-                for (uint32_t u = u0; u < u1; ++u) a.list1[a.sv.segBase[s] + (u - u0)] = u;
-                cnt = u1 - u0;
+    for (size_t i = size_t(ws) * 8 + t; i < size_t(we) * 8; i += nb) nb64[i] = 0ull;
+    __syncthreads();
+    uint32_t* out = a.list1 + a.sv.segBase[blockIdx.x];
+    uint2* cout = a.chunk1 + a.sv.chunkBase[blockIdx.x];
+    unsigned long long news = 0, edges = 0;
+    unsigned written = 0, cwritten = 0;
+    for (uint32_t c0 = ws; c0 < we; c0 += nb / 8) {  // as bfs_update_kernel
+        const uint32_t w = c0 + t / 8, r = w * 8 + b;
+        const unsigned long long srcBit = w == sw ? sb : 0ull;
+        unsigned long long word = 0;
+        if (w < we) {
+            word = first ? sWord[w - ws] : srcBit;
+            if (b == 0) {
+                a.visited[w] = word | srcBit;
+                a.front1[w] = word;
             }
-            news = 1;
-            edges = g.csrPtr ? (g.csrPtr[a.src + 1] - g.csrPtr[a.src]) : 0ull;
         }
-        a.sc.count[a.sv.segs + s] = cnt;
-        a.sc.chunks[a.sv.segs + s] = chunks;
-        a.sc.news[a.sv.segs + s] = news;
-        a.sc.edges[a.sv.segs + s] = edges;
+        uint32_t start = 0, cnt = 0, chunks = 0;
+        const bool any = ((word >> (8 * b)) & 0xFFull) != 0;
+        if (any) {
+            start = g.rsetUnit[r];
+            cnt = g.rsetUnit[r + 1] - start;
+            chunks = rset_chunks(cnt);
+        }
+        if (!__syncthreads_or(any)) continue;
+        unsigned total, cex, ctotal;
+        const unsigned ex = block_exclusive_scan2(chunks ? 0u : cnt, chunks, tmp, total, cex, ctotal);
+        if (!chunks)
+            for (uint32_t j = 0; j < cnt; ++j) out[written + ex + j] = start + j;
+        for (uint32_t j = 0; j < chunks; ++j)
+            cout[cwritten + cex + j] = make_uint2(start + j * kChunkVsets, min(kChunkVsets, cnt - j * kChunkVsets));
+        written += total;
+        cwritten += ctotal;
+        // the rset's new vertices, a thread per rset: few at this level
+        for (uint32_t bits = uint32_t(word >> (8 * b)) & 0xFFu; bits; bits &= bits - 1) {
+            const uint32_t v = r * 8 + __builtin_ctz(bits);
+            a.levels[v] = first ? 1 : 0;
+            news += 1;
+            if (g.csrPtr) edges += g.csrPtr[v + 1] - g.csrPtr[v];
+        }
     }
-    if (tid == 0) {
-        a.levels[a.src] = 0;
+    news = block_sum_u64(news, tmp64);
+    edges = block_sum_u64(edges, tmp64);
+    if (t == 0) {
+        const uint32_t s = a.sv.segs + blockIdx.x;
+        a.sc.count[s] = written;
+        a.sc.chunks[s] = cwritten;
+        a.sc.news[s] = unsigned(news);
+        a.sc.edges[s] = edges;
+    }
+    if (blockIdx.x == 0 && t == 0) {
         level_state_reset(a.ctrl);
+        if (first) {
+            a.levels[a.src] = 0;
+            a.ctrl->state[0] = LevelState{0, 1, 1, 1, 0, 1, deg, 0ull};
+        }
     }
 }
 
@@ -273,8 +341,8 @@ __device__ __forceinline__ void fused_write_lists(const GraphView& g, const Fuse
     }
 }
 
-// head != 0: launched right after the init kernel, for level 1 (its inputs are the root's
-// rset and the reset state, so level_begin's counter reads are skipped).
+// head != 0: launched right after the init kernel; leaves the number of levels it ran in
+// ctrl->iterations (the next traversal's hint whether it is worth launching there).
 __global__ void __launch_bounds__(kFusedBlock) bfs_fused_kernel(GraphView g, BfsArgs a, unsigned Lk, int head) {
     const unsigned Lin = level_of(a.ctrl, a.levelFromCtrl, Lk);
     __shared__ unsigned pre[kMaxSegs], cpre[kMaxSegs];
@@ -295,57 +363,37 @@ __global__ void __launch_bounds__(kFusedBlock) bfs_fused_kernel(GraphView g, Bfs
     bool bottomUp = false;
     unsigned total = 0, ctotal = 0, Le = 0;
     LevelState cur, in;  // state of the level about to be expanded, and of the one before
-    if (head) {
-        // level 1: frontier {src}; level_begin's state, direction rule and list size
-        const uint32_t r = a.src >> 3;
-        const uint32_t u0 = g.rsetUnit[r], u1 = g.rsetUnit[r + 1];
-        const unsigned long long deg = g.csrPtr ? g.csrPtr[a.src + 1] - g.csrPtr[a.src] : 0ull;
-        const uint32_t ch = rset_chunks(u1 - u0);
-        total = ch ? 0u : u1 - u0;
-        ctotal = ch;
-        Le = 1;
-        cur = LevelState{0, 1, 1, 1, 0, 0, deg, 0ull};
-        bottomUp = a.direction == 0 && dp.canBottomUp &&
-                   double(deg) * a.alpha > double(g.nnz - min(deg, g.nnz));
-        if (bottomUp || total + ctotal * kChunkVsets > fuse_vsets(a.fuseQuads)) return;
-    } else {
-        if (!level_begin(c, a.sc, segs, Lin, dp, bottomUp, pre, &total, cpre, &ctotal, &Le, &cur, &in)) return;
-        // too big or bottom-up: the expand kernel enqueued as Lin takes it (its state slot
-        // written above is rewritten there from the same inputs)
-        const unsigned scale = cur.prevNf < in.prevNf ? kFuseShrinkScale : 1u;
-        if (bottomUp || total + ctotal * kChunkVsets > fuse_vsets(scale * a.fuseQuads)) return;
-        if (t == 0 && !c->tailFrom) c->tailFrom = Lin;
-    }
+    if (!level_begin(c, a.sc, segs, Lin, dp, bottomUp, pre, &total, cpre, &ctotal, &Le, &cur, &in)) return;
+    // too big or bottom-up: the expand kernel enqueued as Lin takes it (its state slot
+    // written above is rewritten there from the same inputs)
+    const unsigned scale = cur.prevNf < in.prevNf ? kFuseShrinkScale : 1u;
+    if (bottomUp || total + ctotal * kChunkVsets > fuse_vsets(scale * a.fuseQuads)) return;
+    if (t == 0 && !c->tailFrom) c->tailFrom = Lin;
+    if (t == 0 && head) c->iterations = 1;
     uint32_t* lists = (Lin & 1) ? a.list1 : a.list0;  // read first, rewritten when handing back
     uint2* chunks = (Lin & 1) ? a.chunk1 : a.chunk0;
     unsigned long long* F = (Lin & 1) ? a.front1 : a.front0;  // frontier bitmap, in and out
     const FusedInfo fi{sPf, sQ0, sFb, sU0, sUc};
     FusedQueue qc{pre, reinterpret_cast<uint32_t*>(a.nextB)};
     FusedQueue qn{cpre, reinterpret_cast<uint32_t*>(a.nextB) + g.R};
-    unsigned nq;
-    if (head) {
-        if (t == 0) pre[0] = a.src >> 3;  // read below by this thread only (entry 0)
-        nq = 1;
-    } else {
-        // list entry t and chunk entry t (at most one each): the first vset of an rset
-        uint32_t cand0 = kNoRset, cand1 = kNoRset;
-        if (t < total) {
-            const uint32_t v = list_entry(lists, a.sv, pre, t);
-            const uint32_t r = g.unitRset[v], rp = v ? g.unitRset[v - 1] : kNoRset;
-            if (rp != r) cand0 = r;
-        }
-        if (t < ctotal) {
-            const uint2 ch = chunk_entry(chunks, a.sv, cpre, t);
-            const uint32_t r = g.unitRset[ch.x], rp = ch.x ? g.unitRset[ch.x - 1] : kNoRset;
-            if (rp != r) cand1 = r;
-        }
-        if (t == 0) cntr = 0;
-        __syncthreads();  // the list prefixes are read: they become the queues
-        if (cand0 != kNoRset) qc.lds[atomicAdd(&cntr, 1u)] = cand0;  // <= 1024 + 64 entries
-        if (cand1 != kNoRset) qc.lds[atomicAdd(&cntr, 1u)] = cand1;
-        __syncthreads();
-        nq = __builtin_amdgcn_readfirstlane(cntr);
+    // list entry t and chunk entry t (at most one each): the first vset of an rset
+    uint32_t cand0 = kNoRset, cand1 = kNoRset;
+    if (t < total) {
+        const uint32_t v = list_entry(lists, a.sv, pre, t);
+        const uint32_t r = g.unitRset[v], rp = v ? g.unitRset[v - 1] : kNoRset;
+        if (rp != r) cand0 = r;
     }
+    if (t < ctotal) {
+        const uint2 ch = chunk_entry(chunks, a.sv, cpre, t);
+        const uint32_t r = g.unitRset[ch.x], rp = ch.x ? g.unitRset[ch.x - 1] : kNoRset;
+        if (rp != r) cand1 = r;
+    }
+    if (t == 0) cntr = 0;
+    __syncthreads();  // the list prefixes are read: they become the queues
+    if (cand0 != kNoRset) qc.lds[atomicAdd(&cntr, 1u)] = cand0;  // <= 1024 + 64 entries
+    if (cand1 != kNoRset) qc.lds[atomicAdd(&cntr, 1u)] = cand1;
+    __syncthreads();
+    unsigned nq = __builtin_amdgcn_readfirstlane(cntr);
     uint32_t* vis32 = reinterpret_cast<uint32_t*>(a.visited);
     uint32_t* f32 = reinterpret_cast<uint32_t*>(F);
     unsigned Lcur = Le;
@@ -1072,10 +1120,11 @@ void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
     const auto close = [&] {
         hipLaunchKernelGGL(dev::bfs_final_kernel, wide_grid(g), block, 0, q.stream, gv, a, oldToNew, dst, q.hostCtrl);
     };
-    hipLaunchKernelGGL(dev::bfs_init_kernel, wide_grid(g), block, 0, q.stream, gv, a);
+    hipLaunchKernelGGL(dev::bfs_init_kernel, grid, block, 0, q.stream, gv, a);
     // small levels between chunks of level kernels: from the root, and after every chunk
     const bool fused = a.fuseQuads != 0;
-    if (fused) hipLaunchKernelGGL(dev::bfs_fused_kernel, dim3(1), dim3(dev::kFusedBlock), 0, q.stream, gv, a, 1u, 1);
+    const bool head = fused && q.headSkip == 0;
+    if (head) hipLaunchKernelGGL(dev::bfs_fused_kernel, dim3(1), dim3(dev::kFusedBlock), 0, q.stream, gv, a, 1u, 1);
     if (trace) {
         size_t next = 0;
         auto mark = [&] {
@@ -1138,6 +1187,8 @@ void bfs_finish(Query& q, int32_t* hostLevels, blest_bfs_stats* st) {
     // level kernels the next traversal enqueues before the fused kernel takes over: up to
     // the final run of small shrinking levels, else all this traversal used
     q.levelHint = c.tailFrom ? c.tailFrom - 1 : c.levels - c.fusedLevels;
+    if (q.headSkip) --q.headSkip;
+    else if (c.iterations == 0) q.headSkip = 7;
     // (kept once seen: the bit-matrix levels that follow say the same of the graph)
     if (q.thinQueue0 && c.levels < dev::kThinFewLevels && c.visited / std::max(c.levels, 1u) > dev::kThinWideLevel) {
         q.levelHint = q.thinWide ? q.levelHint : 0;  // the hint counted queue levels

@@ -143,6 +143,8 @@ struct Query {
     // pinned: a chunk's closing kernel stores the control block here, so a poll is one
     // stream synchronisation (no copy, no second round trip for the totals)
     dev::Ctrl* hostCtrl = nullptr;
+    unsigned headSkip = 0;         // traversals to go without the fused kernel right after the init
+                                   // kernel, since the last one found no level to run there
     unsigned levelHint = 0;        // levels of the last traversal (sizes the first chunk)
     dev::Ctrl* ctrl = nullptr;
     int32_t* levels = nullptr;  // n * maxSources

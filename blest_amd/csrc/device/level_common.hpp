@@ -164,6 +164,7 @@ __device__ __forceinline__ void level_state_reset(Ctrl* c) {
     c->levelBase = 1;
     c->fusedLevels = 0;
     c->tailFrom = 0;
+    c->iterations = 0;
     c->state[0] = LevelState{0, 0, 0, 0, 0, 0, 0ull, 0ull};
     c->state[1] = c->state[0];
 }
