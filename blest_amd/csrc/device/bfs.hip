@@ -1214,9 +1214,14 @@ void bfs_finish(Query& q, int32_t* hostLevels, blest_bfs_stats* st) {
 
 // A traversal with its result in `levels` (nullable; host or device memory).
 static void bfs_run(Query& q, uint32_t src, int32_t* levels, bool trace, blest_bfs_stats* st) {
-    int32_t* dst = direct_result(q, levels, q.g->n, "levels");
+    const size_t n = q.g->n;
+    bool onHost = false;
+    int32_t* dst = direct_result(q, levels, n, "levels", &onHost);
+    int32_t* stage = onHost ? host_stage(q, n) : nullptr;
+    if (stage) dst = stage;
     bfs_launch(q, map_source(*q.g, src), trace, dst ? dst : (levels && q.g->hasPerm) ? q.levelsOut : nullptr);
     bfs_finish(q, dst ? nullptr : levels, st);
+    if (stage) std::memcpy(levels, stage, n * sizeof(int32_t));
 }
 
 }  // namespace blest

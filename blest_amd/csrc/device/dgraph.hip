@@ -23,6 +23,7 @@ Query::~Query() {
     for (hipEvent_t e : traceEvents) (void)hipEventDestroy(e);
     for (void* p : allocations) (void)hipFree(p);
     if (hostCtrl) (void)hipHostFree(hostCtrl);
+    if (hostStage) (void)hipHostFree(hostStage);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (evIn) (void)hipEventDestroy(evIn);
@@ -194,12 +195,31 @@ size_t carve_state(const DeviceGraph& g, unsigned char* base, Query& q, bool wit
     return used;
 }
 
-int32_t* direct_result(const Query& q, int32_t* dst, size_t count, const char* what) {
-    if (!dst || !check_result_range(dst, sizeof(int32_t) * count, q.g->device, what)) return nullptr;
+int32_t* direct_result(const Query& q, int32_t* dst, size_t count, const char* what, bool* onHost) {
+    const bool device = dst && check_result_range(dst, sizeof(int32_t) * count, q.g->device, what);
+    if (onHost) *onHost = dst && !device;
+    if (!device) return nullptr;
     // a result in the query's own level array: the traversal reads there what it writes
     const int32_t* own = q.levels;
     if (dst < own + size_t(q.g->n) * q.maxSources && own < dst + count) return nullptr;
     return dst;
+}
+
+int32_t* host_stage(Query& q, size_t count) {
+    if (count * sizeof(int32_t) > kStageBytes) return nullptr;
+    if (count > q.hostStageCount) {
+        if (q.hostStage) (void)hipHostFree(q.hostStage);
+        q.hostStage = nullptr;
+        q.hostStageCount = 0;
+        if (hipHostMalloc(reinterpret_cast<void**>(&q.hostStage), count * sizeof(int32_t), hipHostMallocDefault) !=
+            hipSuccess) {
+            (void)hipGetLastError();
+            q.hostStage = nullptr;
+            return nullptr;  // the ordinary copy
+        }
+        q.hostStageCount = count;
+    }
+    return q.hostStage;
 }
 
 uint32_t map_source(const DeviceGraph& g, uint32_t src) {
