@@ -28,15 +28,26 @@ __device__ __forceinline__ uint32_t column_of(const uint32_t* ptr, uint32_t lo, 
 // found[0] |= 1 where an edge j -> i has no edge i -> j (columns sorted), 2 where a row is
 // out of range.  A thread takes entries a workgroup apart, so a hub's list is spread over
 // workgroups; the columns of a tile are bounded once and searched between the bounds.
+// Bound by the dependent reads of the searches.  Half: only the entries whose column i is
+// the smaller one (fewer entries, then lower ID) are looked up, in that shorter list;
+// found[1] and found[2] count them and the others.  Entries ascending, each entry looked up
+// and present is another one of the second kind, so the graph is symmetric iff all are
+// present and the two counts agree.  found[0] |= 4 where a column is not strictly ascending:
+// that takes the search of every entry.  R-MAT 18 722 -> 312 us, R-MAT 22 17.7 -> 6.4 ms.
+template <bool Half>
 __global__ void __launch_bounds__(kCsrBlock) csr_symmetry_kernel(const uint32_t* ptr, const uint32_t* idx, uint32_t n,
-                                                                 uint32_t nnz, unsigned* found) {
+                                                                 uint32_t nnz, unsigned long long* found) {
     __shared__ uint32_t bound[2];
+    __shared__ unsigned sides[2];
     const uint32_t t0 = blockIdx.x * kTileEntries;  // < nnz
     const uint32_t count = min(kTileEntries, nnz - t0);
-    if (threadIdx.x < 2) bound[threadIdx.x] = column_of(ptr, 0, n - 1, threadIdx.x ? t0 + count - 1 : t0);
+    if (threadIdx.x < 2) {
+        bound[threadIdx.x] = column_of(ptr, 0, n - 1, threadIdx.x ? t0 + count - 1 : t0);
+        sides[threadIdx.x] = 0;
+    }
     __syncthreads();
     const uint32_t c0 = bound[0], c1 = bound[1];
-    unsigned bad = 0;
+    unsigned bad = 0, looked = 0, rest = 0;
     for (uint32_t k = threadIdx.x; k < count; k += kCsrBlock) {
         const uint32_t p = t0 + k, i = idx[p];
         if (i >= n) {
@@ -44,9 +55,20 @@ __global__ void __launch_bounds__(kCsrBlock) csr_symmetry_kernel(const uint32_t*
             continue;
         }
         const uint32_t j = column_of(ptr, c0, c1, p);
-        if (i == j) continue;
         uint32_t lo = ptr[i], hi = ptr[i + 1];
         const uint32_t end = hi;
+        if (Half) {
+            const uint32_t first = ptr[j], mine = ptr[j + 1] - first;
+            if (p > first && idx[p - 1] >= i) bad |= 4u;
+            if (i == j) continue;
+            if (hi - lo > mine || (hi - lo == mine && i > j)) {
+                ++rest;
+                continue;
+            }
+            ++looked;
+        } else if (i == j) {
+            continue;
+        }
         while (lo < hi) {  // first entry of column i that is not below j
             const uint32_t mid = lo + (hi - lo) / 2;
             if (idx[mid] < j) lo = mid + 1;
@@ -54,7 +76,13 @@ __global__ void __launch_bounds__(kCsrBlock) csr_symmetry_kernel(const uint32_t*
         }
         if (lo == end || idx[lo] != j) bad |= 1u;
     }
-    if (bad) atomicOr(found, bad);
+    if (Half) {
+        if (looked) atomicAdd(&sides[0], looked);
+        if (rest) atomicAdd(&sides[1], rest);
+        __syncthreads();
+        if (threadIdx.x < 2 && sides[threadIdx.x]) atomicAdd(&found[1 + threadIdx.x], (unsigned long long)sides[threadIdx.x]);
+    }
+    if (bad) atomicOr(found, (unsigned long long)bad);
 }
 
 // Radix keys that put the highest degree first; the sort is stable, so ties stay by ID.
@@ -138,15 +166,21 @@ bool csr_symmetric_on_device(const uint32_t* ptr, const uint32_t* idx, uint32_t 
     Scratch sc;
     StreamGuard sg;
     BLEST_HIP(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
-    unsigned* found = sc.alloc<unsigned>(1);
-    const unsigned zero = 0;
-    BLEST_HIP(hipMemcpyAsync(found, &zero, sizeof(zero), hipMemcpyHostToDevice, sg.s));
-    hipLaunchKernelGGL(dev::csr_symmetry_kernel, dim3((nnz - 1) / dev::kTileEntries + 1), dim3(dev::kCsrBlock), 0, sg.s,
-                       ptr, idx, n, nnz, found);
-    BLEST_HIP(hipGetLastError());
-    const unsigned got = read_one(found, sg.s);
-    if (got & 2u) throw Error(BLEST_ERR_INVALID_ARGUMENT, "row index out of range");
-    return got == 0;
+    unsigned long long* found = sc.alloc<unsigned long long>(3);
+    unsigned long long got[3] = {0, 0, 0};
+    const auto check = [&](auto kernel) {
+        got[0] = got[1] = got[2] = 0;
+        BLEST_HIP(hipMemcpyAsync(found, got, sizeof(got), hipMemcpyHostToDevice, sg.s));
+        hipLaunchKernelGGL(kernel, dim3((nnz - 1) / dev::kTileEntries + 1), dim3(dev::kCsrBlock), 0, sg.s, ptr, idx, n,
+                           nnz, found);
+        BLEST_HIP(hipGetLastError());
+        BLEST_HIP(hipMemcpyAsync(got, found, sizeof(got), hipMemcpyDeviceToHost, sg.s));
+        BLEST_HIP(hipStreamSynchronize(sg.s));
+        if (got[0] & 2u) throw Error(BLEST_ERR_INVALID_ARGUMENT, "row index out of range");
+    };
+    check(dev::csr_symmetry_kernel<true>);
+    if (got[0] & 4u) check(dev::csr_symmetry_kernel<false>);
+    return got[0] == 0 && got[1] == got[2];
 }
 
 void csr_sort_by_degree(const CSC& csr, const uint32_t* ptr, uint32_t* idx) {

@@ -45,6 +45,29 @@ def test_symmetry_on_device(blest, oracle, name):
             np.testing.assert_array_equal(blest.BVSSBFSKernel(dg).run(src).levels, oracle.bfs(n, hcp, hrows, src))
 
 
+@pytest.mark.parametrize("name", GRAPHS)
+def test_symmetry_balanced_and_repeated(blest, name):
+    """One edge short in each direction (as many entries look up their reverse as do not),
+    and lists with an entry twice: the host's answer."""
+    progress(f"case csr symmetry balanced {name}")
+    g = GRAPHS[name](blest)
+    cp, rows = g.arrays()
+    n, nnz = g.n, len(rows)
+    rng = np.random.default_rng(3)
+    for _ in range(6):
+        h = drop_edge(blest, n, cp, rows, int(rng.integers(nnz)))
+        hcp, hrows = h.arrays()
+        h = drop_edge(blest, n, hcp, hrows, int(rng.integers(nnz - 1)))
+        dg = blest.DeviceGraph(blest.BVSS().construct_from_csc(h), h, None)
+        assert dg.info()["symmetric"] == int(h.check_symmetry())
+    for p in sorted({0, nnz // 2, nnz - 1}):
+        tcp = cp.copy()
+        tcp[int(np.searchsorted(cp, p, side="right")):] += 1
+        h = blest.CSC.from_arrays(n, tcp, np.insert(rows, p, rows[p]))
+        dg = blest.DeviceGraph(blest.BVSS().construct_from_csc(g), h, None)
+        assert dg.info()["symmetric"] == int(h.check_symmetry())
+
+
 @pytest.mark.parametrize("n,src,dst", [(1, [], []), (64, [], []), (65, [0], [64]), (300, [0] * 299, list(range(1, 300)))])
 @pytest.mark.parametrize("bu_probe", [0, -1])
 def test_small_lists(blest, oracle, n, src, dst, bu_probe):
