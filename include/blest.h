@@ -198,8 +198,12 @@ typedef struct blest_device_opts {
                                 graphs with a resident CSR get segments of 4096 vertices down to one
                                 a CU for the single-source level kernels */
     double alpha;            /* top-down -> bottom-up when frontier edges > unexplored edges / alpha */
-    double beta;             /* bottom-up -> top-down when frontier vertices < n / beta */
-    int direction;           /* 0 = optimizing, 1 = top-down only, 2 = bottom-up after level 1 */
+    double beta;             /* bottom-up -> top-down when frontier vertices < n / beta and frontier
+                                edges <= unexplored edges */
+    int direction;           /* 0 = optimizing, 1 = top-down only, 2 = bottom-up after level 1.  Under 0,
+                                a symmetric graph with a resident CSR and either few vertices (at
+                                most 16384) or only short lists (grids, road networks) is searched
+                                by kernels of their own, all levels top-down */
     int keep_csr;            /* upload the bottom-up CSR (needed for direction != 1) */
     uint32_t timeout_ms;     /* bound on every in-kernel wait */
     int use_graphs;          /* level chunks replayed from a captured HIP graph: 0 = once a
@@ -212,7 +216,8 @@ typedef struct blest_device_opts {
     int32_t fuse_quads;      /* single-source BFS: a top-down level whose frontier's slices fill
                                 at most this many quads (4 slices) runs inside one workgroup,
                                 and so do the small levels after it, with no kernel boundary
-                                between them; 0 = default (2048), < 0 = never, at most 65536 */
+                                between them; 0 = default (2048), < 0 = never (nor the kernels of
+                                their own for small graphs and short lists), at most 65536 */
     int32_t bu_probe;        /* bottom-up: each vertex first tests its highest-degree
                                 in-neighbour (an n-entry array built at creation), then its
                                 list; 0 = default (on), < 0 = off (list order only) */
