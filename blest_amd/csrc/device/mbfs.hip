@@ -35,7 +35,6 @@ struct MbfsArgs {
     uint8_t* dirty;              // W bytes: word w holds a vertex whose `next` word was set this level
     uint32_t* list0;
     uint32_t* list1;
-    const uint32_t* srcs;
     uint32_t k;
     Ctrl* ctrl;
     SegView sv;
@@ -117,90 +116,83 @@ __device__ __forceinline__ unsigned long long* mfront(const MbfsArgs& a, uint32_
 // are first staged in LDS (wave w computes words 8w .. 8w+7).  Returns the count.
 struct ListLds {
     unsigned tmp[32];
-    unsigned long long act[kProducerBlock / 8];
 };
 
-template <int NW>
-__device__ __forceinline__ unsigned segment_list(const GraphView& g, const SegView& sv,
-                                                 const unsigned long long* f, uint32_t* list, ListLds& l) {
-    const uint32_t ws = blockIdx.x * sv.wps, we = min(g.W, ws + sv.wps);
-    constexpr unsigned kPer = kWave / 8;  // words per wave per chunk (a chunk is blockDim / 8 words)
-    const unsigned wave = threadIdx.x / kWave;
-    auto prep = [&](uint32_t c0) {
-        bool on[kPer];
-#pragma unroll
-        for (unsigned j = 0; j < kPer; ++j) {  // every word's loads first (at a valid address), then the ballots
-            const uint32_t w = c0 + wave * kPer + j, v = w * 64 + lane_id();
-            const bool ok = w < we && v < g.n;
-            Bits<NW> b;
-            b.load(f, ok ? v : 0u);
-            on[j] = ok && b.any();
-        }
-#pragma unroll
-        for (unsigned j = 0; j < kPer; ++j) {
-            const unsigned long long x = __ballot(on[j]);
-            if (lane_id() == 0) l.act[wave * kPer + j] = x;
-        }
-        __syncthreads();
-    };
-    // chunks start at ws + k * blockDim/8, so a word's place in its chunk is (w - ws) % (blockDim/8)
-    return block_write_vsets(
-        g.rsetUnit, ws, we, prep, [&](uint32_t w) { return l.act[(w - ws) % (blockDim.x / 8)]; },
-        list + sv.segBase[blockIdx.x], l.tmp);
-}
+struct MbfsRoots {
+    uint32_t v[128];  // reordered IDs
+};
 
+// Everything a traversal starts from, a workgroup per segment: its vertices' records cleared,
+// the roots among them set (level 0), counted and listed.  All of it is the segment's own,
+// so workgroup barriers order the steps, and the roots come as an argument.  Bound by the
+// cleared bytes on a large graph and by the launch on a small one.  (As a
+// copy of the roots, a clearing kernel, a kernel for the roots and one that read every
+// level-0 word back for the lists: 8.6 us of kernels and three more boundaries on R-MAT 14,
+// 66.6 on R-MAT 22 with 128 roots; here 4.9 and 49.)
 template <int NW>
-__global__ void __launch_bounds__(kProducerBlock) mbfs_init_kernel(GraphView g, MbfsArgs a) {
-    const unsigned tid = blockIdx.x * blockDim.x + threadIdx.x, nthreads = gridDim.x * blockDim.x;
-    unsigned long long* f0 = a.hist;  // level 0
+__global__ void __launch_bounds__(kProducerBlock) mbfs_start_kernel(GraphView g, MbfsArgs a, MbfsRoots roots) {
+    __shared__ ListLds l;
+    __shared__ uint32_t sRoot[128];  // the segment's roots
+    __shared__ unsigned sRoots;
+    __shared__ unsigned long long sEdges;
+    const uint32_t ws = blockIdx.x * a.sv.wps, we = min(g.W, ws + a.sv.wps);
+    if (threadIdx.x == 0) {
+        sRoots = 0;
+        sEdges = 0;
+    }
     // vertices without edges can only ever be reached by their own root: they start
     // saturated, so no slice or rset waits on them (the slots past n likewise)
-    for (uint32_t v = tid; v < g.W * 64; v += nthreads) {  // whole waves: 64 consecutive v
+    for (uint32_t w = ws + threadIdx.x / kWave; w < we; w += kProducerBlock / kWave) {
+        const uint32_t v = w * 64 + lane_id();
         const bool isolated = v >= g.n || (g.csrPtr && g.csrPtr[v + 1] == g.csrPtr[v]);
         const unsigned long long bits = __ballot(isolated);
         if (lane_id() == 0) {
-            a.full[v >> 6] = bits;
-            a.any[v >> 6] = 0ull;
-            a.any[g.W + (v >> 6)] = 0ull;
-            a.dirty[v >> 6] = 0;
+            a.full[w] = bits;
+            a.any[w] = 0ull;
+            a.any[g.W + w] = 0ull;
+            a.dirty[w] = 0;
         }
     }
-    for (size_t i = tid; i < size_t(g.n) * NW; i += nthreads) {
+    unsigned long long* f0 = a.hist;  // level 0
+    const size_t v1 = min(size_t(g.n), size_t(we) * 64);
+    for (size_t i = size_t(ws) * 64 * NW + threadIdx.x; i < v1 * NW; i += kProducerBlock) {
         f0[i] = 0ull;
         a.vn[2 * i] = 0ull;
         a.vn[2 * i + 1] = 0ull;
     }
-    for (uint32_t s = tid; s < a.sv.segs; s += nthreads) {
-        a.sc.news[a.sv.segs + s] = 0;
-        a.sc.edges[a.sv.segs + s] = 0;
-    }
-    if (tid == 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
         level_state_reset(a.ctrl);
         a.ctrl->histTop = 0;
     }
-}
-
-// Roots set their bits and level 0, and count into their segment's slot-1 counters.
-template <int NW>
-__global__ void mbfs_seed_kernel(GraphView g, MbfsArgs a) {
-    const unsigned j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= a.k) return;
-    const uint32_t v = a.srcs[j];
-    const unsigned long long bit = 1ull << (j & 63);
-    atomicOr(vis_at<NW>(a, v) + j / 64, bit);
-    atomicOr(&a.hist[size_t(v) * NW + j / 64], bit);
-    atomicOr(&a.any[v >> 6], 1ull << (v & 63));  // level 0: parity half 0
-    a.levels[size_t(j) * g.n + v] = 0;
-    const uint32_t seg = (v >> 6) / a.sv.wps;
-    atomicAdd(&a.sc.news[a.sv.segs + seg], 1u);
-    if (g.csrPtr) atomicAdd(&a.sc.edges[a.sv.segs + seg], (unsigned long long)(g.csrPtr[v + 1] - g.csrPtr[v]));
-}
-
-template <int NW>
-__global__ void __launch_bounds__(kProducerBlock) mbfs_first_list_kernel(GraphView g, MbfsArgs a) {
-    __shared__ ListLds l;
-    const unsigned cnt = segment_list<NW>(g, a.sv, a.hist, a.list1, l);
-    if (threadIdx.x == 0) a.sc.count[a.sv.segs + blockIdx.x] = cnt;
+    __syncthreads();
+    const unsigned j = threadIdx.x;
+    const uint32_t v = j < a.k ? roots.v[j] : 0u;
+    if (j < a.k && v >> 6 >= ws && v >> 6 < we) {
+        sRoot[atomicAdd(&sRoots, 1u)] = v;
+        const unsigned long long bit = 1ull << (j & 63);
+        atomicOr(vis_at<NW>(a, v) + j / 64, bit);
+        atomicOr(&f0[size_t(v) * NW + j / 64], bit);
+        atomicOr(&a.any[v >> 6], 1ull << (v & 63));  // level 0: parity half 0
+        a.levels[size_t(j) * g.n + v] = 0;
+        if (g.csrPtr) atomicAdd(&sEdges, (unsigned long long)(g.csrPtr[v + 1] - g.csrPtr[v]));
+    }
+    __syncthreads();
+    const unsigned count = sRoots;
+    unsigned listed = 0;
+    if (count)
+        listed = block_write_vsets(
+            g.rsetUnit, ws, we, [](uint32_t) {},
+            [&](uint32_t w) {
+                unsigned long long bits = 0;
+                for (unsigned i = 0; i < count; ++i) bits |= sRoot[i] >> 6 == w ? 1ull << (sRoot[i] & 63) : 0ull;
+                return bits;
+            },
+            a.list1 + a.sv.segBase[blockIdx.x], l.tmp);
+    if (threadIdx.x == 0) {
+        a.sc.news[a.sv.segs + blockIdx.x] = count;
+        a.sc.edges[a.sv.segs + blockIdx.x] = sEdges;
+        a.sc.count[a.sv.segs + blockIdx.x] = listed;
+    }
 }
 
 // Launched with mbfs_expand_block<NW>() threads per workgroup, one per segment: the grid
@@ -947,19 +939,16 @@ static void mbfs_ensure_state(Query& q, uint32_t nw) {
     q.mFull = q.alloc<unsigned long long>(g.W);
     q.mAny = q.alloc<unsigned long long>(2 * size_t(g.W));
     q.mDirty = q.alloc<uint8_t>(g.W);
-    if (!q.srcs) q.srcs = q.alloc<uint32_t>(128);
     if (!q.rootStats) q.rootStats = q.alloc<dev::RootStats>(128);
     q.mbfsWords = nw;
 }
 
 template <int NW, int ALGO>
-static void mbfs_enqueue_levels(Query& q, const dev::MbfsArgs& a, int32_t* dst) {
+static void mbfs_enqueue_levels(Query& q, const dev::MbfsArgs& a, const dev::MbfsRoots& roots, int32_t* dst) {
     DeviceGraph& g = *q.g;
     const GraphView gv = g.view();
     const dim3 grid = wide_grid(g), block(dev::kProducerBlock), eblock(dev::mbfs_expand_block<NW>());
-    hipLaunchKernelGGL(dev::mbfs_init_kernel<NW>, grid, block, 0, q.stream, gv, a);
-    hipLaunchKernelGGL(dev::mbfs_seed_kernel<NW>, dim3(2), dim3(64), 0, q.stream, gv, a);
-    hipLaunchKernelGGL(dev::mbfs_first_list_kernel<NW>, grid, block, 0, q.stream, gv, a);
+    hipLaunchKernelGGL(dev::mbfs_start_kernel<NW>, grid, block, 0, q.stream, gv, a, roots);
     dev::MbfsArgs ar = a;
     ar.levelFromCtrl = 1;
     run_levels(
@@ -1000,9 +989,8 @@ static void mbfs_run(Query& q, const uint32_t* srcs, uint32_t k, int32_t* hostLe
             check_result_range(rows[j], sizeof(int32_t) * size_t(g.n), g.device, "result row");
         }
     mbfs_ensure_state(q, nw);
-    std::vector<uint32_t> mapped(k);
-    for (uint32_t j = 0; j < k; ++j) mapped[j] = map_source(g, srcs[j]);
-    BLEST_HIP(hipMemcpyAsync(q.srcs, mapped.data(), 4 * size_t(k), hipMemcpyHostToDevice, q.stream));
+    dev::MbfsRoots roots{};
+    for (uint32_t j = 0; j < k; ++j) roots.v[j] = map_source(g, srcs[j]);
     dev::MbfsArgs a;
     a.levels = q.levels;
     a.vn = q.mVis;
@@ -1016,7 +1004,6 @@ static void mbfs_run(Query& q, const uint32_t* srcs, uint32_t k, int32_t* hostLe
     a.slicePull = (g.symmetric && !g.hasCsr) ? 1 : 0;
     a.list0 = q.list0;
     a.list1 = q.list1;
-    a.srcs = q.srcs;
     a.k = k;
     a.ctrl = q.ctrl;
     a.sv = g.wide_view();
@@ -1033,11 +1020,11 @@ static void mbfs_run(Query& q, const uint32_t* srcs, uint32_t k, int32_t* hostLe
     a.levelFromCtrl = 0;
     BLEST_HIP(hipEventRecord(q.ev0, q.stream));
     if (nw == 1) {
-        if (algo == 1) mbfs_enqueue_levels<1, 1>(q, a, dst);
-        else mbfs_enqueue_levels<1, 0>(q, a, dst);
+        if (algo == 1) mbfs_enqueue_levels<1, 1>(q, a, roots, dst);
+        else mbfs_enqueue_levels<1, 0>(q, a, roots, dst);
     } else {
-        if (algo == 1) mbfs_enqueue_levels<2, 1>(q, a, dst);
-        else mbfs_enqueue_levels<2, 0>(q, a, dst);
+        if (algo == 1) mbfs_enqueue_levels<2, 1>(q, a, roots, dst);
+        else mbfs_enqueue_levels<2, 0>(q, a, roots, dst);
     }
     const dev::Ctrl& c = *q.hostCtrl;  // as of the last poll
     q.levelHint = c.levels;
