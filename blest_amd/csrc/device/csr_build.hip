@@ -138,44 +138,42 @@ __global__ void csr_units_kernel(const uint32_t* ptr, uint32_t n, uint32_t own, 
 
 }  // namespace dev
 
-void csr_list_units(const uint32_t* ptr, uint32_t n, uint32_t own, uint32_t unit,
+void csr_list_units(hipStream_t st, const uint32_t* ptr, uint32_t n, uint32_t own, uint32_t unit,
                     const std::function<uint2*(uint32_t)>& units) {
     Scratch sc;
-    StreamGuard sg;
-    BLEST_HIP(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
+    const StreamDrain drain{st};
     uint32_t* cnt = sc.alloc<uint32_t>(size_t(n) + 1);
     uint32_t* first = sc.alloc<uint32_t>(size_t(n) + 1);
     const dim3 block(dev::kCsrBlock);
-    hipLaunchKernelGGL(dev::csr_unit_counts_kernel, grid_for(uint64_t(n) + 1), block, 0, sg.s, ptr, n, own, unit, cnt);
+    hipLaunchKernelGGL(dev::csr_unit_counts_kernel, grid_for(uint64_t(n) + 1), block, 0, st, ptr, n, own, unit, cnt);
     BLEST_HIP(hipGetLastError());
     size_t bytes = 0;
-    BLEST_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, cnt, first, size_t(n) + 1, sg.s));
+    BLEST_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, cnt, first, size_t(n) + 1, st));
     void* temp = sc.alloc<uint8_t>(bytes);
-    BLEST_HIP(hipcub::DeviceScan::ExclusiveSum(temp, bytes, cnt, first, size_t(n) + 1, sg.s));
-    const uint32_t count = read_one(first + n, sg.s);
+    BLEST_HIP(hipcub::DeviceScan::ExclusiveSum(temp, bytes, cnt, first, size_t(n) + 1, st));
+    const uint32_t count = read_one(first + n, st);
     uint2* out = units(count);
     if (count) {
-        hipLaunchKernelGGL(dev::csr_units_kernel, grid_for(count), block, 0, sg.s, ptr, n, own, unit, first, count, out);
+        hipLaunchKernelGGL(dev::csr_units_kernel, grid_for(count), block, 0, st, ptr, n, own, unit, first, count, out);
         BLEST_HIP(hipGetLastError());
     }
-    BLEST_HIP(hipStreamSynchronize(sg.s));
+    BLEST_HIP(hipStreamSynchronize(st));
 }
 
-bool csr_symmetric_on_device(const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t nnz) {
+bool csr_symmetric_on_device(hipStream_t st, const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t nnz) {
     if (nnz == 0) return true;
     Scratch sc;
-    StreamGuard sg;
-    BLEST_HIP(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
+    const StreamDrain drain{st};
     unsigned long long* found = sc.alloc<unsigned long long>(3);
     unsigned long long got[3] = {0, 0, 0};
     const auto check = [&](auto kernel) {
         got[0] = got[1] = got[2] = 0;
-        BLEST_HIP(hipMemcpyAsync(found, got, sizeof(got), hipMemcpyHostToDevice, sg.s));
-        hipLaunchKernelGGL(kernel, dim3((nnz - 1) / dev::kTileEntries + 1), dim3(dev::kCsrBlock), 0, sg.s, ptr, idx, n,
+        BLEST_HIP(hipMemcpyAsync(found, got, sizeof(got), hipMemcpyHostToDevice, st));
+        hipLaunchKernelGGL(kernel, dim3((nnz - 1) / dev::kTileEntries + 1), dim3(dev::kCsrBlock), 0, st, ptr, idx, n,
                            nnz, found);
         BLEST_HIP(hipGetLastError());
-        BLEST_HIP(hipMemcpyAsync(got, found, sizeof(got), hipMemcpyDeviceToHost, sg.s));
-        BLEST_HIP(hipStreamSynchronize(sg.s));
+        BLEST_HIP(hipMemcpyAsync(got, found, sizeof(got), hipMemcpyDeviceToHost, st));
+        BLEST_HIP(hipStreamSynchronize(st));
         if (got[0] & 2u) throw Error(BLEST_ERR_INVALID_ARGUMENT, "row index out of range");
     };
     check(dev::csr_symmetry_kernel<true>);
@@ -183,7 +181,7 @@ bool csr_symmetric_on_device(const uint32_t* ptr, const uint32_t* idx, uint32_t 
     return got[0] == 0 && got[1] == got[2];
 }
 
-void csr_sort_by_degree(const CSC& csr, const uint32_t* ptr, uint32_t* idx) {
+void csr_sort_by_degree(hipStream_t st, const CSC& csr, const uint32_t* ptr, uint32_t* idx) {
     const uint32_t n = csr.n;
     // column batches of at most 2^28 entries (one column may exceed that alone)
     constexpr uint64_t kBatch = uint64_t(1) << 28;
@@ -202,9 +200,7 @@ void csr_sort_by_degree(const CSC& csr, const uint32_t* ptr, uint32_t* idx) {
     }
     if (maxItems > 0x7FFFFFFFull || n > 0x7FFFFFFFu) throw Error(BLEST_ERR_UNSUPPORTED, "list too long for a device sort");
     Scratch sc;
-    StreamGuard sg;
-    BLEST_HIP(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
-    hipStream_t st = sg.s;
+    const StreamDrain drain{st};
     uint32_t* order = sc.alloc<uint32_t>(n);
     uint32_t* rank = sc.alloc<uint32_t>(n);
     uint32_t* keysIn = sc.alloc<uint32_t>(std::max<uint64_t>(maxItems, n));
@@ -239,15 +235,13 @@ void csr_sort_by_degree(const CSC& csr, const uint32_t* ptr, uint32_t* idx) {
     BLEST_HIP(hipStreamSynchronize(st));
 }
 
-void csr_marks(const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t words, uint32_t* probe,
-               unsigned long long* noIn) {
-    StreamGuard sg;
-    BLEST_HIP(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
+void csr_marks(hipStream_t st, const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t words,
+               uint32_t* probe, unsigned long long* noIn) {
     const dim3 block(dev::kCsrBlock);
-    if (probe) hipLaunchKernelGGL(dev::csr_probe_kernel, grid_for(n), block, 0, sg.s, ptr, idx, n, probe);
-    hipLaunchKernelGGL(dev::csr_no_in_kernel, grid_for(uint64_t(words) * 64), block, 0, sg.s, ptr, n, words, noIn);
+    if (probe) hipLaunchKernelGGL(dev::csr_probe_kernel, grid_for(n), block, 0, st, ptr, idx, n, probe);
+    hipLaunchKernelGGL(dev::csr_no_in_kernel, grid_for(uint64_t(words) * 64), block, 0, st, ptr, n, words, noIn);
     BLEST_HIP(hipGetLastError());
-    BLEST_HIP(hipStreamSynchronize(sg.s));
+    BLEST_HIP(hipStreamSynchronize(st));
 }
 
 }  // namespace blest

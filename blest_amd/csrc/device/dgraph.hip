@@ -7,6 +7,7 @@
 #include "csr_build.hpp"
 #include "dgraph.hpp"
 #include "level_common.hpp"
+#include "scratch.hpp"
 #include "segments.hpp"
 #include "small_traverse.hpp"
 
@@ -255,9 +256,9 @@ void blest_device_opts_default(blest_device_opts* o) {
 
 // On the device; on the host where the sort's scratch (about 2 GiB at most, 16 bytes a
 // vertex) does not fit beside the graph or a list is longer than a device sort takes.
-static void sort_lists_by_degree(const CSC& csr, const uint32_t* ptr, uint32_t* idx) {
+static void sort_lists_by_degree(hipStream_t st, const CSC& csr, const uint32_t* ptr, uint32_t* idx) {
     try {
-        csr_sort_by_degree(csr, ptr, idx);
+        csr_sort_by_degree(st, csr, ptr, idx);
         return;
     } catch (const Error& e) {
         if (e.code != BLEST_ERR_OUT_OF_DEVICE_MEMORY && e.code != BLEST_ERR_UNSUPPORTED) throw;
@@ -450,7 +451,9 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                         if (c.nnz()) BLEST_HIP(hipMemcpy(g.csrIdx, csr->rows.data(), 4 * c.nnz(), hipMemcpyHostToDevice));
                     };
                     upload();
-                    g.symmetric = csr_symmetric_on_device(g.csrPtr, g.csrIdx, c.n, uint32_t(c.nnz()));
+                    StreamGuard prep;
+                    BLEST_HIP(hipStreamCreateWithFlags(&prep.s, hipStreamNonBlocking));
+                    g.symmetric = csr_symmetric_on_device(prep.s, g.csrPtr, g.csrIdx, c.n, uint32_t(c.nnz()));
                     if (!ghIsCsr && !g.symmetric) {
                         tr = csc_transpose(c);
                         csr = &tr;
@@ -463,7 +466,7 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                         // coalesced by a sweep's first probe instead of one random index line
                         // per vertex.  Levels do not depend on the scan order, and the
                         // multi-source sweeps read whole lists.
-                        sort_lists_by_degree(*csr, g.csrPtr, g.csrIdx);
+                        sort_lists_by_degree(prep.s, *csr, g.csrPtr, g.csrIdx);
                         g.probe = g.alloc<uint32_t>(c.n);
                     }
                     g.hasCsr = true;
@@ -476,8 +479,8 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                     g.thinSegs = ((g.W - 1) >> g.thinShift) + 1;
                     // vertices without in-neighbours: a bottom-up sweep skips them
                     g.noIn = g.alloc<unsigned long long>(g.W);
-                    csr_marks(g.csrPtr, g.csrIdx, c.n, g.W, g.probe, g.noIn);
-                    csr_list_units(g.csrPtr, c.n, kPullOwn, kPullUnit, [&](uint32_t count) {
+                    csr_marks(prep.s, g.csrPtr, g.csrIdx, c.n, g.W, g.probe, g.noIn);
+                    csr_list_units(prep.s, g.csrPtr, c.n, kPullOwn, kPullUnit, [&](uint32_t count) {
                         g.pullCount = count;
                         return g.pullUnits = g.alloc<uint2>(count);
                     });

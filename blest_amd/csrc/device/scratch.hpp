@@ -32,6 +32,12 @@ struct StreamGuard {
     }
 };
 
+// Waits for a stream that outlives the step, so that the step's buffers are free to go.
+struct StreamDrain {
+    hipStream_t s;
+    ~StreamDrain() { (void)hipStreamSynchronize(s); }
+};
+
 inline dim3 grid_for(uint64_t items, unsigned block = 256) {
     return dim3(unsigned(std::max<uint64_t>(1, std::min<uint64_t>((items + block - 1) / block, 65536))));
 }
