@@ -483,10 +483,13 @@ static void cc_run(Query& q, int algo, uint32_t* hostLabels, blest_cc_stats* st)
     // fewer swaps (1023-square grid 157 -> 96 us for the second entry, 8 -> 2 workgroups per CU)
     const dim3 few(std::min<uint32_t>(grid.x, uint32_t(g.cus) * 2));
     if (!q.labels) {
-        q.labels = q.alloc<uint32_t>(g.n);
-        q.labelsAux = q.alloc<uint32_t>(g.n);
-        q.ccCounts = q.alloc<uint32_t>(2 * size_t(g.cus) * 8 + 1);
+        // one allocation: all of it or none, so that a call that found no room leaves
+        // nothing half made for the next one
+        const size_t n = (size_t(g.n) + 63) / 64 * 64, counts = 2 * size_t(g.cus) * 8 + 1;
         q.hostCcCounts.resize(size_t(g.cus) * 8);
+        q.labels = q.alloc<uint32_t>(2 * n + counts);
+        q.labelsAux = q.labels + n;
+        q.ccCounts = q.labelsAux + n;
     }
     GraphView gv = g.view();
     unsigned iterations = 1;

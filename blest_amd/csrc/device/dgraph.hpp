@@ -16,13 +16,18 @@
 
 namespace blest {
 
+// The runtime keeps a failed call's error for the thread's next hipGetLastError, which is
+// the check after a launch: taken here, so that the next call on the thread does not fail
+// for what went wrong in this one.
 #define BLEST_HIP(call)                                                                        \
     do {                                                                                       \
         hipError_t e_ = (call);                                                                \
-        if (e_ != hipSuccess)                                                                  \
+        if (e_ != hipSuccess) {                                                                \
+            (void)hipGetLastError();                                                           \
             throw ::blest::Error(e_ == hipErrorOutOfMemory ? BLEST_ERR_OUT_OF_DEVICE_MEMORY    \
                                                            : BLEST_ERR_DEVICE,                 \
                                  std::string(#call) + ": " + hipGetErrorString(e_));           \
+        }                                                                                      \
     } while (0)
 
 // Read-only view of the device graph passed by value to kernels.

@@ -920,10 +920,23 @@ static void mbfs_ensure_state(Query& q, uint32_t nw) {
     // (declared in dgraph.hpp: the history depth also sizes the query footprint)
     DeviceGraph& g = *q.g;
     if (q.mbfsWords >= nw) return;
-    for (void* p : {static_cast<void*>(q.mVis), static_cast<void*>(q.mFront0), static_cast<void*>(q.mFront1),
-                    static_cast<void*>(q.mHist), static_cast<void*>(q.mFull), static_cast<void*>(q.mAny),
-                    static_cast<void*>(q.mDirty)})
-        q.release(p);
+    // all of the state or none: without the words its old arrays are gone, and an
+    // allocation that fails gives back those before it
+    const auto drop = [&] {
+        q.mbfsWords = 0;
+        const auto give = [&]<class T>(T*& p) {
+            q.release(p);
+            p = nullptr;
+        };
+        give(q.mVis);
+        give(q.mFront0);
+        give(q.mFront1);
+        give(q.mHist);
+        give(q.mFull);
+        give(q.mAny);
+        give(q.mDirty);
+    };
+    drop();
     // a new layout invalidates every captured multi-source level chunk
     for (int k : {kGraphMbfs1, kGraphMbfs2})
         if (q.graphs[k].exec) {
@@ -931,15 +944,20 @@ static void mbfs_ensure_state(Query& q, uint32_t nw) {
             q.graphs[k].exec = nullptr;
         }
     const size_t words = size_t(g.n) * nw;
-    q.mVis = q.alloc<unsigned long long>(2 * words);  // visited + next, interleaved per vertex
-    q.mFront0 = q.alloc<unsigned long long>(words);
-    q.mFront1 = q.alloc<unsigned long long>(words);
-    q.mHistLevels = mbfs_history_levels(g.n, nw);
-    q.mHist = q.alloc<unsigned long long>(words * (q.mHistLevels + 1));
-    q.mFull = q.alloc<unsigned long long>(g.W);
-    q.mAny = q.alloc<unsigned long long>(2 * size_t(g.W));
-    q.mDirty = q.alloc<uint8_t>(g.W);
-    if (!q.rootStats) q.rootStats = q.alloc<dev::RootStats>(128);
+    try {
+        q.mVis = q.alloc<unsigned long long>(2 * words);  // visited + next, interleaved per vertex
+        q.mFront0 = q.alloc<unsigned long long>(words);
+        q.mFront1 = q.alloc<unsigned long long>(words);
+        q.mHistLevels = mbfs_history_levels(g.n, nw);
+        q.mHist = q.alloc<unsigned long long>(words * (q.mHistLevels + 1));
+        q.mFull = q.alloc<unsigned long long>(g.W);
+        q.mAny = q.alloc<unsigned long long>(2 * size_t(g.W));
+        q.mDirty = q.alloc<uint8_t>(g.W);
+        if (!q.rootStats) q.rootStats = q.alloc<dev::RootStats>(128);
+    } catch (...) {
+        drop();
+        throw;
+    }
     q.mbfsWords = nw;
 }
 
