@@ -711,19 +711,19 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID bfs_expand
         }
         int k = cand ? __builtin_ctz(cand) : kBuGroup;
         uint32_t p = pick(pb, k) + 1, p1 = pick(pe, k);
-        uint32_t budget = p + kBuBudget;
+        uint32_t budget = part_end(p, p1, kBuBudget);
         unsigned step = 2;
         while (k < kBuGroup) {  // p < p1 here
-            const uint32_t lim = min(p + step, p1);
+            const uint32_t len = min(step, p1 - p);
             uint32_t nb[kBuBatch], fw[kBuBatch];
 #pragma unroll
-            for (int i = 0; i < kBuBatch; ++i) nb[i] = p + i < lim ? g.csrIdx[p + i] : 0u;
+            for (int i = 0; i < kBuBatch; ++i) nb[i] = uint32_t(i) < len ? g.csrIdx[p + i] : 0u;
 #pragma unroll
-            for (int i = 0; i < kBuBatch; ++i) fw[i] = p + i < lim ? fin32[nb[i] >> 5] : 0u;
+            for (int i = 0; i < kBuBatch; ++i) fw[i] = uint32_t(i) < len ? fin32[nb[i] >> 5] : 0u;
             bool hit = false;
 #pragma unroll
             for (int i = 0; i < kBuBatch; ++i) hit |= (fw[i] >> (nb[i] & 31)) & 1u;
-            p = lim;
+            p += len;
             step = min(2 * step, unsigned(kBuBatch));
             bool next = hit || p >= p1;
             if (!next && p >= budget) {
@@ -742,7 +742,7 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID bfs_expand
                 k = cand ? __builtin_ctz(cand) : kBuGroup;
                 p = pick(pb, k) + 1;
                 p1 = pick(pe, k);
-                budget = p + kBuBudget;
+                budget = part_end(p, p1, kBuBudget);
                 step = 2;
             }
         }
@@ -770,9 +770,9 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID bfs_expand
         const uint32_t u = heavyU[h];
         const uint32_t p0 = g.csrPtr[u], p1 = g.csrPtr[u + 1];
         bool hit = false;
-        for (uint32_t q0 = heavyP[h]; q0 < p1 && !hit; q0 += kWave) {  // wave-uniform
-            const uint32_t q = q0 + lane;
-            hit = __ballot(q < p1 && test_bit(fin, g.csrIdx[min(q, p1 - 1)])) != 0ull;
+        for (uint32_t q0 = heavyP[h]; q0 < p1 && !hit; q0 = part_end(q0, p1, kWave)) {  // wave-uniform
+            const bool ok = in_part(q0, lane, p1);
+            hit = __ballot(ok && test_bit(fin, g.csrIdx[ok ? q0 + lane : q0])) != 0ull;
         }
         if (hit && lane == 0) {
             const unsigned long long bit = 1ull << (u & 63);

@@ -204,7 +204,7 @@ __global__ void __launch_bounds__(kCcBlock) cc_sample_hook_kernel(GraphView g, u
                                                                   uint32_t last) {
     for (uint32_t v = blockIdx.x * kCcBlock + threadIdx.x; v < g.n; v += gridDim.x * kCcBlock) {
         const uint32_t b = g.csrPtr[v], e = g.csrPtr[v + 1];
-        for (uint32_t i = b + first; i < min(e, b + last); ++i) {
+        for (uint32_t i = part_end(b, e, first); i < part_end(b, e, last); ++i) {
             const uint32_t u = g.csrIdx[i];
             if (ld_parent_near(p, u) != ld_parent_near(p, v)) hook_near(p, v, u);
         }
@@ -235,8 +235,8 @@ __global__ void __launch_bounds__(kCcBlock) cc_rest_kernel(GraphView g, uint32_t
     for (uint32_t v = blockIdx.x * kCcBlock + threadIdx.x; v < n64; v += gridDim.x * kCcBlock) {
         uint32_t b = 0, e = 0;
         if (v < g.n && ld_parent_near(p, v) != big) {
-            b = g.csrPtr[v] + kCcSampled + 1;
             e = g.csrPtr[v + 1];
+            b = part_end(g.csrPtr[v], e, kCcSampled + 1);
         }
         const bool heavy = b < e && e - b > kCcHeavy;
         if (!heavy)
@@ -244,7 +244,7 @@ __global__ void __launch_bounds__(kCcBlock) cc_rest_kernel(GraphView g, uint32_t
         for (unsigned long long h = __ballot(heavy); h; h &= h - 1) {
             const int l = __builtin_ctzll(h);
             const uint32_t hv = __shfl(v, l, kWave), hb = __shfl(b, l, kWave), he = __shfl(e, l, kWave);
-            for (uint32_t i = hb + lane; i < he; i += kWave) hook_near(p, hv, g.csrIdx[i]);
+            for (uint32_t i = lane; in_part(hb, i, he); i += kWave) hook_near(p, hv, g.csrIdx[hb + i]);
         }
     }
 }

@@ -124,7 +124,7 @@ __global__ void csr_no_in_kernel(const uint32_t* ptr, uint32_t n, uint32_t words
 __global__ void csr_unit_counts_kernel(const uint32_t* ptr, uint32_t n, uint32_t own, uint32_t unit, uint32_t* cnt) {
     for (uint64_t v = blockIdx.x * uint64_t(kCsrBlock) + threadIdx.x; v <= n; v += uint64_t(gridDim.x) * kCsrBlock) {
         const uint32_t deg = v < n ? ptr[v + 1] - ptr[v] : 0u;
-        cnt[v] = deg > own ? (deg - own + unit - 1) / unit : 0u;
+        cnt[v] = deg > own ? (deg - own - 1) / unit + 1 : 0u;
     }
 }
 

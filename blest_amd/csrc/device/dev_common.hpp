@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "list_range.hpp"
+
 namespace blest {
 namespace dev {
 

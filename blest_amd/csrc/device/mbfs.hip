@@ -272,19 +272,18 @@ __device__ __forceinline__ void mbfs_pull_csr(const GraphView& g, const MbfsArgs
             const int from = row == 0 ? l[0] : row == 1 ? l[1] : row == 2 ? l[2] : l[3];
             const int at = max(from, 0);
             const uint32_t q0 = __shfl(p0, at, kWave), end = __shfl(p1, at, kWave);  // every lane shuffles
-            const uint32_t q1 = from < 0 ? q0 : min(end, q0 + kPullOwn);
+            const uint32_t q1 = from < 0 ? q0 : part_end(q0, end, kPullOwn);
             Bits<NW> miss, acc;
             acc.zero();
 #pragma unroll
             for (int i = 0; i < NW; ++i) miss.w[i] = __shfl(need.w[i], at, kWave);
             bool done = false;
             for (uint32_t s = 0; s < kPullOwn; s += 16) {
-                const bool act = !done && q0 + s < q1;
+                const bool act = !done && in_part(q0, s, q1);
                 if (!__ballot(act)) break;
-                const uint32_t q = q0 + s + sub;
                 Bits<NW> F;
                 F.zero();
-                if (act && q < q1) F.load(fin, g.csrIdx[q]);
+                if (act && in_part(q0, s + sub, q1)) F.load(fin, g.csrIdx[q0 + s + sub]);
                 done = true;
 #pragma unroll
                 for (int i = 0; i < NW; ++i) {
@@ -317,7 +316,7 @@ __device__ __forceinline__ void mbfs_pull_csr(const GraphView& g, const MbfsArgs
         const uint2 hu = g.pullUnits[h];
         const uint32_t v = __builtin_amdgcn_readfirstlane(hu.x), p0 = __builtin_amdgcn_readfirstlane(hu.y);
         if (test_bit(a.full, v)) continue;
-        const uint32_t p1 = min(g.csrPtr[v + 1], p0 + kPullUnit);
+        const uint32_t p1 = part_end(p0, g.csrPtr[v + 1], kPullUnit);
         const unsigned long long* rec = vis_at<NW>(a, v);
         Bits<NW> need, got;
         got.zero();
@@ -328,14 +327,13 @@ __device__ __forceinline__ void mbfs_pull_csr(const GraphView& g, const MbfsArgs
             open |= need.w[i] != 0;
         }
         if (!__ballot(open)) continue;
-        const uint32_t p = p0 + lane * 4;
-        if (p < p1) {
-            const u32x4_a4 u = *reinterpret_cast<const u32x4_a4*>(g.csrIdx + p);
+        if (in_part(p0, lane * 4, p1)) {
+            const u32x4_a4 u = *reinterpret_cast<const u32x4_a4*>(g.csrIdx + p0 + lane * 4);
             Bits<NW> F[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 F[j].zero();
-                if (p + j < p1) F[j].load(fin, u[j]);
+                if (in_part(p0, lane * 4 + j, p1)) F[j].load(fin, u[j]);
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j)
