@@ -236,7 +236,7 @@ BVSS bvss_build_on_device(const CSC& g, bool fullPadding, int device) {
         maxSegs = std::max<uint64_t>(maxSegs, r1 - r0);
     }
     if (maxItems > uint64_t(0x7FFFFFFF)) throw Error(BLEST_ERR_UNSUPPORTED, "an rset holds more than 2^31 entries");
-    uint32_t* keysIn = sc.alloc<uint32_t>(maxItems);
+    uint32_t* keysIn = sc.alloc<uint32_t>(std::max<uint64_t>(maxItems, 2));
     uint32_t* keysOut = sc.alloc<uint32_t>(maxItems);
     uint32_t* flag = sc.alloc<uint32_t>(maxItems);
     uint32_t* pos = sc.alloc<uint32_t>(maxItems);
@@ -323,9 +323,10 @@ BVSS bvss_build_on_device(const CSC& g, bool fullPadding, int device) {
     hipLaunchKernelGGL(dev::bb_scatter_kernel, grid_for(sreal), dim3(256), 0, st, sRows, sMasks,
                        (unsigned long long)sreal, sliceStart, rsetSlot, R, int(fullPadding), dRowIds,
                        reinterpret_cast<uint8_t*>(dMasks));
-    constexpr uint32_t kCountBlocks = 1024;
-    unsigned long long* dBits = sc.alloc<unsigned long long>(kCountBlocks);
-    hipLaunchKernelGGL(dev::bb_edges_kernel, dim3(kCountBlocks), dim3(256), 0, st, sMasks, (unsigned long long)sreal, dBits);
+    // the sort's keys are done with: their place takes the counts
+    const uint32_t countBlocks = uint32_t(std::min<uint64_t>(1024, std::max<uint64_t>(maxItems, 2) / 2));
+    unsigned long long* dBits = reinterpret_cast<unsigned long long*>(keysIn);
+    hipLaunchKernelGGL(dev::bb_edges_kernel, dim3(countBlocks), dim3(256), 0, st, sMasks, (unsigned long long)sreal, dBits);
     hipLaunchKernelGGL(dev::bb_divergence_kernel, grid_for(V), dim3(256), 0, st, dSsp, dRowIds, V, dTerm);
     BLEST_HIP(hipGetLastError());
 
@@ -343,7 +344,7 @@ BVSS bvss_build_on_device(const CSC& g, bool fullPadding, int device) {
     b.rowIds.resize(S);
     b.masks.resize(S / 4);
     std::vector<double> term(V);
-    std::vector<unsigned long long> bits(kCountBlocks);
+    std::vector<unsigned long long> bits(countBlocks);
     BLEST_HIP(hipMemcpyAsync(bits.data(), dBits, 8 * bits.size(), hipMemcpyDeviceToHost, st));
     BLEST_HIP(hipMemcpyAsync(b.sliceSetPtrs.data(), dSsp, 8 * (size_t(V) + 1), hipMemcpyDeviceToHost, st));
     if (V) BLEST_HIP(hipMemcpyAsync(b.virtualToReal.data(), dV2r, 4 * size_t(V), hipMemcpyDeviceToHost, st));

@@ -120,51 +120,12 @@ __global__ void csr_no_in_kernel(const uint32_t* ptr, uint32_t n, uint32_t words
     }
 }
 
-// cnt[v] = units of list v (cnt[n] = 0, so an exclusive scan ends in the total)
-__global__ void csr_unit_counts_kernel(const uint32_t* ptr, uint32_t n, uint32_t own, uint32_t unit, uint32_t* cnt) {
-    for (uint64_t v = blockIdx.x * uint64_t(kCsrBlock) + threadIdx.x; v <= n; v += uint64_t(gridDim.x) * kCsrBlock) {
-        const uint32_t deg = v < n ? ptr[v + 1] - ptr[v] : 0u;
-        cnt[v] = deg > own ? (deg - own - 1) / unit + 1 : 0u;
-    }
-}
-
-__global__ void csr_units_kernel(const uint32_t* ptr, uint32_t n, uint32_t own, uint32_t unit, const uint32_t* first,
-                                 uint32_t count, uint2* units) {
-    for (uint64_t u = blockIdx.x * uint64_t(kCsrBlock) + threadIdx.x; u < count; u += uint64_t(gridDim.x) * kCsrBlock) {
-        const uint32_t v = column_of(first, 0, n - 1, uint32_t(u));
-        units[u] = make_uint2(v, ptr[v] + own + (uint32_t(u) - first[v]) * unit);
-    }
-}
-
 }  // namespace dev
 
-void csr_list_units(hipStream_t st, const uint32_t* ptr, uint32_t n, uint32_t own, uint32_t unit,
-                    const std::function<uint2*(uint32_t)>& units) {
-    Scratch sc;
-    const StreamDrain drain{st};
-    uint32_t* cnt = sc.alloc<uint32_t>(size_t(n) + 1);
-    uint32_t* first = sc.alloc<uint32_t>(size_t(n) + 1);
-    const dim3 block(dev::kCsrBlock);
-    hipLaunchKernelGGL(dev::csr_unit_counts_kernel, grid_for(uint64_t(n) + 1), block, 0, st, ptr, n, own, unit, cnt);
-    BLEST_HIP(hipGetLastError());
-    size_t bytes = 0;
-    BLEST_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, cnt, first, size_t(n) + 1, st));
-    void* temp = sc.alloc<uint8_t>(bytes);
-    BLEST_HIP(hipcub::DeviceScan::ExclusiveSum(temp, bytes, cnt, first, size_t(n) + 1, st));
-    const uint32_t count = read_one(first + n, st);
-    uint2* out = units(count);
-    if (count) {
-        hipLaunchKernelGGL(dev::csr_units_kernel, grid_for(count), block, 0, st, ptr, n, own, unit, first, count, out);
-        BLEST_HIP(hipGetLastError());
-    }
-    BLEST_HIP(hipStreamSynchronize(st));
-}
-
-bool csr_symmetric_on_device(hipStream_t st, const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t nnz) {
+bool csr_symmetric_on_device(hipStream_t st, const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t nnz,
+                             unsigned long long* found) {
     if (nnz == 0) return true;
-    Scratch sc;
     const StreamDrain drain{st};
-    unsigned long long* found = sc.alloc<unsigned long long>(3);
     unsigned long long got[3] = {0, 0, 0};
     const auto check = [&](auto kernel) {
         got[0] = got[1] = got[2] = 0;

@@ -6,25 +6,19 @@
 
 #include <hip/hip_runtime.h>
 
-#include <functional>
-
 #include "../csc.hpp"
 
 namespace blest {
 
 // Whether every stored edge has its reverse (columns sorted); throws
-// BLEST_ERR_INVALID_ARGUMENT for an entry that is not below n.
-bool csr_symmetric_on_device(hipStream_t st, const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t nnz);
+// BLEST_ERR_INVALID_ARGUMENT for an entry that is not below n.  found: room for 3 words.
+bool csr_symmetric_on_device(hipStream_t st, const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t nnz,
+                             unsigned long long* found);
 // Orders every list by degree, highest first, ties by ID; csr: the same lists on the host.
 void csr_sort_by_degree(hipStream_t st, const CSC& csr, const uint32_t* ptr, uint32_t* idx);
 // probe (nullable): each list's first entry, 0 for an empty one; noIn: bit v of the words
 // set where list v is empty.
 void csr_marks(hipStream_t st, const uint32_t* ptr, const uint32_t* idx, uint32_t n, uint32_t words,
                uint32_t* probe, unsigned long long* noIn);
-
-// Units of the lists longer than `own` entries: how many, and (vertex, first entry) of each
-// unit of `unit` entries into units(count), which allocates.
-void csr_list_units(hipStream_t st, const uint32_t* ptr, uint32_t n, uint32_t own, uint32_t unit,
-                    const std::function<uint2*(uint32_t)>& units);
 
 }  // namespace blest

@@ -276,6 +276,22 @@ static void sort_lists_by_degree(hipStream_t st, const CSC& csr, const uint32_t*
     BLEST_HIP(hipMemcpy(idx, sorted.data(), 4 * sorted.size(), hipMemcpyHostToDevice));
 }
 
+// (vertex, first entry) of the list parts that multi-source pull levels deal out; none
+// where no list is longer than kPullOwn.  From the host's copy of the offsets: no scratch.
+static std::vector<uint2> pull_units(const std::vector<uint32_t>& cp, uint32_t n) {
+    const unsigned threads = n < (1u << 20) ? 1u : std::min(hw_threads(), 16u);
+    std::vector<std::vector<uint2>> parts(threads);
+    parallel_blocks(n, threads, [&](uint64_t v0, uint64_t v1, unsigned t) {
+        for (uint64_t v = v0; v < v1; ++v)
+            if (cp[v + 1] - cp[v] > kPullOwn)
+                for (uint32_t p = cp[v] + kPullOwn; p < cp[v + 1]; p = dev::part_end(p, cp[v + 1], kPullUnit))
+                    parts[t].push_back(make_uint2(uint32_t(v), p));
+    });
+    std::vector<uint2> units = std::move(parts[0]);
+    for (unsigned t = 1; t < threads; ++t) units.insert(units.end(), parts[t].begin(), parts[t].end());
+    return units;
+}
+
 // gh: the CSC the BVSS was built from (ghIsCsr = false; its transpose is the bottom-up
 // CSR unless the graph is symmetric), or that transpose itself (ghIsCsr = true, as the
 // reference's BVSS keeps it, BVSS::getCSR()).
@@ -446,6 +462,9 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                     const CSC* csr = &c;
                     g.csrPtr = g.alloc<uint32_t>(size_t(c.n) + 1);
                     g.csrIdx = g.alloc<uint32_t>(c.nnz() + dev::kBatchTd);  // small_traverse reads whole steps
+                    // vertices without in-neighbours (a bottom-up sweep skips them); before
+                    // that the symmetry check's counters
+                    g.noIn = g.alloc<unsigned long long>(std::max(g.W, 3u));
                     const auto upload = [&] {
                         BLEST_HIP(hipMemcpy(g.csrPtr, csr->colPtrs.data(), 4 * (size_t(c.n) + 1), hipMemcpyHostToDevice));
                         if (c.nnz()) BLEST_HIP(hipMemcpy(g.csrIdx, csr->rows.data(), 4 * c.nnz(), hipMemcpyHostToDevice));
@@ -453,7 +472,7 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                     upload();
                     StreamGuard prep;
                     BLEST_HIP(hipStreamCreateWithFlags(&prep.s, hipStreamNonBlocking));
-                    g.symmetric = csr_symmetric_on_device(prep.s, g.csrPtr, g.csrIdx, c.n, uint32_t(c.nnz()));
+                    g.symmetric = csr_symmetric_on_device(prep.s, g.csrPtr, g.csrIdx, c.n, uint32_t(c.nnz()), g.noIn);
                     if (!ghIsCsr && !g.symmetric) {
                         tr = csc_transpose(c);
                         csr = &tr;
@@ -477,13 +496,17 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                                         c.nnz() <= dev::kThinMidEdges);
                     while ((g.W - 1) >> g.thinShift >= dev::kThinMaxSegs) ++g.thinShift;
                     g.thinSegs = ((g.W - 1) >> g.thinShift) + 1;
-                    // vertices without in-neighbours: a bottom-up sweep skips them
-                    g.noIn = g.alloc<unsigned long long>(g.W);
                     csr_marks(prep.s, g.csrPtr, g.csrIdx, c.n, g.W, g.probe, g.noIn);
-                    csr_list_units(prep.s, g.csrPtr, c.n, kPullOwn, kPullUnit, [&](uint32_t count) {
-                        g.pullCount = count;
-                        return g.pullUnits = g.alloc<uint2>(count);
-                    });
+                    const std::vector<uint2> units =
+                        maxDegree > kPullOwn || csr == &tr ? pull_units(csr->colPtrs, c.n) : std::vector<uint2>();
+                    if (!units.empty()) try {
+                            g.pullUnits = g.alloc<uint2>(units.size());
+                            BLEST_HIP(hipMemcpy(g.pullUnits, units.data(), sizeof(uint2) * units.size(),
+                                                hipMemcpyHostToDevice));
+                            g.pullCount = uint32_t(units.size());
+                        } catch (const Error& e) {  // the pull scans whole lists without them
+                            if (e.code != BLEST_ERR_OUT_OF_DEVICE_MEMORY) throw;
+                        }
                 }
             }
             if (inv_perm) {
@@ -591,8 +614,16 @@ blest_status blest_query_create(blest_device_graph* dg, uint32_t max_sources, bl
             // One allocation for the state that stays inside the library (17 took longer than
             // the rest of the call); the level arrays are their own, so that a result range
             // that overruns them is told apart from one that fits.
-            const size_t bytes = carve_state(g, nullptr, q, false, g.thin, true);
-            carve_state(g, q.alloc<unsigned char>(bytes), q, false, g.thin, true);
+            const auto carve = [&](bool thin) {
+                const size_t bytes = carve_state(g, nullptr, q, false, thin, true);
+                carve_state(g, q.alloc<unsigned char>(bytes), q, false, thin, true);
+            };
+            try {
+                carve(g.thin);
+            } catch (const Error& e) {  // no room for the vertex queues: the bit-matrix levels do without
+                if (!g.thin || e.code != BLEST_ERR_OUT_OF_DEVICE_MEMORY) throw;
+                carve(false);
+            }
             BLEST_HIP(hipMemset(q.ctrl, 0, sizeof(dev::Ctrl)));
             q.levels = q.alloc<int32_t>(size_t(g.n) * max_sources);
             if (g.hasPerm) q.levelsOut = q.alloc<int32_t>(size_t(g.n) * max_sources);

@@ -230,6 +230,7 @@ __device__ __forceinline__ void mbfs_pull_csr(const GraphView& g, const MbfsArgs
     const unsigned wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
     const unsigned nwaves = (gridDim.x * blockDim.x) / kWave;
     const Bits<NW> rootMask = root_mask<NW>(a.k);
+    const uint32_t most = g.pullUnits ? kPullOwn : 0xFFFFFFFFu;  // no units (short lists, no room for them): whole lists
     for (uint32_t w = wave; w < g.W; w += nwaves) {
         const unsigned long long open = ~a.full[w];  // the slots past n are full
         if (!open) continue;
@@ -272,13 +273,13 @@ __device__ __forceinline__ void mbfs_pull_csr(const GraphView& g, const MbfsArgs
             const int from = row == 0 ? l[0] : row == 1 ? l[1] : row == 2 ? l[2] : l[3];
             const int at = max(from, 0);
             const uint32_t q0 = __shfl(p0, at, kWave), end = __shfl(p1, at, kWave);  // every lane shuffles
-            const uint32_t q1 = from < 0 ? q0 : part_end(q0, end, kPullOwn);
+            const uint32_t q1 = from < 0 ? q0 : part_end(q0, end, most);
             Bits<NW> miss, acc;
             acc.zero();
 #pragma unroll
             for (int i = 0; i < NW; ++i) miss.w[i] = __shfl(need.w[i], at, kWave);
             bool done = false;
-            for (uint32_t s = 0; s < kPullOwn; s += 16) {
+            for (uint32_t s = 0;; s += 16) {
                 const bool act = !done && in_part(q0, s, q1);
                 if (!__ballot(act)) break;
                 Bits<NW> F;
@@ -306,7 +307,7 @@ __device__ __forceinline__ void mbfs_pull_csr(const GraphView& g, const MbfsArgs
             unsigned long long* nr = next_at<NW>(a, v);
 #pragma unroll
             for (int i = 0; i < NW; ++i) {
-                if (deg <= kPullOwn) nr[i] = got.w[i];  // this lane alone writes the record
+                if (deg <= most) nr[i] = got.w[i];  // this lane alone writes the record
                 else if (got.w[i]) atomicOr(nr + i, got.w[i]);
             }
         }

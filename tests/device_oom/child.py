@@ -95,7 +95,64 @@ def query_state():
         check(held["q"], many)
 
 
-GROUPS = {f.__name__: f for f in (query_state,)}
+def creation():
+    """Graphs and queries: what only makes them faster (the device sort's scratch, the shares of
+    long lists, vertex queues) is done without.  The eleven allocations that a graph needs are
+    its segment bases, chunk bases, slices (five arrays), lists (two), probes and empty-list
+    marks; a query needs its state and its level array."""
+    rng = np.random.default_rng(3)
+    graphs = {"hubs": (B.CSC.rmat(11, 16, seed=4), 2), "short lists": (B.CSC.grid(60, 0.9, 0.01, 3), 1),
+              "directed": (B.CSC.from_edges(3000, rng.integers(0, 40, 20000), rng.integers(0, 3000, 20000),
+                                            undirected=False), 2)}
+    for name, (g, query_needs) in graphs.items():
+        cp, rows = g.arrays()
+        bv = B.BVSS().construct_from_csc(g)
+        roots = [int(r) for r in g.pick_roots(3, seed=1)]
+        want = {r: oracle.bfs(g.n, cp, rows, r) for r in roots}
+        held = {}
+
+        def check(dg):
+            for direction in (0, 2):
+                dg.set_thresholds(15, 18, direction)
+                k = B.BVSSBFSKernel(dg)
+                for r in roots:
+                    np.testing.assert_array_equal(k.run(r).levels, want[r])
+                for row, r in zip(mbfs(B._Query(dg, 64), roots, g.n), roots):
+                    np.testing.assert_array_equal(row, want[r])
+            dg.set_thresholds(15, 18, 0)
+
+        def graph():
+            held["dg"] = B.DeviceGraph(bv, g, None)
+
+        for ok in attempts(f"{name}: graph", graph, needed=11):
+            if ok:
+                check(held["dg"])
+
+        def query():
+            held["q"] = B.BVSSBFSKernel(held["dg"])
+
+        for ok in attempts(f"{name}: query", query, needed=query_needs):
+            if ok:
+                for r in roots:
+                    np.testing.assert_array_equal(held["q"].run(r).levels, want[r])
+
+
+def construction():
+    """The bit matrix built on the device needs all of its 24 arrays."""
+    g = B.CSC.rmat(11, 16, seed=4)
+    want = B.BVSS().construct_from_csc(g).arrays()
+    held = {}
+
+    def build():
+        held["b"] = B.BVSS().construct_on_device(g)
+
+    for ok in attempts("device construction", build, needed=24):
+        got = B.BVSS().construct_on_device(g).arrays()
+        for k in want:
+            np.testing.assert_array_equal(got[k], want[k])
+
+
+GROUPS = {f.__name__: f for f in (query_state, creation, construction)}
 
 if __name__ == "__main__":
     GROUPS[sys.argv[2]]()

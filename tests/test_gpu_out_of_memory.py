@@ -22,7 +22,7 @@ def fail_malloc(tmp_path_factory):
     return lib
 
 
-@pytest.mark.parametrize("group", ["query_state"])
+@pytest.mark.parametrize("group", ["query_state", "creation", "construction"])
 def test_failed_allocations(fail_malloc, group):
     progress(f"case failed allocations {group}")
     r = subprocess.run([sys.executable, "-u", str(HERE / "child.py"), str(fail_malloc), group], capture_output=True,
