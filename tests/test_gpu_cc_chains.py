@@ -1,0 +1,76 @@
+"""Connected components of graphs whose seed forest is made of long chains: vertices numbered
+along their paths, with ends around the tiles that the seed kernel shortens chains in."""
+import ctypes as C
+
+import numpy as np
+import pytest
+from conftest import progress
+
+pytestmark = pytest.mark.gpu
+
+
+def strided(n, step):
+    """`step` interleaved paths: each vertex is joined to the one `step` before it."""
+    v = np.arange(n - step)
+    return n, v, v + step
+
+
+def comb(n, leg):
+    """A spine with paths of `leg` vertices hung from it."""
+    spine = np.arange(n // leg - 1) * leg
+    v = np.arange(n)
+    v = v[v % leg != leg - 1]
+    return n, np.concatenate([spine, v]), np.concatenate([spine + leg, v + 1])
+
+
+def ring(n):
+    v = np.arange(n)
+    return n, v, (v + 1) % n
+
+
+CASES = {
+    "path_1023": lambda: strided(1023, 1),
+    "path_1024": lambda: strided(1024, 1),
+    "path_1025": lambda: strided(1025, 1),
+    "path_4097": lambda: strided(4097, 1),
+    "path_700000": lambda: strided(700000, 1),   # more tiles than workgroups
+    "strided_2": lambda: strided(5001, 2),
+    "strided_1023": lambda: strided(9000, 1023),
+    "strided_1024": lambda: strided(9000, 1024),
+    "comb_2": lambda: comb(6000, 2),
+    "comb_30": lambda: comb(6000, 30),
+    "ring_2049": lambda: ring(2049),
+}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_cc_chains(blest, oracle, name):
+    progress(f"case cc chains {name}")
+    n, src, dst = CASES[name]()
+    for label, ids in (("ascending", np.arange(n)), ("descending", np.arange(n)[::-1])):
+        g = blest.CSC.from_edges(n, ids[src], ids[dst])
+        want, comps = oracle.cc(n, *g.arrays())
+        for opts in ({}, {"bu_probe": -1}):
+            k = blest.BVSSCCKernel(blest.DeviceGraph(blest.BVSS().construct_from_csc(g), g, None, **opts))
+            res = k.run()
+            np.testing.assert_array_equal(res.components, want, err_msg=f"{label} {opts}")
+            assert res.no_components == comps
+
+
+def test_chains_are_not_walked_link_by_link(blest):
+    """With the lists resident, components of a path take no longer than with every slice's edges
+    hooked (a chain over all vertices took four times as long)."""
+    progress("case cc chain time")
+    n, src, dst = strided(1 << 20, 1)
+    g = blest.CSC.from_edges(n, src, dst)
+    bv = blest.BVSS().construct_from_csc(g)
+    st = blest._lib.CcStats()
+    ms = {}
+    for label, opts in (("lists", {}), ("slices", {"keep_csr": 0, "direction": 1})):
+        k = blest.BVSSCCKernel(blest.DeviceGraph(bv, g, None, **opts))
+        ms[label] = 1e9
+        for _ in range(7):
+            blest.check(blest._lib.load().blest_cc(k.q._h, 0, None, C.byref(st)))
+            assert st.no_components == 1
+            ms[label] = min(ms[label], st.kernel_ms)
+    assert ms["lists"] <= ms["slices"], ms
