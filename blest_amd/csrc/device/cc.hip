@@ -149,13 +149,12 @@ constexpr unsigned kCcVotes = 256;
 constexpr uint32_t kCcHeavy = 64;  // longer lists are hooked by a whole wave
 constexpr int kCcBlock = 256;
 
-__device__ __forceinline__ uint32_t find_root_near(uint32_t* p, uint32_t x) {
+// Reads only: a halving store of values that lag behind could put an older, lower ancestor
+// back in the place of a newer one.
+__device__ __forceinline__ uint32_t find_root_near(const uint32_t* p, uint32_t x) {
     uint32_t par = ld_parent_near(p, x);
     while (par != x) {
-        const uint32_t gp = ld_parent_near(p, par);
-        if (gp == par) return par;
-        __hip_atomic_store(p + x, gp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        x = gp;
+        x = par;
         par = ld_parent_near(p, x);
     }
     return x;
@@ -507,8 +506,10 @@ static void cc_run(Query& q, int algo, uint32_t* hostLabels, blest_cc_stats* st)
     const dim3 block(dev::kCcBlock);
     const dim3 grid(std::min<uint32_t>(uint32_t(g.cus) * 8, (g.n + dev::kCcBlock - 1) / dev::kCcBlock));
     // the sampled hooks meet at the trees that swallow the rest: fewer waves at once fail
-    // fewer swaps (1023-square grid 157 -> 96 us for the second entry, 8 -> 2 workgroups per CU)
-    const dim3 few(std::min<uint32_t>(grid.x, uint32_t(g.cus) * 2));
+    // fewer swaps (whole call with all and a quarter of the workgroups: 300-square grid 306
+    // and 190 us, mean degree 5 and 100 K vertices 441 and 204; an eighth is slower on
+    // grids, 223 and 274 on the 1023-square one in RCM order)
+    const dim3 few(std::max<uint32_t>(1, grid.x / 4));
     if (!q.labels) {
         // one allocation: all of it or none, so that a call that found no room leaves
         // nothing half made for the next one
