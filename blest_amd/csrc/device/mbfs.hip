@@ -773,6 +773,7 @@ __global__ void __launch_bounds__(kProducerBlock) BLEST_RESIDENT_GRID mbfs_updat
 // of one vertex a thread 1.31 ms; with four vertices a thread and the history read by the
 // 32 roots, four times in all, 1.55; non-temporal stores 1.15.
 constexpr unsigned kFinalBlock = 512;  // threads, and vertices of a tile
+constexpr int32_t kLate = 31;          // plane bits of a pair found past the history (levels to 16)
 typedef int32_t i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // rows start at any multiple of 4 bytes
 
 template <int NW>
@@ -806,10 +807,14 @@ __global__ void __launch_bounds__(kFinalBlock) mbfs_final_kernel(GraphView g, Mb
                 }
             }
         }
-        bool deep = false;  // a pair found past the history, stored when found
+        bool deep = false;  // pairs found past the history, stored when found: kLate in the planes
 #pragma unroll
         for (int i = 0; i < NW; ++i) {
-            deep |= (late.w[i] & ~in.w[i]) != 0;
+            const unsigned long long past = late.w[i] & ~in.w[i];
+            deep |= past != 0;
+            in.w[i] |= past;
+#pragma unroll
+            for (int b = 0; b < 5; ++b) plane[b].w[i] |= past;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
 #pragma unroll
@@ -817,7 +822,7 @@ __global__ void __launch_bounds__(kFinalBlock) mbfs_final_kernel(GraphView g, Mb
                 sPlane[5][2 * i + h][t] = uint32_t(in.w[i] >> (32 * h));
             }
         }
-        const bool careful = __syncthreads_or(deep) || v0 + kFinalBlock > g.n;
+        const bool stored = __syncthreads_or(deep), whole = v0 + kFinalBlock <= g.n;
         uint32_t p[6][4];
 #pragma unroll
         for (int b = 0; b < 6; ++b) {
@@ -838,18 +843,21 @@ __global__ void __launch_bounds__(kFinalBlock) mbfs_final_kernel(GraphView g, Mb
                 for (int b = 0; b < 5; ++b) x |= ((p[b][q] >> j) & 1u) << b;
                 l[q] = int32_t(x) | (int32_t((p[5][q] >> j) & 1u) - 1);  // -1 where no history level has it
             }
-            if (!careful) {
+            if (whole) {
+                if (stored && (l[0] == kLate || l[1] == kLate || l[2] == kLate || l[3] == kLate)) {
+                    const i32x4_a4 was = *reinterpret_cast<const i32x4_a4*>(a.levels + at);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) l[q] = l[q] == kLate ? was[q] : l[q];
+                }
                 *reinterpret_cast<i32x4_a4*>(a.levels + at) = l;
                 if (dst) *reinterpret_cast<i32x4_a4*>(dst + at) = l;
                 continue;
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const size_t u = v0 + 4 * quad + q;
-                if (u >= g.n) continue;
-                int32_t x = l[q];
-                if (x < 0 && ((vis_at<NW>(a, uint32_t(u))[r / 64] >> (r & 63u)) & 1ull)) x = a.levels[at + q];
-                else a.levels[at + q] = x;
+                if (v0 + 4 * quad + q >= g.n) continue;
+                const int32_t x = l[q] == kLate ? a.levels[at + q] : l[q];
+                a.levels[at + q] = x;
                 if (dst) dst[at + q] = x;
             }
         }
