@@ -1059,6 +1059,7 @@ static void thin_launch(Query& q, const dev::BfsArgs& b, const uint32_t* oldToNe
     const auto fused = [&](const dev::ThinArgs& x, unsigned L) {
         hipLaunchKernelGGL(dev::thin_fused_kernel, dim3(1), dim3(dev::kThinFusedBlock), 0, q.stream, gv, x, L);
     };
+    q.onQueues = true;
     hipLaunchKernelGGL(dev::thin_init_kernel, wide_grid(g), dim3(dev::kProducerBlock), 0, q.stream, gv, a);
     fused(a, 1);
     run_levels(
@@ -1113,10 +1114,13 @@ void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
         q.pending = true;
         return;
     }
-    if (!trace && q.thinQueue0 && !q.thinWide && g.opts.direction == 0 && g.opts.fuse_quads > 0) {
+    const bool wide = g.thinWide.load(std::memory_order_relaxed);
+    if (!trace && q.thinQueue0 && !wide && g.opts.direction == 0 && g.opts.fuse_quads > 0) {
         thin_launch(q, a, oldToNew, dst);
         return;
     }
+    if (wide && q.onQueues) q.levelHint = 0;
+    q.onQueues = false;
     const auto close = [&] {
         hipLaunchKernelGGL(dev::bfs_final_kernel, wide_grid(g), block, 0, q.stream, gv, a, oldToNew, dst, q.hostCtrl);
     };
@@ -1182,6 +1186,7 @@ void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
 void bfs_finish(Query& q, int32_t* hostLevels, blest_bfs_stats* st) {
     DeviceGraph& g = *q.g;
     BLEST_HIP(hipStreamSynchronize(q.stream));
+    const bool ran = q.pending;
     q.pending = false;
     const dev::Ctrl& c = *q.hostCtrl;
     // level kernels the next traversal enqueues before the fused kernel takes over: up to
@@ -1189,11 +1194,9 @@ void bfs_finish(Query& q, int32_t* hostLevels, blest_bfs_stats* st) {
     q.levelHint = c.tailFrom ? c.tailFrom - 1 : c.levels - c.fusedLevels;
     if (q.headSkip) --q.headSkip;
     else if (c.iterations == 0) q.headSkip = 7;
-    // (kept once seen: the bit-matrix levels that follow say the same of the graph)
-    if (q.thinQueue0 && c.levels < dev::kThinFewLevels && c.visited / std::max(c.levels, 1u) > dev::kThinWideLevel) {
-        q.levelHint = q.thinWide ? q.levelHint : 0;  // the hint counted queue levels
-        q.thinWide = true;
-    }
+    if (ran && q.onQueues && c.levels < dev::kThinFewLevels &&
+        c.visited / std::max(c.levels, 1u) > dev::kThinWideLevel)
+        g.thinWide.store(true, std::memory_order_relaxed);
     float ms = 0;
     BLEST_HIP(hipEventElapsedTime(&ms, q.ev0, q.ev1));
     if (st) {

@@ -37,7 +37,6 @@ struct DeviceSlot {
     dev::Ctrl* hostCtrl = nullptr;  // pinned
     hipError_t setupErr = hipSuccess;
     std::string setupWhat;
-    unsigned levelHint = 0;  // depth of the last traversal (sizes the level driver's first chunk)
 };
 std::array<DeviceSlot, kMaxDevices> g_slots;
 
@@ -134,14 +133,16 @@ blest_status blest_bfs_noalloc(const blest_device_graph* dg, uint32_t src, int32
         q.ev1 = slot.ev1;
         q.hostCtrl = slot.hostCtrl;
         q.noGraphs = true;  // instantiating a captured graph would allocate
-        q.levelHint = slot.levelHint;
+        q.levelHint = g.noallocHint;  // sizes the level driver's first chunk
+        q.onQueues = g.noallocOnQueues;
         carve_state(g, slot.ptr, q, g.hasPerm, thin, false);
         if (!g.hasPerm) q.levels = levels;  // reordered IDs are the caller's IDs
         hipLaunchKernelGGL(clear_ctrl_kernel, dim3(1), dim3(64), 0, q.stream, q.ctrl);
         BLEST_HIP(hipGetLastError());
         bfs_launch(q, s, false, g.hasPerm ? levels : nullptr);
         bfs_finish(q, nullptr, st);
-        slot.levelHint = q.levelHint;
+        g.noallocHint = q.levelHint;
+        g.noallocOnQueues = q.onQueues;
     });
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <algorithm>
+#include <atomic>
 
 #include <hip/hip_runtime.h>
 
@@ -86,7 +87,14 @@ struct DeviceGraph {
     uint32_t* probe = nullptr;           // first bottom-up probe per vertex
     uint2* pullUnits = nullptr;
     uint32_t pullCount = 0;
-    bool thin = false;                   // every list short: single-source levels over vertex queues
+    bool thin = false;                   // short lists: single-source levels over vertex queues
+    // a queue traversal of this graph had few, wide levels: the bit-matrix levels are faster
+    // (the graph's, not a query's: queries are made anew, and blest_bfs_noalloc has none)
+    std::atomic<bool> thinWide{false};
+    // what blest_bfs_noalloc keeps from one traversal of this graph to the next (under the
+    // lock of its device's scratch)
+    unsigned noallocHint = 0;
+    bool noallocOnQueues = false;
     uint32_t thinSegs = 1, thinShift = 0;
     size_t thin_queue_entries() const { return size_t(thinSegs) << (6 + thinShift); }
     uint32_t *permNewToOld = nullptr, *permOldToNew = nullptr;  // device copies
@@ -166,7 +174,7 @@ struct Query {
     // vertex queues of a thin graph's levels (thin_levels.hpp); null otherwise
     uint32_t *thinQueue0 = nullptr, *thinQueue1 = nullptr, *thinCount = nullptr;
     unsigned long long* thinEdges = nullptr;
-    bool thinWide = false;  // the last such traversal had few, wide levels: the bit-matrix levels are faster
+    bool onQueues = false;  // the last single-source traversal ran on them (levelHint counts its levels)
     int32_t* levelsOut = nullptr;  // original-order copy (when the graph carries a permutation)
     uint32_t* labels = nullptr;    // CC
     uint32_t* labelsAux = nullptr;
