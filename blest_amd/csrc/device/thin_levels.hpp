@@ -116,14 +116,19 @@ __device__ __forceinline__ void thin_finish(const ThinArgs& a, unsigned levels, 
 // A workgroup keeps its discoveries in LDS, numbered within their segment, and takes each
 // segment's room with one atomic: queue order follows vertex order, so 512 consecutive
 // entries discover into a few segments.  (An atomic per discovery on the 1,024 counters
-// serialised on their 32 cache lines: 200 us for a level of 330 K vertices.)
-constexpr unsigned kThinFound = 2048;  // discoveries held; past them appended one by one
+// serialised on their 32 cache lines: 200 us for a level of 330 K vertices.)  It writes them
+// out after its last entries, and before that whenever it holds so many that its next 512
+// entries, at most kThinMaxDegree discoveries each, might not fit; only lists longer than
+// that can still overflow, and are appended one by one.  (2,048 held and the rest appended
+// one by one: first BFS of the 7-ary tree of 4 M vertices 1,852 us, this way 393.)
+constexpr unsigned kThinHeld = 2048;
+constexpr unsigned kThinFound = kThinHeld + kThinBlock * kThinMaxDegree;
 
 __global__ void __launch_bounds__(kThinBlock) thin_level_kernel(GraphView g, ThinArgs a, unsigned Lk) {
     const unsigned L = level_of(a.ctrl, a.levelFromCtrl, Lk);
     __shared__ unsigned pre[kThinMaxSegs], tmp[16];
     __shared__ unsigned long long tmp64[16];
-    __shared__ unsigned sCnt[kThinMaxSegs], sFound;
+    __shared__ unsigned sCnt[kThinMaxSegs], room[kThinMaxSegs], sFound;
     __shared__ uint2 found[kThinFound];  // (vertex, number within the segment)
     Ctrl* c = a.ctrl;
     const unsigned done = ld_relaxed(&c->done);
@@ -148,16 +153,29 @@ __global__ void __launch_bounds__(kThinBlock) thin_level_kernel(GraphView g, Thi
     const uint32_t* qin = (L & 1) ? a.queue1 : a.queue0;
     uint32_t* qout = (L & 1) ? a.queue0 : a.queue1;
     uint32_t* counts = a.count + ((L + 1) % 3) * kThinMaxSegs;
+    // every thread, the list complete: room in each segment, then the entries
+    const auto write_out = [&] {
+        for (unsigned i = threadIdx.x; i < kThinMaxSegs; i += kThinBlock)
+            if (sCnt[i]) room[i] = atomicAdd(counts + i, sCnt[i]);
+        __syncthreads();
+        const unsigned nf = min(sFound, kThinFound);
+        for (unsigned k = threadIdx.x; k < nf; k += kThinBlock) {
+            const uint32_t s = found[k].x >> (6 + a.shift);
+            qout[(size_t(s) << (6 + a.shift)) + room[s] + found[k].y] = found[k].x;
+        }
+    };
     unsigned edges = 0;
-    for (unsigned e = tid; e < total; e += nthreads) {
-        const uint32_t v = thin_entry(a, qin, pre, e);
+    for (unsigned e0 = blockIdx.x * kThinBlock; e0 < total; e0 += nthreads) {  // the same for the workgroup
+        const unsigned e = e0 + threadIdx.x;
+        const uint32_t v = e < total ? thin_entry(a, qin, pre, e) : 0u;
         const u32x2_a4 d = *reinterpret_cast<const u32x2_a4*>(g.csrPtr + v);
-        edges += d.y - d.x;
-        for (uint32_t p = d.x; p < d.y; p += kThinStep) {
+        const uint32_t end = e < total ? d.y : d.x;
+        edges += end - d.x;
+        for (uint32_t p = d.x; p < end; p += kThinStep) {
             uint32_t u[kThinStep], w[kThinStep];
             thin_neighbours(g, p, u);
 #pragma unroll
-            for (int j = 0; j < kThinStep; ++j) w[j] = p + j < d.y ? a.visited[u[j] >> 5] : ~0u;
+            for (int j = 0; j < kThinStep; ++j) w[j] = p + j < end ? a.visited[u[j] >> 5] : ~0u;
             // not yet visited (a stale word only shows fewer bits: the atomic decides)
 #pragma unroll
             for (int j = 0; j < kThinStep; ++j) {
@@ -173,17 +191,20 @@ __global__ void __launch_bounds__(kThinBlock) thin_level_kernel(GraphView g, Thi
                     else thin_append(a, qout, counts, u[j]);
                 }
         }
+        if (e0 + nthreads >= total) break;
+        __syncthreads();
+        const bool full = sFound > kThinHeld;
+        __syncthreads();  // every thread has read
+        if (!full) continue;
+        write_out();
+        __syncthreads();
+        for (unsigned i = threadIdx.x; i < kThinMaxSegs; i += kThinBlock) sCnt[i] = 0;
+        if (threadIdx.x == 0) sFound = 0;
+        __syncthreads();
     }
     const unsigned long long sum = block_sum_u64(edges, tmp64);  // its barriers complete the list
     if (threadIdx.x == 0 && sum) a.edges[blockIdx.x] += sum;     // this workgroup's alone
-    for (unsigned i = threadIdx.x; i < kThinMaxSegs; i += kThinBlock)
-        if (sCnt[i]) pre[i] = atomicAdd(counts + i, sCnt[i]);
-    __syncthreads();
-    const unsigned nf = min(sFound, kThinFound);
-    for (unsigned k = threadIdx.x; k < nf; k += kThinBlock) {
-        const uint32_t s = found[k].x >> (6 + a.shift);
-        qout[(size_t(s) << (6 + a.shift)) + pre[s] + found[k].y] = found[k].x;
-    }
+    write_out();
 }
 
 // Small levels back to back in one workgroup, the queue in LDS: enqueued after the init

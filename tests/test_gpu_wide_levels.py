@@ -49,3 +49,34 @@ def test_verdict_is_the_graphs(blest):
         levels, st = noalloc(blest, dg, 0, g.n)
         np.testing.assert_array_equal(levels, depth)
         assert rep == 0 or st.bu_levels > 0
+
+
+@pytest.mark.parametrize("n, arity", [(1_000_000, 7), (600_000, 5), (500_000, 31)])
+def test_more_discoveries_than_are_held(blest, n, arity):
+    """Queue levels (the first traversal of a graph) whose workgroups write out more than once; with
+    31 children each, 512 entries alone discover more than fits."""
+    progress(f"case wide levels n={n} arity={arity}")
+    g, depth = tree(blest, n, arity)
+    perm = np.random.default_rng(6).permutation(n).astype(np.uint32)
+    mixed, _ = tree(blest, n, arity)
+    mixed.apply_permutation(perm)
+    for graph, inv in ((g, None), (mixed, perm)):
+        dg = blest.DeviceGraph(blest.BVSS().construct_from_csc(graph), graph, inv)
+        res = blest.BVSSBFSKernel(dg).run(0)
+        np.testing.assert_array_equal(res.levels, depth)
+        assert res.bu_levels == 0 and res.no_visited == n and res.edges_in_component == n - 1
+
+
+def test_first_wide_traversal(blest):
+    """It may not cost several of those that follow on the bit matrix (it was seven times theirs)."""
+    progress("case wide levels first traversal time")
+    g, depth = tree(blest, 4_000_000, 7)
+    bv = blest.BVSS().construct_from_csc(g)
+    st, first, later = blest._lib.BfsStats(), [], []
+    for rep in range(4):
+        k = blest.BVSSBFSKernel(blest.DeviceGraph(bv, g, None))
+        for out in (first, later, later):
+            blest.check(blest._lib.load().blest_bfs(k.q._h, 0, None, C.byref(st)))
+            assert st.total_levels == depth.max() + 1
+            out.append(st.kernel_ms)
+    assert np.median(first) <= 3 * np.median(later), (first, later)
