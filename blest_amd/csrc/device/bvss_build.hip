@@ -26,6 +26,7 @@
 #include "../bvss.hpp"
 #include "dgraph.hpp"
 #include "scratch.hpp"
+#include "segmented_sort.hpp"
 
 namespace blest {
 namespace dev {
@@ -247,9 +248,8 @@ BVSS bvss_build_on_device(const CSC& g, bool fullPadding, int device) {
     uint8_t* sMasks = sc.alloc<uint8_t>(nnz);
     int endBit = 3;
     while ((uint64_t(1) << (endBit - 3)) < n) ++endBit;
-    size_t sortBytes = 0, scanBytes = 0;
-    BLEST_HIP(hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, sortBytes, keysIn, keysOut, int(maxItems),
-                                                         int(maxSegs), off, off + 1, 0, endBit, st));
+    const size_t sortBytes = segmented_sort_bytes(uint32_t(maxItems), uint32_t(maxSegs), endBit, st);
+    size_t scanBytes = 0;
     BLEST_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, scanBytes, flag, pos, int(maxItems), st));
     void* temp = sc.alloc<uint8_t>(std::max(sortBytes, scanBytes));
 
@@ -271,12 +271,10 @@ BVSS bvss_build_on_device(const CSC& g, bool fullPadding, int device) {
         hipLaunchKernelGGL(dev::bb_fill_u8_kernel, grid_for(items), dim3(256), 0, st, head, uint8_t(0), size_t(items));
         hipLaunchKernelGGL(dev::bb_heads_kernel, grid_for(nseg), dim3(256), 0, st, off, nseg, head);
         BLEST_HIP(hipGetLastError());
-        size_t tb = sortBytes;
-        BLEST_HIP(hipcub::DeviceSegmentedRadixSort::SortKeys(temp, tb, keysIn, keysOut, int(items), int(nseg), off,
-                                                             off + 1, 0, endBit, st));
+        segmented_sort(temp, sortBytes, keysIn, keysOut, items, nseg, off, endBit, st);
         hipLaunchKernelGGL(dev::bb_flags_kernel, grid_for(items), dim3(256), 0, st, keysOut, head, items, flag);
         BLEST_HIP(hipGetLastError());
-        tb = scanBytes;
+        size_t tb = scanBytes;
         BLEST_HIP(hipcub::DeviceScan::ExclusiveSum(temp, tb, flag, pos, int(items), st));
         const uint32_t total = read_one(pos + items - 1, st) + read_one(flag + items - 1, st);
         hipLaunchKernelGGL(dev::bb_slices_kernel, grid_for(items), dim3(256), 0, st, keysOut, flag, pos, items, sreal,

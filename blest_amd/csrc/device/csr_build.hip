@@ -7,6 +7,7 @@
 
 #include "csr_build.hpp"
 #include "scratch.hpp"
+#include "segmented_sort.hpp"
 
 namespace blest {
 namespace dev {
@@ -169,10 +170,9 @@ void csr_sort_by_degree(hipStream_t st, const CSC& csr, const uint32_t* ptr, uin
     uint32_t* off = sc.alloc<uint32_t>(maxCols + 1);
     int bits = 1;
     while ((uint64_t(1) << bits) < n) ++bits;
-    size_t pairBytes = 0, segBytes = 0;
+    size_t pairBytes = 0;
+    const size_t segBytes = segmented_sort_bytes(uint32_t(maxItems), uint32_t(maxCols), bits, st);
     BLEST_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, pairBytes, keysIn, keysOut, rank, order, int(n), 0, 32, st));
-    BLEST_HIP(hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, segBytes, keysIn, keysOut, int(maxItems), int(maxCols),
-                                                         off, off + 1, 0, bits, st));
     void* temp = sc.alloc<uint8_t>(std::max(pairBytes, segBytes));
     const dim3 block(dev::kCsrBlock);
     hipLaunchKernelGGL(dev::csr_degree_keys_kernel, grid_for(n), block, 0, st, ptr, n, keysIn, rank);
@@ -187,9 +187,7 @@ void csr_sort_by_degree(hipStream_t st, const CSC& csr, const uint32_t* ptr, uin
         hipLaunchKernelGGL(dev::csr_offsets_kernel, grid_for(uint64_t(cols) + 1), block, 0, st, ptr, c0, cols, e0, off);
         hipLaunchKernelGGL(dev::csr_gather_kernel, grid_for(items), block, 0, st, rank, idx + e0, items, keysIn);
         BLEST_HIP(hipGetLastError());
-        size_t bytes = segBytes;
-        BLEST_HIP(hipcub::DeviceSegmentedRadixSort::SortKeys(temp, bytes, keysIn, keysOut, int(items), int(cols), off,
-                                                             off + 1, 0, bits, st));
+        segmented_sort(temp, segBytes, keysIn, keysOut, items, cols, off, bits, st);
         hipLaunchKernelGGL(dev::csr_gather_kernel, grid_for(items), block, 0, st, order, keysOut, items, idx + e0);
         BLEST_HIP(hipGetLastError());
     }
