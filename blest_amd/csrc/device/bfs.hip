@@ -984,8 +984,6 @@ __global__ void __launch_bounds__(kProducerBlock) bfs_final_kernel(GraphView g, 
 
 // The whole traversal of a small symmetric graph in one workgroup (small_traverse.hpp):
 // no level kernel, no poll per chunk of levels.
-constexpr uint64_t kSmallEdges = 1u << 18;     // see small_graph()
-
 __global__ void __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(4)))
 bfs_small_kernel(GraphView g, BfsArgs a, const uint32_t* oldToNew, int32_t* dst, Ctrl* host) {
     extern __shared__ unsigned long long bitmaps[];
@@ -1022,17 +1020,9 @@ static ExpandKernel expand_kernel_for(const DeviceGraph& g) {
     }
 }
 
-// Graphs that one workgroup traverses faster than level kernels do.  Its time grows with
-// the words of the bitmap, which every level passes over, and with the edges; a level pair
-// costs 15 us and more whatever it holds (us per call, one workgroup and level kernels:
-// Erdos-Renyi of mean degree 4, 2 K vertices 44 and 139, 8 K 78 and 142, 20 K 149 and 177;
-// mean degree 3, 50 K 397 and 224; R-MAT 13 of edge factor 16 52 and 104).  Only the
-// default schedule: a fixed direction, levels never fused and always-replayed chunks keep
-// their level kernels.
-static bool small_graph(const DeviceGraph& g) {
-    return g.symmetric && g.hasCsr && g.n <= dev::kSmallVertices && g.nnz <= dev::kSmallEdges &&
-           g.opts.direction == 0 && g.opts.fuse_quads > 0 && g.opts.use_graphs != 1;
-}
+// Only the default schedule takes the paths of paths.hpp: a fixed direction and levels never
+// fused keep the level kernels, and so do always-replayed chunks on a small graph.
+static bool default_schedule(const DeviceGraph& g) { return g.opts.direction == 0 && g.opts.fuse_quads > 0; }
 
 // The traversal over vertex queues (thin_levels.hpp); ev0 is recorded.
 static void thin_launch(Query& q, const dev::BfsArgs& b, const uint32_t* oldToNew, int32_t* dst) {
@@ -1104,7 +1094,7 @@ void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
     const ExpandKernel expand = expand_kernel_for(g);
     const uint32_t* oldToNew = g.hasPerm ? g.permOldToNew : nullptr;
     BLEST_HIP(hipEventRecord(q.ev0, q.stream));
-    if (!trace && !q.thinQueue0 && small_graph(g)) {
+    if (!trace && !q.thinQueue0 && g.small && default_schedule(g) && g.opts.use_graphs != 1) {
         hipLaunchKernelGGL(dev::bfs_small_kernel, dim3(1), dim3(dev::kBatchBlock), 3 * sizeof(unsigned long long) * g.W,
                            q.stream, gv, a, oldToNew, dst, q.hostCtrl);
         BLEST_HIP(hipGetLastError());
@@ -1115,7 +1105,7 @@ void bfs_launch(Query& q, uint32_t src, bool trace, int32_t* dst) {
         return;
     }
     const bool wide = g.thinWide.load(std::memory_order_relaxed);
-    if (!trace && q.thinQueue0 && !wide && g.opts.direction == 0 && g.opts.fuse_quads > 0) {
+    if (!trace && q.thinQueue0 && !wide && default_schedule(g)) {
         thin_launch(q, a, oldToNew, dst);
         return;
     }

@@ -7,6 +7,7 @@
 #include "csr_build.hpp"
 #include "dgraph.hpp"
 #include "level_common.hpp"
+#include "paths.hpp"
 #include "scratch.hpp"
 #include "segments.hpp"
 #include "small_traverse.hpp"
@@ -489,11 +490,8 @@ static blest_status create_device_graph(const blest_bvss* bh, const blest_csc* g
                         g.probe = g.alloc<uint32_t>(c.n);
                     }
                     g.hasCsr = true;
-                    g.thin = g.symmetric && c.nnz() <= uint64_t(dev::kThinMeanDegree) * c.n &&
-                             (maxDegree <= dev::kThinMaxDegree
-                                  ? c.n <= dev::kThinMaxVertices
-                                  : maxDegree <= dev::kThinMidDegree && c.n > dev::kThinMidFrom &&
-                                        c.nnz() <= dev::kThinMidEdges);
+                    g.thin = g.symmetric && dev::thin_graph(c.n, c.nnz(), maxDegree);
+                    g.small = g.symmetric && dev::small_graph(c.n, c.nnz());
                     while ((g.W - 1) >> g.thinShift >= dev::kThinMaxSegs) ++g.thinShift;
                     g.thinSegs = ((g.W - 1) >> g.thinShift) + 1;
                     csr_marks(prep.s, g.csrPtr, g.csrIdx, c.n, g.W, g.probe, g.noIn);

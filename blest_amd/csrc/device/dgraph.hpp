@@ -88,6 +88,7 @@ struct DeviceGraph {
     uint2* pullUnits = nullptr;
     uint32_t pullCount = 0;
     bool thin = false;                   // short lists: single-source levels over vertex queues
+    bool small = false;                  // few vertices and edges: one workgroup's BFS, unless thin
     // a queue traversal of this graph had few, wide levels: the bit-matrix levels are faster
     // (the graph's, not a query's: queries are made anew, and blest_bfs_noalloc has none)
     std::atomic<bool> thinWide{false};

@@ -18,24 +18,7 @@ namespace dev {
 constexpr int kMaxSegs = 2048;
 constexpr int kProducerBlock = 512;
 
-// Graphs traversed over vertex queues (thin_levels.hpp): at most kThinMeanDegree list
-// entries a vertex on average, and
-//   no list longer than kThinMaxDegree (grids, road networks: many levels), up to
-//     kThinMaxVertices, past which a level's claims outweigh what its launches save (us per
-//     BFS, queues and bit matrix: grids of 300, 1000, 2047 and 4096 squared 314 and 585,
-//     489 and 917, 812 and 1602, 4532 and 3373);
-//   or no list longer than kThinMidDegree (sparse random graphs) from kThinMidFrom
-//     vertices, below which one workgroup is faster (bfs_small_kernel; mean degree 4: 8 K
-//     vertices 78 against 90, 20 K 149 against 114), up to kThinMidEdges (mean degree 3:
-//     0.1 M vertices 144 and 219, 0.26 M 200 and 275, 0.4 M 227 and 296, 0.8 M 339 and 313).
-// A graph that passes but turns out to have few, wide levels (kThinFewLevels,
-// kThinWideLevel vertices on average) is left to the bit matrix after its first traversal.
-constexpr uint32_t kThinMeanDegree = 5, kThinMaxDegree = 8, kThinMidDegree = 32;
-constexpr uint32_t kThinMaxVertices = 6u << 20, kThinMidFrom = 8192, kThinMidEdges = 21u << 16;
-constexpr uint32_t kThinFewLevels = 40, kThinWideLevel = 32768;
-// The one-workgroup BFS (bfs_small_kernel): up to so many vertices.
-constexpr uint32_t kSmallVertices = 16384;
-constexpr uint32_t kThinMaxSegs = 1024;
+constexpr uint32_t kThinMaxSegs = 1024;  // segments of a vertex queue (thin_levels.hpp)
 
 // A level kernel runs one workgroup per segment, and its level ends with its slowest
 // workgroup, so the default grid (4 workgroups of 512 threads per CU = 8 waves per SIMD)

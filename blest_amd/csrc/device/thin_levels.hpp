@@ -1,6 +1,6 @@
-// Top-down BFS levels over vertex queues, for graphs whose lists are all short (grids, road
-// networks): symmetric, resident CSR, no list longer than kThinMaxDegree and few entries a
-// vertex on average.  Such a traversal has dozens of thin levels.  In the bit-matrix form a
+// Top-down BFS levels over vertex queues, for graphs whose lists are short (grids, road
+// networks, sparse random graphs; paths.hpp): symmetric, resident CSR, few entries a vertex
+// on average.  Such a traversal has dozens of thin levels.  In the bit-matrix form a
 // level is two kernels, and both touch every segment whatever the frontier holds: the
 // update packs a byte per vertex, the expansion looks up a vset and a frontier byte per
 // listed rset.  Bottom-up sweeps do not pay either: a list of four seldom ends early.  Here
@@ -20,6 +20,7 @@
 #pragma once
 
 #include "level_common.hpp"
+#include "paths.hpp"
 #include "small_traverse.hpp"
 
 namespace blest {
