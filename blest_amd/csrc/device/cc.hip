@@ -238,7 +238,8 @@ __global__ void __launch_bounds__(kCcBlock) cc_sample_hook_kernel(GraphView g, u
 }
 
 // giant[0] = the root that most of the sampled vertices hang under (one workgroup; p is
-// compressed).  Each thread counts the votes for its own sample's root.
+// compressed).  Each thread counts the votes for its own sample's root.  The rest's hooks may
+// link that root under another: cc_min_original_kernel leaves the tree's final root in giant[1].
 __global__ void __launch_bounds__(kCcVotes) cc_giant_kernel(const uint32_t* p, uint32_t n, uint32_t* giant) {
     __shared__ uint32_t root[kCcVotes];
     __shared__ unsigned long long best;
@@ -287,13 +288,13 @@ __device__ __forceinline__ void lower_min(uint32_t* minOf, uint32_t root, uint32
 }
 
 __global__ void __launch_bounds__(kCcBlock) cc_min_original_kernel(const uint32_t* p, const uint32_t* newToOld,
-                                                                   uint32_t* minOf, const uint32_t* giant,
+                                                                   uint32_t* minOf, uint32_t* giant,
                                                                    uint32_t* giantMin, uint32_t* rootsPerBlock,
                                                                    uint32_t n) {
     __shared__ unsigned long long tmp64[16];
     __shared__ uint32_t blockMin;
     const unsigned lane = lane_id();
-    const uint32_t big = giant[0];
+    const uint32_t big = p[giant[0]];
     if (threadIdx.x == 0) blockMin = 0xFFFFFFFFu;
     __syncthreads();
     uint32_t bigMin = 0xFFFFFFFFu;
@@ -337,6 +338,7 @@ __global__ void __launch_bounds__(kCcBlock) cc_min_original_kernel(const uint32_
     if (threadIdx.x == 0) {
         rootsPerBlock[blockIdx.x] = uint32_t(total);
         giantMin[blockIdx.x] = blockMin;
+        if (blockIdx.x == 0) giant[1] = big;
     }
 }
 
@@ -350,7 +352,7 @@ __global__ void __launch_bounds__(kCcBlock) cc_relabel_kernel(const uint32_t* p,
                                                               const uint32_t* minOf, const uint32_t* giant,
                                                               const uint32_t* giantMin, uint32_t* out, uint32_t n) {
     __shared__ uint32_t all;
-    const uint32_t big = giant[0];
+    const uint32_t big = giant[1];
     if (threadIdx.x == 0) all = 0xFFFFFFFFu;
     __syncthreads();
     uint32_t m = 0xFFFFFFFFu;
@@ -513,7 +515,7 @@ static void cc_run(Query& q, int algo, uint32_t* hostLabels, blest_cc_stats* st)
     if (!q.labels) {
         // one allocation: all of it or none, so that a call that found no room leaves
         // nothing half made for the next one
-        const size_t n = (size_t(g.n) + 63) / 64 * 64, counts = 2 * size_t(g.cus) * 8 + 1;
+        const size_t n = (size_t(g.n) + 63) / 64 * 64, counts = 2 * size_t(g.cus) * 8 + 2;
         q.hostCcCounts.resize(size_t(g.cus) * 8);
         q.labels = q.alloc<uint32_t>(2 * n + counts);
         q.labelsAux = q.labels + n;
@@ -538,7 +540,6 @@ static void cc_run(Query& q, int algo, uint32_t* hostLabels, blest_cc_stats* st)
         vote();
         hipLaunchKernelGGL(dev::cc_rest_kernel, grid, block, 0, q.stream, gv, q.labels, giant);
         hipLaunchKernelGGL(dev::cc_compress_kernel, grid, block, 0, q.stream, q.labels, g.n);
-        vote();
         BLEST_HIP(hipGetLastError());
     } else if (algo == 0) {
         // no CSR resident: every slice's edges are hooked

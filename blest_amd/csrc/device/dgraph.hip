@@ -675,7 +675,7 @@ blest_status blest_query_footprint(const blest_device_graph* dg, uint32_t max_so
             b += (4ull + mbfs_history_levels(g.n, nw) + 1) * 8ull * g.n * nw + 4ull * 128 + 16ull * 128;
             b += 2ull * 8ull * g.W + g.W;  // frontier-any bitmaps, dirty word marks
         }
-        b += 4ull * (2 * ((uint64_t(g.n) + 63) / 64 * 64) + uint64_t(g.cus) * 16 + 1);  // CC labels, counts
+        b += 4ull * (2 * ((uint64_t(g.n) + 63) / 64 * 64) + uint64_t(g.cus) * 16 + 2);  // CC labels, counts
         *bytes = b;
     });
 }

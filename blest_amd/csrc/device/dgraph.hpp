@@ -179,7 +179,7 @@ struct Query {
     int32_t* levelsOut = nullptr;  // original-order copy (when the graph carries a permutation)
     uint32_t* labels = nullptr;    // CC
     uint32_t* labelsAux = nullptr;
-    uint32_t* ccCounts = nullptr;  // per workgroup: roots, the giant tree's minimum; then its root
+    uint32_t* ccCounts = nullptr;  // per workgroup: roots, the giant tree's minimum; then its root as voted and in the end
     std::vector<uint32_t> hostCcCounts;
     // multi-source state, allocated on first use: words per vertex x n
     uint32_t mbfsWords = 0;
