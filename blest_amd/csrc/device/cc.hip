@@ -126,7 +126,11 @@ __global__ void cc_compress_kernel(uint32_t* p, uint32_t n) {
 // ----------------------------------------------- components from the CSR (algo 0)
 // Hooking every edge of the graph costs a pass over all slices with two dependent walks
 // per edge, and on a social graph the concurrent compare-and-swaps meet at the hubs'
-// roots.  With the (symmetric) CSR resident almost no edge needs to be hooked:
+// roots.  With the (symmetric) CSR resident almost no edge needs to be hooked.  The plan (hook
+// sampled neighbours, compress, find the most frequent tree, finish only what lies outside
+// it) is that of Afforest (Sutton, Ben-Nun and Barak, "Optimizing Parallel Graph Connectivity
+// Computation via Subgraph Sampling", IPDPS 2018); the seed forest, the hooks and the minima
+// are this kernel's own:
 //   seed    a vertex takes its highest-degree neighbour (the first of its list) as
 //           parent when that neighbour ranks above it: (degree, smaller ID).  Ranks rise
 //           along parents, so this is a forest, made without one atomic;
@@ -143,7 +147,7 @@ __global__ void cc_compress_kernel(uint32_t* p, uint32_t n) {
 // Bound by the launches and the dependent walks, not by memory (R-MAT 20: 8 MB of
 // offsets, probes and parents).  Measured (MI355X, whole call): R-MAT 20 natural order,
 // labels on the device, 1.5-3.9 ms with every slice hooked (by the graph's seed) ->
-// 0.142 ms; 1023-square grid in RCM order, labels to the host, 13.2 -> 0.50 ms.
+// 0.142 ms; 1023-square grid in RCM order, labels to the host, 13.2 -> 0.48 ms.
 constexpr uint32_t kCcSampled = 2;
 constexpr unsigned kCcVotes = 256;
 constexpr uint32_t kCcHeavy = 64;  // longer lists are hooked by a whole wave

@@ -200,10 +200,17 @@ typedef struct blest_device_opts {
     double alpha;            /* top-down -> bottom-up when frontier edges > unexplored edges / alpha */
     double beta;             /* bottom-up -> top-down when frontier vertices < n / beta and frontier
                                 edges <= unexplored edges */
-    int direction;           /* 0 = optimizing, 1 = top-down only, 2 = bottom-up after level 1.  Under 0,
-                                a symmetric graph with a resident CSR and either few vertices (at
-                                most 16384) or only short lists (grids, road networks) is searched
-                                by kernels of their own, all levels top-down */
+    int direction;           /* 0 = optimizing, 1 = top-down only, 2 = bottom-up after level 1.  Under 0, a
+                                symmetric graph with a resident CSR may be searched by kernels of
+                                their own instead of the level kernels.  Short lists (at most 5
+                                entries a vertex on average and none longer than 8, up to 6 x 2^20
+                                vertices; or none longer than 32, more than 8192 vertices, up to
+                                1376256 entries): over vertex queues, all levels top-down, without
+                                alpha and beta; left for the level kernels once a traversal had
+                                few, wide levels.  Other graphs of at most 16384 vertices and 262144
+                                entries: in one workgroup, with alpha and beta (frontier vertices
+                                alone decide the way back).  The knobs below that shape the level
+                                kernels do nothing there */
     int keep_csr;            /* upload the bottom-up CSR (needed for direction != 1) */
     uint32_t timeout_ms;     /* bound on every in-kernel wait */
     int use_graphs;          /* level chunks replayed from a captured HIP graph: 0 = once a
@@ -266,7 +273,8 @@ blest_status blest_device_graph_set_fuse(blest_device_graph* dg, int32_t fuse_qu
  * candidate timed as the mean HIP-event time of single-source BFS from `roots`
  * (original IDs) after one warm-up pass; a candidate replaces the best so far only when
  * it is more than 1% faster, so ties between candidates within timing noise keep the
- * earlier (default-side) choice.  base (nullable) supplies the other fields;
+ * earlier (default-side) choice.  On graphs searched by kernels of their own (see direction)
+ * most knobs change nothing and the defaults stay.  base (nullable) supplies the other fields;
  * best receives the fastest opts, best_ms its mean time, trials the candidates run. */
 blest_status blest_autotune_bfs(const blest_bvss* b, const blest_csc* g, const uint32_t* perm_old_to_new,
                                 const uint32_t* roots, uint32_t nroots, const blest_device_opts* base,
@@ -307,7 +315,8 @@ void* blest_query_levels_device(blest_query* q);
  * tight serving loops or harnesses that forbid it).  Same traversal and result as
  * blest_bfs, without a blest_query: the traversal state lives in a 64 MiB device array
  * that the library holds on each GPU it runs on until the process ends, and the kernels
- * run on `stream` (hipStream_t, NULL = the null stream).  levels: device memory of the
+ * run on `stream` (hipStream_t, NULL = the null stream); a short-list graph runs over vertex
+ * queues where they fit the array as well, else on the level kernels.  levels: device memory of the
  * graph's device, n int32 entries in original IDs (-1 = unreachable).  A graph whose
  * state exceeds the array (about 4.2 M vertices and 1.1 M vsets, e.g. R-MAT scale 22,
  * fit) is rejected with BLEST_ERR_INVALID_ARGUMENT.  Calls on one GPU share the array
@@ -321,7 +330,8 @@ blest_status blest_bfs_noalloc(const blest_device_graph* dg, uint32_t src, int32
  * levels[k*n] (row r = root r). */
 /* Per-level timing (tracing; no reference counterpart beyond its commented-out
  * per-level clock stamps, BFS/BVSSBFSKernel.cuh:56-58): a single-source BFS that
- * records a HIP event after every kernel.  Level L = 1..total_levels - 1 expands
+ * records a HIP event after every kernel.  It always runs the level kernels, also on graphs
+ * that blest_bfs searches by kernels of their own.  Level L = 1..total_levels - 1 expands
  * frontier L-1 (bottom_up = direction taken) and folds the result into frontier L. */
 typedef struct blest_level_trace {
     uint32_t level, bottom_up;
@@ -340,7 +350,8 @@ blest_status blest_mbfs(blest_query* q, const uint32_t* srcs, uint32_t k, int32_
 /* CCKernel::run() (CC/CCKernel.cuh:51-54): connected components of a symmetric
  * graph.  labels[n] = smallest original vertex ID of the component (the
  * canonical form; the reference's compaction at CC/BVSSCCKernel.cuh:1284-1290
- * is not reproduced).  algo: 0 = hook + compress over BVSS slices,
+ * is not reproduced).  algo: 0 = hook + compress, over the lists of a resident CSR, else over
+ * the BVSS slices;
  * 1 = min-label propagation over BVSS (CC/BVSSCCKernel.cuh:33-276). */
 typedef struct blest_cc_stats {
     double kernel_ms;
@@ -407,7 +418,8 @@ void blest_server_free(blest_server* s);
 /* Many small independent graphs, one root each, traversed by one persistent
  * launch (one workgroup per graph, bitmaps in LDS). */
 typedef struct blest_graph_batch blest_graph_batch;
-/* graphs: count CSC handles (each n <= 65536*4). */
+/* graphs: count CSC handles, each symmetric with 1 <= n <= 131072 (16-bit lists up to 65536
+ * vertices, 32-bit ones above). */
 blest_status blest_graph_batch_create(const blest_csc* const* graphs, uint32_t count, int device,
                                       blest_graph_batch** out);
 void blest_graph_batch_free(blest_graph_batch* gb);
